@@ -349,14 +349,12 @@ int lbx_addressing(lbx_ctx* ctx);
  * s(r+c_l, inv l) (module_moment_propagation.f90:218-229): LBX_MP_RECOMPUTED
  * keeps each node's density and flow (32 bytes) and recomputes them in the
  * step with the set-up's own arithmetic; LBX_MP_STORED keeps the 18
- * probabilities of each node (144 bytes in FP64, 72 in the FP32 forms);
- * LBX_MP_MIXED keeps the 10 of the directions with c_z != 0 (whose neighbours
- * lie a plane away) and recomputes the 8 others from the density and flow.
- * All give the same bits.  LBX_MP_AUTO (default): recomputed for two or more
- * FP64 tracers (their coefficients are shared, and 112 bytes less per node
- * pays), stored for one tracer and in the FP32 forms (where the recomputation
- * costs more than the bytes it saves).  Takes effect at the next
- * lbx_mp_init*.  No counterpart in the reference. */
+ * probabilities of each node (144 bytes in FP64, 72 in the FP32 forms).  All
+ * give the same bits.  LBX_MP_MIXED is taken as LBX_MP_RECOMPUTED.
+ * LBX_MP_AUTO (default) chooses by the size of the step's arrays: FP64 stores
+ * them while the arrays fit the 32 MiB of L2, the FP32 forms unless one
+ * tracer's arrays outgrow the 256 MiB last-level cache.  Takes effect at the
+ * next lbx_mp_init*.  No counterpart in the reference. */
 #define LBX_MP_AUTO       (-1)
 #define LBX_MP_STORED     0
 #define LBX_MP_RECOMPUTED 1
@@ -391,7 +389,7 @@ int lbx_sync(lbx_ctx* ctx);
  * instance in its LB phase, one MP launch every instance in its MP phase,
  * over one packed fluid-node list with per-instance offsets (lbx_batch.hip).
  * Each instance's results are bit-identical to the single-lattice path with
- * the same input (LB fields, P; VACF with 256-node blocks).  No counterpart
+ * the same input (LB fields, P, VACF).  No counterpart
  * in the reference (it solves one lattice per process); it serves batched
  * and continuously batched workloads.  A batch is used by one thread. */
 typedef struct lbxb lbxb;
@@ -433,9 +431,9 @@ int lbxb_info(lbxb* b, int32_t id, int32_t* phase, int32_t* status, int64_t* lb_
 int lbxb_result(lbxb* b, int32_t id, double deff[3], double* vacf, int64_t vacf_rows, double* rho, double* jx,
                 double* jy, double* jz);
 
-/* Block size (64, 128 or 256 nodes) of the LB and MP launches.  LB results
- * do not depend on it; VACF and D_eff sum per block, so they agree across
- * block sizes to rounding. */
+/* Block size (64, 128 or 256 nodes) of the LB launches; the results do not
+ * depend on it.  Moment propagation always runs one 256-thread block per tile
+ * of its layout: mp_block is checked, kept and reported, no more. */
 int lbxb_set_block(lbxb* b, int32_t lb_block, int32_t mp_block);
 
 /* lbx_set_check_interval for every instance of a batch (set before the
@@ -459,12 +457,13 @@ int lbxb_launch_mode(lbxb* b);
 int lbxb_set_addressing(lbxb* b, int32_t wide);
 int lbxb_addressing(lbxb* b);
 /* Autotuner: on the current state, without changing it, times 64-, 128-
- * and 256-node blocks per phase with one launch per step and keeps the
- * fastest, then times those launches replayed from a captured graph and as
- * one persistent cooperative launch per phase, and keeps the launch mode
- * with the least LB + MP time.  times[LBXB_AUTOTUNE_TIMES] (may be NULL) =
- * mean ms per step of LB-64, LB-128, LB-256, MP-64, MP-128, MP-256,
- * LB-graph, MP-graph, LB-persistent, MP-persistent (0: phase not timed). */
+ * and 256-node LB blocks with one launch per step and keeps the fastest (the
+ * MP launches, the same for every mp_block, are timed under each), then times
+ * those launches replayed from a captured graph and as one persistent
+ * cooperative launch per phase, and keeps the launch mode with the least
+ * LB + MP time.  times[LBXB_AUTOTUNE_TIMES] (may be NULL) = mean ms per step of
+ * LB-64, LB-128, LB-256, MP-64, MP-128, MP-256, LB-graph, MP-graph,
+ * LB-persistent, MP-persistent (0: phase not timed). */
 #define LBXB_AUTOTUNE_TIMES 10
 int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_block, double* times);
 /* Device time (HIP events around each phase of each round) and work done. */

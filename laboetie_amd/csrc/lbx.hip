@@ -13,9 +13,9 @@
 //                 up to 64
 //   j[3][Nfp]     flux of the last completed step (the next step's j_old)
 //   rho[Nfp]      density (written at set-up and when a run ends)
-// Moment propagation adds win[18][Nfp] (incoming scattering probabilities),
-// rem[Nfp], ustar[3][Nfp], P[2][3][Nfp] and, with adsorption, Pa[2][3][Nfp].
-// Every kernel runs one thread per packed fluid node, 256-node tiles, so all
+// Moment propagation has its own node order and tiles (lbx_mp.h): (rho, v),
+// rem, u*, P[2] and, with adsorption, Pa[2] per node.
+// Every LB kernel runs one thread per packed fluid node, 256-node tiles, so all
 // lanes work and every fetched cache line holds fluid data.
 #include <hip/hip_runtime.h>
 
@@ -33,6 +33,7 @@
 #include "../../include/lbx.h"
 #include "lbx_device.h"
 #include "lbx_kernels.h"
+#include "lbx_mp.h"
 #include "lbx_tables.h"
 
 #pragma clang fp contract(off)
@@ -72,7 +73,6 @@ struct lbx_ctx {
     double tau = 1.0, A = 0, B = 0, C = 0;
     float A32 = 0, B32 = 0;      // FP32-shift collision: A + B = 1 exactly (fp32_relaxation)
     int32_t check_every = 1;     // stage-2 steps between l2err measurements (kCheckEvery in FP32 storage)
-    uint32_t* mp_tile_order = nullptr;  // MP: tiles in band-major order (NULL: packed order)
     int64_t nfi = 0;
     int64_t floor_window = 0;    // FP32-storage forms: l2err floor test (0: off)
     int device = 0;
@@ -86,7 +86,6 @@ struct lbx_ctx {
     uint32_t* nodes = nullptr;
     uint32_t* map = nullptr;
     uint32_t ntiles = 0;
-    double* part = nullptr;      // per-block VACF partials, two buffers of 3*kMaxTracers per tile
     unsigned long long* slots = nullptr;  // [3][kSlots] l2err slots
     Ctrl* ctrl = nullptr;
     Ctrl ctrl_h{};               // host copy that reset_ctrl uploads from (read by the stream's next copy)
@@ -95,16 +94,14 @@ struct lbx_ctx {
     std::vector<uint32_t> nodes_h;
     // moment propagation
     bool mp_ready = false;
-    double* win = nullptr;       // FP64 form
-    double* ustar = nullptr;
-    float* win32 = nullptr;      // FP32-storage forms
-    float* ustar32 = nullptr;
-    double* rv = nullptr;        // (rho, v) per node: the step recomputes the incoming probabilities from it
-    int32_t mp_coef = LBX_MP_AUTO;        // where the next MP set-up's step takes its incoming probabilities
-    int32_t mp_coef_on = LBX_MP_STORED;   // ... and the current MP state's (kCoef* in the kernels)
-    double* rem = nullptr;
-    double* P[2] = {nullptr, nullptr};
-    double* Pa[2] = {nullptr, nullptr};
+    MpTiles mpt;                 // the geometry's tiles (built by the first MP set-up, kept)
+    uint32_t mp_ntiles = 0;
+    bool mp_general = false;     // some neighbours have no LDS slot
+    bool mp_divide = false;      // densities or flows outside quotient()'s range
+    double* part = nullptr;      // VACF partials, two buffers of 3 kMaxTracers per tile
+    MpFields<double> mpf;        // FP64 form
+    MpFields<float> mpf32;       // FP32-storage forms (P, Pa, (rho, v), rem are FP64 in both)
+    int32_t mp_coef = LBX_MP_AUTO;  // lbx_set_mp_coefficients (every form gives the same bits)
     double* vtrace = nullptr;
     int mp_now = 0;
     int64_t mp_it = 0;
@@ -192,50 +189,36 @@ void free_mp(lbx_ctx* c) {
         (void)hipStreamSynchronize(c->stream);
         c->mpp.active = false;
     }
-    dfree(c->win);
-    dfree(c->rv);
-    dfree(c->rem);
-    dfree(c->ustar);
-    dfree(c->win32);
-    dfree(c->ustar32);
-    dfree(c->P[0]);
-    dfree(c->P[1]);
-    dfree(c->Pa[0]);
-    dfree(c->Pa[1]);
+    auto fields = [](auto& f) {
+        dfree(f.rv);
+        dfree(f.win);
+        dfree(f.rem);
+        dfree(f.ustar);
+        for (int b = 0; b < 2; ++b) {
+            dfree(f.P[b]);
+            dfree(f.Pa[b]);
+        }
+    };
+    fields(c->mpf);
+    fields(c->mpf32);
     dfree(c->vtrace);
-    dfree(c->mp_tile_order);
     c->mp_ready = false;
 }
 
-#ifndef LBX_MP_BAND
-#define LBX_MP_BAND 32
-#endif
-// MP tile order: bands of kMpBandRows box rows, plane by plane within a band,
-// so that the z-neighbour rows a tile gathers were read by tiles that ran just
-// before it on the same XCD (0: the packed order).  Each tile still covers
-// the same nodes and writes its VACF partial by tile, so the bits do not
-// depend on the order.
-constexpr int32_t kMpBandRows = LBX_MP_BAND;
-
-int band_tile_order(lbx_ctx* c, int32_t band_rows, uint32_t** out) {
-    if (band_rows <= 0 || c->ntiles < 2 || *out) return LBX_OK;
-    std::vector<std::pair<uint64_t, uint32_t>> key(c->ntiles);
-    const uint64_t lx = (uint64_t)c->lx, ly = (uint64_t)c->ly;
-    for (uint32_t t = 0; t < c->ntiles; ++t) {
-        const uint64_t r = c->nodes_h[std::min<uint64_t>((uint64_t)t * kBlock, c->Nf - 1)] & kIndexMask;
-        const uint64_t y = (r / lx) % ly, z = r / (lx * ly);
-        key[t] = {((y / (uint64_t)band_rows) * (uint64_t)c->lz + z) << 32 | t, t};
-    }
-    std::sort(key.begin(), key.end());
-    std::vector<uint32_t> order(c->ntiles);
-    for (uint32_t t = 0; t < c->ntiles; ++t) order[t] = key[t].second;
-    LBX_TRY(dalloc(out, c->ntiles));
-    LBX_TRY(hipMemcpyAsync(*out, order.data(), c->ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    return hip_status(hipStreamSynchronize(c->stream));  // order is a local
+void free_tiles(lbx_ctx* c) {
+    dfree(c->mpt.info);
+    dfree(c->mpt.halo);
+    dfree(c->mpt.tab4);
+    dfree(c->mpt.tab2);
+    dfree(c->mpt.perm);
+    dfree(c->mpt.inv);
+    dfree(c->part);
+    c->mp_ntiles = 0;
 }
 
 void free_all(lbx_ctx* c) {
     free_mp(c);
+    free_tiles(c);
     if (c->mpp.vt_h) (void)hipHostFree(c->mpp.vt_h);
     if (c->mpp.ctrl_h) (void)hipHostFree(c->mpp.ctrl_h);
     c->mpp.vt_h = nullptr;
@@ -249,7 +232,6 @@ void free_all(lbx_ctx* c) {
     dfree(c->rho);
     dfree(c->nodes);
     dfree(c->map);
-    dfree(c->part);
     dfree(c->slots);
     dfree(c->ctrl);
     dfree(c->l2ring);
@@ -427,99 +409,193 @@ int upload_shift(lbx_ctx* c, const double* n_full, float* gdst) {
     return hip_status(hipStreamSynchronize(c->stream));
 }
 
-template <typename W>
-W* win_buf(lbx_ctx* c) {
-    if constexpr (std::is_same<W, float>::value) return c->win32; else return c->win;
+// The MP tiles of the context's geometry: counted, grouped, placed and
+// tabled on the device (lbx_mp.h).  Tiles whose halo outgrows a brick's are
+// taken apart while the tile count stays within mp_tile_bound; beyond that
+// the lattice runs the general step, whose tiles may have neighbours without
+// an LDS slot.
+int build_tiles(lbx_ctx* c) {
+    if (c->mp_ntiles) return LBX_OK;
+    MpBuild d{};
+    d.b = make_bricks((uint32_t)c->lx, (uint32_t)c->ly, (uint32_t)c->lz);
+    d.nodes = c->nodes;
+    d.map = c->map;
+    d.dlx = c->dlx;
+    d.dly = c->dly;
+    d.bound = mp_tile_bound(c->Nf);
+    MpBuild* dd = nullptr;
+    MpBuilt* db = nullptr;
+    uint32_t *count = nullptr, *base = nullptr;
+    uint8_t* split = nullptr;
+    MpBuilt h{};
+    const uint32_t gw = (d.b.norder + kBlock / 64 - 1) / (kBlock / 64);
+    MpTiles& t = c->mpt;
+    hipStream_t s = c->stream;
+    int st = LBX_OK;
+    auto group = [&](const uint8_t* sp) {
+        hipLaunchKernelGGL(k_mpb_group, dim3(1), dim3(kBlock), 0, s, dd, db, count, base, t.info, sp);
+        if (!st) st = hip_status(hipGetLastError());
+        if (!st) st = hip_status(hipMemcpyAsync(&h, db, sizeof(h), hipMemcpyDeviceToHost, s));
+        if (!st) st = hip_status(hipStreamSynchronize(s));
+    };
+    auto table = [&](uint32_t pitch, uint8_t* sp) {
+        if (st) return;
+        const uint64_t entries = (uint64_t)h.ntiles * kMpTile;
+        dfree(t.perm);
+        dfree(t.halo);
+        dfree(t.tab4);
+        dfree(t.tab2);
+        st = dalloc(&t.perm, entries);
+        if (!st) st = dalloc(&t.halo, (uint64_t)h.ntiles * pitch);
+        if (!st) st = dalloc(&t.tab4, entries);
+        if (!st) st = dalloc(&t.tab2, entries);
+        if (st) return;
+        t.pitch = pitch;
+        hipLaunchKernelGGL(k_mpb_place, dim3(gw), dim3(kBlock), 0, s, dd, db, base, t.perm, t.inv);
+        hipLaunchKernelGGL((pitch > kHaloMax ? k_mpb_table<true> : k_mpb_table<false>), dim3(h.ntiles), dim3(kBlock), 0,
+                           s, dd, db, t, sp);
+        st = hip_status(hipGetLastError());
+        if (!st) st = hip_status(hipMemcpyAsync(&h, db, sizeof(h), hipMemcpyDeviceToHost, s));
+        if (!st) st = hip_status(hipStreamSynchronize(s));
+    };
+    st = dalloc(&dd, 1);
+    if (!st) st = dalloc(&db, 1);
+    if (!st) st = dalloc(&count, d.b.norder);
+    if (!st) st = dalloc(&base, d.b.norder);
+    if (!st) st = dalloc(&split, d.bound);
+    if (!st) st = dalloc(&t.info, d.bound);
+    if (!st) st = dalloc(&t.inv, (uint64_t)c->Nf);
+    if (!st) st = hip_status(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
+    if (!st) {
+        hipLaunchKernelGGL(k_mpb_count, dim3(gw), dim3(kBlock), 0, s, dd, count);
+        group(nullptr);
+        table(kHaloMax, split);
+        c->mp_general = false;
+        if (!st && h.halo_max > kHaloMax) {
+            group(split);
+            if (!st && h.ntiles > 0) {
+                table(kHaloMax, nullptr);
+            } else {
+                group(nullptr);
+                table(kHaloMaxGen, nullptr);
+                c->mp_general = true;
+            }
+        }
+    }
+    if (!st) st = dalloc(&c->part, 6 * (uint64_t)kMaxTracers * h.ntiles);
+    dfree(dd);
+    dfree(db);
+    dfree(count);
+    dfree(base);
+    dfree(split);
+    if (st) {
+        free_tiles(c);
+        return st;
+    }
+    c->mp_ntiles = h.ntiles;
+    return LBX_OK;
 }
+
 template <typename W>
-W* ustar_buf(lbx_ctx* c) {
-    if constexpr (std::is_same<W, float>::value) return c->ustar32; else return c->ustar;
+MpFields<W>& mp_fields(lbx_ctx* c) {
+    if constexpr (std::is_same<W, float>::value) return c->mpf32; else return c->mpf;
+}
+
+// the P and Pa buffers of the context's precision form
+double* const* mp_moments(lbx_ctx* c, bool adsorbed) {
+    if (f32_storage(c->prec)) return adsorbed ? c->mpf32.Pa : c->mpf32.P;
+    return adsorbed ? c->mpf.Pa : c->mpf.P;
+}
+
+// the arrays of a propagation of ntr tracers
+template <typename W>
+int alloc_fields(lbx_ctx* c, int ntr, bool any_ads, bool stored) {
+    MpFields<W>& f = mp_fields<W>(c);
+    const uint64_t n = (uint64_t)c->mp_ntiles * kMpTile;
+    int st = stored ? dalloc(&f.win, 9 * n) : dalloc(&f.rv, 2 * n);
+    if (!st) st = dalloc(&f.rem, n);
+    if (!st) st = dalloc(&f.ustar, 3 * n);
+    for (int b = 0; b < 2; ++b) {
+        if (!st) st = dalloc(&f.P[b], 3 * (uint64_t)ntr * n);
+        // Pa of a tracer without adsorption is never read or written
+        if (!st && any_ads) st = dalloc(&f.Pa[b], 3 * (uint64_t)ntr * n);
+    }
+    return st;
 }
 
 // k_mp_prep + the VACF(0) reduction for the context's tracers
 template <typename W>
 void launch_mp_prep(lbx_ctx* c, const double fext[3], double eps) {
     MpPrepArgs<W> a;
+    a.t = c->mpt;
+    a.f = mp_fields<W>(c);
     a.rho = c->rho;
     a.j = c->j;
     a.nodes = c->nodes;
     a.map = c->map;
-    a.win = c->mp_coef_on == LBX_MP_RECOMPUTED ? nullptr : win_buf<W>(c);
-    a.win_z = c->mp_coef_on == LBX_MP_MIXED ? 1 : 0;
-    a.rv = c->mp_coef_on == LBX_MP_STORED ? nullptr : c->rv;
-    a.rem = c->rem;
-    a.ustar = ustar_buf<W>(c);
-    a.P0 = c->P[0];
     a.partials = c->part;
     a.ctrl = c->ctrl;
     a.dlx = c->dlx;
     a.dly = c->dly;
     a.lz = c->lz;
-    a.Nf = c->Nf;
     a.Np = c->Np;
     a.fx = fext[0];
     a.fy = fext[1];
     a.fz = fext[2];
     a.lambda = c->lambda;
     a.eps = eps;
-    a.tile0 = 0;
     a.tp = c->tp;
-    const uint32_t gt = c->ntiles;
+    const uint32_t gt = c->mp_ntiles;
     with_tracers(c->ntr, [&](auto TT) {
         constexpr int T = TT;
-        hipLaunchKernelGGL((k_mp_prep<T, W>), dim3(gt), dim3(kBlock), 0, c->stream, a);
+        hipLaunchKernelGGL((k_mp_prep<T, W>), dim3(gt), dim3(kBlock), 0, c->stream, a, 0u);
         hipLaunchKernelGGL(k_mp_reduce<3 * T>, dim3(1), dim3(kBlock), 0, c->stream, c->part, gt, nullptr, c->ctrl, 0,
                            (int64_t)0, 0, 0.0, 0.0);
     });
 }
 
-// one k_mp_step launch (and, with the convergence test, its VACF reduction)
+template <int T, typename W, bool RV, bool GEN>
+__global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void k_mp_step(MpStepArgs<W> a) {
+    // block 0 only reduces the previous step: its few round trips to memory
+    // run beside the tiles instead of before one of them
+    if (blockIdx.x == 0)
+        mp_reduce_prev<T, W>(a, gridDim.x - 1);
+    else
+        mp_step_tile<T, W, RV, GEN>(a, xcd_tile() - 1);
+}
+
+// one k_mp_step launch
 template <typename W>
 void launch_mp_step(lbx_ctx* c, int now, int64_t it, int64_t k, int32_t stop_on_convergence, double lim1,
                            double lim2) {
-    const uint32_t gt = c->ntiles;
+    const uint32_t gt = c->mp_ntiles;
     const int nv = 3 * c->ntr;
     MpStepArgs<W> a;
-    a.win = win_buf<W>(c);
-    a.rem = c->rem;
-    a.ustar = ustar_buf<W>(c);
-    a.nodes = c->nodes;
-    a.map = c->map;
-    a.Pn = c->P[now];
-    a.Px = c->P[now ^ 1];
-    a.Pan = c->any_ads ? c->Pa[now] : nullptr;
-    a.Pax = c->any_ads ? c->Pa[now ^ 1] : nullptr;
-    // partial buffers alternate by step; the previous step's VACF (and its
-    // convergence test) is reduced by block 0 of this step's kernel
+    a.t = c->mpt;
+    a.fields(mp_fields<W>(c), now != 0);
+    a.any_ads = c->any_ads;
+    // partial buffers alternate by step
     a.partials = c->part + (uint64_t)nv * gt * (it & 1);
     a.prev_partials = k > 0 ? c->part + (uint64_t)nv * gt * ((it - 1) & 1) : nullptr;
     a.prev_vtrace = c->vtrace + nv * (k - 1);
     a.check_conv = stop_on_convergence;
     a.lim1 = lim1;
     a.lim2 = lim2;
-    a.win = c->mp_coef_on == LBX_MP_RECOMPUTED ? nullptr : win_buf<W>(c);
-    a.rv = c->mp_coef_on == LBX_MP_STORED ? nullptr : c->rv;
     a.lambda = c->lambda;
     a.it = it;
     a.ctrl = c->ctrl;
+    a.tp = c->tp;
+    a.nodes = c->nodes;
+    a.map = c->map;
     a.dlx = c->dlx;
     a.dly = c->dly;
     a.lz = c->lz;
-    a.Nf = c->Nf;
-    a.Np = c->Np;
-    a.any_ads = c->any_ads;
-    a.tp = c->tp;
-    a.tile_order = c->mp_tile_order;
     with_tracers(c->ntr, [&](auto TT) {
         constexpr int T = TT;
-        auto pick = [&](auto CFT) {
-            constexpr int CF = decltype(CFT)::value;
-            return c->wide ? k_mp_step<true, T, W, CF> : k_mp_step<false, T, W, CF>;
-        };
-        auto kern = c->mp_coef_on == LBX_MP_RECOMPUTED ? pick(std::integral_constant<int, kCoefRecomputed>{})
-                    : c->mp_coef_on == LBX_MP_MIXED   ? pick(std::integral_constant<int, kCoefMixed>{})
-                                                      : pick(std::integral_constant<int, kCoefStored>{});
-        hipLaunchKernelGGL(kern, dim3(gt), dim3(kBlock), 0, c->stream, a);
+        const bool gen = c->mp_general || c->mp_divide;
+        auto kern = a.rv ? (gen ? k_mp_step<T, W, true, true> : k_mp_step<T, W, true, false>)
+                           : (c->mp_general ? k_mp_step<T, W, false, true> : k_mp_step<T, W, false, false>);
+        hipLaunchKernelGGL(kern, dim3(gt + 1), dim3(kBlock), 0, c->stream, a);
     });
 }
 
@@ -567,10 +643,13 @@ int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precisio
     const uint64_t N = (uint64_t)lx * ly * lz, Np = (N + 63) / 64 * 64;
     const uint64_t pop = f32_storage(precision) ? 4 : 8;  // populations; also win and u* of moment propagation
     uint64_t b = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + N * 8 +
-                 nblocks(N) * 6 * kMaxTracers * 8 + sizeof(Ctrl) + kRing * 8;
+                 sizeof(Ctrl) + kRing * 8;
     if (with_mp > 0) {  // with_mp tracers, each with adsorption (the upper bound)
         const uint64_t T = (uint64_t)std::min(with_mp, kMaxTracers);
-        b += (18 + 3) * Np * pop + Np * 8 + 12 * T * Np * 8 + kMpChunk * 3 * T * 8;
+        const Bricks br = make_bricks((uint32_t)lx, (uint32_t)ly, (uint32_t)lz);
+        const uint64_t tiles = std::min<uint64_t>((uint64_t)br.nbx * br.nby * br.nbz, mp_tile_bound((uint32_t)N));
+        b += tiles * kMpTile * (4 * 8 + 8 + 3 * pop + 24 + 4 + 12 * T * 8) + tiles * (kHaloMax * 4 + 6 * kMaxTracers * 8) +
+             Np * 4 + kMpChunk * 3 * T * 8;
     }
     return (int64_t)b;
 }
@@ -639,7 +718,6 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     if (!st) st = dalloc(&c->rho, c->Np);
     if (!st) st = dalloc(&c->nodes, (uint64_t)c->Nf);
     if (!st) st = dalloc(&c->map, (uint64_t)c->N);
-    if (!st) st = dalloc(&c->part, 6 * (uint64_t)kMaxTracers * c->ntiles);
     if (!st) st = dalloc(&c->slots, 3 * kSlots);
     if (!st) st = dalloc(&c->ctrl, 1);
     if (!st) st = dalloc(&c->l2ring, kRing);
@@ -947,6 +1025,24 @@ int lbx_flow(lbx_ctx* c, double* rho, double* jx, double* jy, double* jz) {
     return LBX_OK;
 }
 
+// Whether a propagation keeps the 18 incoming probabilities per node or
+// recomputes them from (rho, v) in the step (LBX_MP_AUTO).  Stored: fewer
+// operations; recomputed: 112 bytes less per node and step in FP64, 40 in the
+// FP32 forms.  Measured (us per step, stored / recomputed):
+//   FP64  64^3 BCC (21 MB of state) 6.0 / 7.5, three tracers 12.3 / 13.4;
+//         128^3 BCC 28.5 / 26.1, 58 / 48; 256^3 medium 553 / 397, 911 / 808
+//   FP32  64^3 6.0 / 7.7; 128^3 21.6 / 26.4, 42 / 48; 150x97x121 medium 32 / 40;
+//         256^3 402 / 387, three tracers 758 / 803
+// So FP64 stores while the step's arrays fit the 32 MiB of L2, and the FP32
+// forms unless one tracer's arrays outgrow the 256 MiB last-level cache.
+static bool mp_stored(const lbx_ctx* c, int32_t ntr) {
+    if (c->mp_coef != LBX_MP_AUTO) return c->mp_coef == LBX_MP_STORED;
+    const bool f32 = f32_storage(c->prec);
+    const uint64_t per_node = (18 + 3) * (f32 ? 4 : 8) + 8 + 24 + 48 * (uint64_t)ntr;
+    const uint64_t bytes = per_node * (uint64_t)c->Nf;
+    return f32 ? ntr > 1 || bytes <= (256ull << 20) : bytes <= (32ull << 20);
+}
+
 static int mp_setup(lbx_ctx* c, const double fext[3], double Db, int32_t ntr, const double* ka, const double* kd,
                     double* vacf0) {
     const double eps = DBL_EPSILON;
@@ -969,41 +1065,20 @@ static int mp_setup(lbx_ctx* c, const double fext[3], double Db, int32_t ntr, co
         tp.one_minus_kd[t] = 1.0 - kd[t];
         any_ads = any_ads || tp.ads[t];
     }
-    const uint64_t np3 = 3 * (uint64_t)ntr * c->Np;
-    int st = LBX_OK;
-    const bool shift = f32_storage(c->prec);
-    // the automatic form: the recomputation pays for several FP64 tracers (measured at 128^3 and
-    // 256^3); for one tracer, and in the FP32 forms, the stored probabilities are as fast or faster
-    c->mp_coef_on = c->mp_coef != LBX_MP_AUTO ? c->mp_coef
-                                             : (!shift && ntr >= 2 ? LBX_MP_RECOMPUTED : LBX_MP_STORED);
-    // stored probabilities: 18 per node, or the kZDirs with c_z != 0 in the mixed form
-    const uint64_t nwin = c->mp_coef_on == LBX_MP_STORED ? 18 : (c->mp_coef_on == LBX_MP_MIXED ? kZDirs : 0);
-    if (!st && !shift && nwin) st = dalloc(&c->win, nwin * c->Np);
-    if (!st && !shift) st = dalloc(&c->ustar, 3 * c->Np);
-    if (!st && shift && nwin) st = dalloc(&c->win32, nwin * c->Np);
-    if (!st && shift) st = dalloc(&c->ustar32, 3 * c->Np);
-    if (!st && c->mp_coef_on != LBX_MP_STORED) st = dalloc(&c->rv, 4 * c->Np);
-    if (!st) st = dalloc(&c->rem, c->Np);
-    if (!st) st = dalloc(&c->P[0], np3);
-    if (!st) st = dalloc(&c->P[1], np3);
+    LBX_TRY(build_tiles(c));
+    const bool stored = mp_stored(c, ntr);
+    int st = f32_storage(c->prec) ? alloc_fields<float>(c, ntr, any_ads, stored)
+                                  : alloc_fields<double>(c, ntr, any_ads, stored);
     if (!st) st = dalloc(&c->vtrace, 3 * (uint64_t)ntr * kMpChunk);
-    // Pa of a tracer without adsorption is never read or written
-    if (!st && any_ads) st = dalloc(&c->Pa[0], np3);
-    if (!st && any_ads) st = dalloc(&c->Pa[1], np3);
     if (st) {
         free_mp(c);
         return st;
     }
-    for (int b = 0; b < 2; ++b) {
-        LBX_TRY(hipMemsetAsync(c->P[b], 0, np3 * sizeof(double), c->stream));
-        if (any_ads) LBX_TRY(hipMemsetAsync(c->Pa[b], 0, np3 * sizeof(double), c->stream));
-    }
     LBX_TRY(reset_ctrl(c));
-    LBX_TRY(band_tile_order(c, kMpBandRows, &c->mp_tile_order));
     c->ntr = ntr;
     c->tp = tp;
     c->any_ads = any_ads;
-    if (shift)
+    if (f32_storage(c->prec))
         launch_mp_prep<float>(c, fext, eps);
     else
         launch_mp_prep<double>(c, fext, eps);
@@ -1012,6 +1087,7 @@ static int mp_setup(lbx_ctx* c, const double fext[3], double Db, int32_t ntr, co
     LBX_TRY(read_ctrl(c, &h));
     if (vacf0)
         for (int k = 0; k < 3 * ntr; ++k) vacf0[k] = h.vacf0[k];
+    c->mp_divide = h.mp_divide != 0;
     c->mp_ready = true;
     c->mp_now = 0;
     c->mp_it = 0;
@@ -1070,7 +1146,7 @@ static int mp_chunk_launch(lbx_ctx* c, int64_t S, int32_t stop, double* vt_h, Ct
         with_tracers(c->ntr, [&](auto TT) {
             constexpr int T = TT;
             hipLaunchKernelGGL(k_mp_reduce<3 * T>, dim3(1), dim3(kBlock), 0, c->stream,
-                               c->part + (uint64_t)nv * c->ntiles * (it & 1), c->ntiles, c->vtrace + nv * (S - 1),
+                               c->part + (uint64_t)nv * c->mp_ntiles * (it & 1), c->mp_ntiles, c->vtrace + nv * (S - 1),
                                c->ctrl, 1, it, stop, lim1, lim2);
         });
     }
@@ -1164,28 +1240,34 @@ int lbx_mp_get_tracer(lbx_ctx* c, int32_t tracer, double* P, double* Pa) {
     if (!c) return LBX_ERR_ARG;
     if (!c->mp_ready || c->mpp.active) return LBX_ERR_STATE;  // a begun chunk is waited for first
     if (tracer < 0 || tracer >= c->ntr) return LBX_ERR_ARG;
-    const int K = 3 * c->ntr;
-    std::vector<double> packed((size_t)K * c->Np);
-    // the tracer's three components (comp_index layout) into (3,lx,ly,lz), 0 at solids
+    // the tracer's three components into (3,lx,ly,lz), 0 at solids, a run of
+    // box nodes at a time through a device buffer
+    constexpr uint32_t kRun = 1u << 22;
+    double* box = nullptr;
+    LBX_TRY(dalloc(&box, 3 * (uint64_t)std::min(c->N, kRun)));
     auto fetch = [&](const double* src, double* dst) -> int {
-        LBX_TRY(hipMemcpyAsync(packed.data(), src, packed.size() * sizeof(double), hipMemcpyDeviceToHost,
-                               c->stream));
-        LBX_TRY(hipStreamSynchronize(c->stream));
-        std::memset(dst, 0, 3 * (size_t)c->N * sizeof(double));
-        for (uint32_t i = 0; i < c->Nf; ++i) {
-            const size_t r = c->nodes_h[i] & kIndexMask;
-            for (int a = 0; a < 3; ++a) dst[3 * r + a] = packed[comp_index(K, 3 * tracer + a, i, c->Np)];
+        for (uint64_t r0 = 0; r0 < c->N; r0 += kRun) {
+            const uint32_t n = (uint32_t)std::min<uint64_t>(kRun, c->N - r0);
+            LBX_TRY(hipMemsetAsync(box, 0, 3 * (uint64_t)n * sizeof(double), c->stream));
+            hipLaunchKernelGGL(k_mp_box, dim3(c->mp_ntiles), dim3(kBlock), 0, c->stream, src, c->mpt, 0u, c->nodes,
+                               c->ntr, tracer, box, (uint32_t)r0, n);
+            LBX_TRY(hipGetLastError());
+            LBX_TRY(hipMemcpyAsync(dst + 3 * r0, box, 3 * (uint64_t)n * sizeof(double), hipMemcpyDeviceToHost,
+                                   c->stream));
+            LBX_TRY(hipStreamSynchronize(c->stream));
         }
         return LBX_OK;
     };
-    if (P) LBX_TRY(fetch(c->P[c->mp_now], P));
-    if (Pa) {
+    int st = LBX_OK;
+    if (P) st = fetch(mp_moments(c, false)[c->mp_now], P);
+    if (!st && Pa) {
         if (c->tp.ads[tracer])
-            LBX_TRY(fetch(c->Pa[c->mp_now], Pa));
+            st = fetch(mp_moments(c, true)[c->mp_now], Pa);
         else
             std::memset(Pa, 0, 3 * (size_t)c->N * sizeof(double));
     }
-    return LBX_OK;
+    dfree(box);
+    return st;
 }
 
 int lbx_mp_get(lbx_ctx* c, double* P, double* Pa) { return lbx_mp_get_tracer(c, 0, P, Pa); }

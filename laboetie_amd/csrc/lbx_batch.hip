@@ -4,19 +4,20 @@
 // Layout.  All instances share one packed fluid-node list: instance b owns the
 // node range [node_off, node_end) (node_off a multiple of 256, so every 128-
 // or 256-node tile belongs to one instance) and a range of a shared full-box
-// map array.  Populations, flux, density and the moment-propagation arrays
-// are the single-lattice arrays over the whole list (plane stride = the node
-// capacity).  tile_inst[] maps each 256-node tile to its instance, and a
-// device table of BInst entries holds every instance's geometry, physics and
-// the work of the current round.
+// map array.  Populations, flux and density are the single-lattice arrays over
+// the whole list (plane stride = the node capacity).  tile_inst[] maps each
+// 256-node tile to its instance, and a device table of BInst entries holds
+// every instance's geometry, physics and the work of the current round.
+// Moment propagation runs on its own tiles (lbx_mp.h), laid out when an
+// instance enters it: an instance whose nodes take n tiles of the list from
+// tile t on has the 2n tiles from 2t on to itself (a layout never needs more).
 //
 // One LB launch advances every instance in the LB phase by one step, one MP
 // launch every instance in the MP phase; the blocks of other instances leave
 // at once.  The per-block work is lb_step_tile / mp_step_tile, the functions
 // the single-lattice kernels run, on a per-instance view (its own step index,
 // control block, l2err slots, VACF partials), so an instance's results are
-// bit-identical to a single-lattice run of the same input (with 256-node
-// blocks; 128-node blocks group the VACF sums differently).
+// bit-identical to a single-lattice run of the same input.
 //
 // Phases (host-driven between rounds, as the single-lattice host loop does):
 // LB stage 1 -> (redo of the switch step with the force on) -> LB stage 2 ->
@@ -37,6 +38,7 @@
 #include "../../include/lbx.h"
 #include "lbx_device.h"
 #include "lbx_kernels.h"
+#include "lbx_mp.h"
 #include "lbx_tables.h"
 
 #pragma clang fp contract(off)
@@ -68,7 +70,9 @@ struct BInst {
     // this round's MP work
     int32_t mp_on, any_ads;
     int64_t mp_it0, mp_n;         // launch k runs MP step mp_it0 + k + 1 while k < mp_n
-    int32_t mp_repeat, pad_;      // every launch recomputes step mp_it0 + 1 (timing)
+    int32_t mp_repeat;            // every launch recomputes step mp_it0 + 1 (timing)
+    uint32_t mp_tile0, mp_ntiles; // its MP tiles
+    double lambda;
     TracerParams tp;
 };
 
@@ -167,125 +171,112 @@ __global__ __launch_bounds__(64) void kb_lb_finalize(const BInst* insts, unsigne
 template <typename W>
 struct BatchMpView {
     const BInst* insts;
-    const uint32_t* tile_inst;
-    const uint32_t* act;          // the 256-node tiles of the instances in the phase, ascending
-    const W* win;
-    const double* rem;
-    const W* ustar;
+    const uint32_t* tile_inst;    // of each MP tile
+    const uint32_t* act;          // the MP tiles of the instances in the phase, ascending
+    MpTiles t;
+    MpFields<W> f;
     const uint32_t* nodes;
     const uint32_t* maps;
-    double* P0;
-    double* P1;
-    double* Pa0;
-    double* Pa1;
-    double* part0;                // per-block VACF partials by step parity, indexed by BLOCK-node tile
-    double* part1;
+    double* part[2];              // VACF partials by step parity, 3 per MP tile
     double* vtrace;               // [k][inst][3]
     uint32_t vt_stride;           // instance slots per vtrace row
     Ctrl* ctrl;
-    uint64_t Np;
 };
 
-// MP launch k of a round on one BLOCK-node tile (mp_repeat: every launch
-// recomputes step mp_it0 + 1, for timing)
-template <int BLOCK, bool Wide, typename W, bool XR>
+// MP launch k of a round on one MP tile (mp_repeat: every launch recomputes
+// step mp_it0 + 1, for timing).  FP64 recomputes the incoming probabilities,
+// the FP32 forms keep them.
+template <typename W, bool GEN>
 __device__ __forceinline__ void kb_mp_tile(const BatchMpView<W>& v, uint32_t tile, int64_t k, int32_t reduce_prev) {
-    const uint32_t id = v.tile_inst[tile / (kTile / BLOCK)];
+    const uint32_t id = v.tile_inst[tile];
     if (id == kNoInst) return;
     const BInst& in = v.insts[id];
     if (!in.mp_on || k >= in.mp_n) return;
     const int64_t it = in.mp_it0 + (in.mp_repeat ? 0 : k) + 1;  // P(it) -> P(it+1); P(m) lives in buffer (m-1)&1
-    const uint32_t first = in.tile_first * (kTile / BLOCK);
     MpStepArgs<W> a;
-    a.win = v.win;
-    a.rem = v.rem;
-    a.ustar = v.ustar;
-    a.nodes = v.nodes;
-    a.map = v.maps + in.map_off;
-    a.Pn = (it - 1) & 1 ? v.P1 : v.P0;
-    a.Px = it & 1 ? v.P1 : v.P0;
-    a.Pan = (it - 1) & 1 ? v.Pa1 : v.Pa0;
-    a.Pax = it & 1 ? v.Pa1 : v.Pa0;
-    a.partials = it & 1 ? v.part1 : v.part0;
+    a.t = v.t;
+    a.fields(v.f, ((it - 1) & 1) != 0);
+    a.any_ads = in.any_ads;
+    a.partials = it & 1 ? v.part[1] : v.part[0];
     a.prev_partials = (reduce_prev && !in.mp_repeat && k > 0)
-                          ? ((it - 1) & 1 ? v.part1 : v.part0) + 3 * (uint64_t)first
+                          ? ((it - 1) & 1 ? v.part[1] : v.part[0]) + 3 * (uint64_t)in.mp_tile0
                           : nullptr;
     a.prev_vtrace = v.vtrace + ((uint64_t)(k - 1) * v.vt_stride + id) * 3;
     a.it = it;
+    a.lambda = in.lambda;
     a.ctrl = v.ctrl + id;
+    a.tp = in.tp;
+    a.nodes = v.nodes;
+    a.map = v.maps + in.map_off;
     a.dlx = in.dlx;
     a.dly = in.dly;
     a.lz = in.lz;
-    a.Nf = in.node_end;
-    a.Np = v.Np;
-    a.any_ads = in.any_ads;
-    a.tp = in.tp;
-    mp_step_tile<BLOCK, Wide, 1, W, kCoefStored, XR>(a, tile, tile == first, in.ntiles * (kTile / BLOCK));
+    if (tile == in.mp_tile0) mp_reduce_prev<1, W>(a, in.mp_ntiles);
+    mp_step_tile<1, W, std::is_same<W, double>::value, GEN>(a, tile);
 }
 
-// XR: some live instance is more than one node wide along x (the MP step's
-// reuse of the lanes' z-neighbours, compiled out for batches of 2-D instances)
-template <int BLOCK, bool Wide, typename W, bool XR>
-__global__ __launch_bounds__(BLOCK) void kb_mp_step(BatchMpView<W> v, int64_t k, int32_t reduce_prev) {
-    kb_mp_tile<BLOCK, Wide, W, XR>(v, active_tile<BLOCK>(v.act, xcd_tile()), k, reduce_prev);
+template <typename W, bool GEN>
+__global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void kb_mp_step(BatchMpView<W> v, int64_t k, int32_t reduce_prev) {
+    kb_mp_tile<W, GEN>(v, v.act[xcd_tile()], k, reduce_prev);
 }
 
-// VACF of an MP instance's last step of the round: partials of TILE-node
-// tiles, reduced by the NT threads of one block
-template <int TILE, int NT>
-__device__ __forceinline__ void kb_mp_reduce_inst(const BInst* insts, const double* part0, const double* part1,
-                                                  double* vtrace, uint32_t vt_stride, Ctrl* ctrl, uint32_t id) {
-    __shared__ double lds[NT / 64 * 3];
-    const BInst& in = insts[id];
+// VACF of an MP instance's last step of the round (one block)
+template <typename W>
+__device__ __forceinline__ void kb_mp_reduce_inst(const BatchMpView<W>& v, uint32_t id) {
+    __shared__ double lds[kBlock / 64 * 3];
+    const BInst& in = v.insts[id];
     if (!in.mp_on || in.mp_n <= 0 || in.mp_repeat) return;
     const int64_t it = in.mp_it0 + in.mp_n;
-    const uint32_t first = in.tile_first * (kTile / TILE);
-    const double* part = (it & 1 ? part1 : part0) + 3 * (uint64_t)first;
-    mp_reduce_block<3, NT>(part, in.ntiles * (kTile / TILE), vtrace + ((uint64_t)(in.mp_n - 1) * vt_stride + id) * 3,
-                           ctrl + id, 1, it, 0, 0.0, 0.0, lds);
+    const double* part = (it & 1 ? v.part[1] : v.part[0]) + 3 * (uint64_t)in.mp_tile0;
+    mp_reduce_block<3, kBlock>(part, in.mp_ntiles, v.vtrace + ((uint64_t)(in.mp_n - 1) * v.vt_stride + id) * 3,
+                               v.ctrl + id, 1, it, 0, 0.0, 0.0, lds);
 }
 
 // (one block per instance slot)
-template <int BLOCK>
-__global__ __launch_bounds__(kBlock) void kb_mp_reduce_last(const BInst* insts, const double* part0,
-                                                            const double* part1, double* vtrace, uint32_t vt_stride,
-                                                            Ctrl* ctrl) {
-    kb_mp_reduce_inst<BLOCK, kBlock>(insts, part0, part1, vtrace, vt_stride, ctrl, blockIdx.x);
+template <typename W>
+__global__ __launch_bounds__(kBlock) void kb_mp_reduce_last(BatchMpView<W> v) {
+    kb_mp_reduce_inst(v, blockIdx.x);
 }
 
-// A whole round in one cooperative launch: S_lb LB steps, the LB closing
-// reduction, S_mp MP steps and the MP closing reduction, every block looping
-// over its share of the tiles with a grid-wide barrier between steps.  The
-// per-tile work and its order of partial sums are those of the per-step
-// launches, so the results are the same bits.  Every block runs every
-// barrier: the loops have grid-uniform bounds and the per-tile functions
-// only return from the tile, never from the kernel.
-template <int BLOCK, bool Wide, typename E, typename R, typename W, bool XR>
-__global__ __launch_bounds__(BLOCK) void kb_round(BatchView<E, R> lv, BatchMpView<W> mv, int64_t S_lb, int64_t S_mp,
-                                                  uint32_t ntiles, uint32_t ninst, int32_t lb_redo_only) {
-    cooperative_groups::grid_group grid = cooperative_groups::this_grid();
-    // the tiles of XCD x (blocks b = x mod 8) are one contiguous range
+// The steps of one phase of a round in one cooperative launch: every block
+// loops over its share of the tiles with a grid-wide barrier between steps,
+// then the closing reduction.  The per-tile work and its order of partial sums
+// are those of the per-step launches, so the results are the same bits.  Every
+// block runs every barrier: the loops have grid-uniform bounds and the
+// per-tile functions only return from the tile, never from the kernel.
+// f(l) for this block's share of the logical tiles: the tiles of XCD x
+// (blocks b = x mod 8) are one contiguous range
+template <typename F>
+__device__ __forceinline__ void block_share(uint32_t ntiles, F&& f) {
     const uint32_t nb = gridDim.x, b = blockIdx.x, x = b & 7u, local = b >> 3;
     const uint32_t nblk = (nb >> 3) + (x < (nb & 7u) ? 1u : 0u);
     const uint32_t per = (ntiles + 7u) / 8u;
     const uint32_t t0 = x * per, t1 = min(ntiles, t0 + per);
-    for (int64_t k = 0; k < S_lb; ++k) {
-        for (uint32_t l = t0 + local; l < t1; l += nblk) kb_lb_tile<BLOCK, Wide, E, R>(lv, active_tile<BLOCK>(lv.act, l), k);
+    for (uint32_t l = t0 + local; l < t1; l += nblk) f(l);
+}
+
+template <int BLOCK, bool Wide, typename E, typename R>
+__global__ __launch_bounds__(BLOCK) void kb_lb_round(BatchView<E, R> v, int64_t S, uint32_t ntiles, uint32_t ninst,
+                                                     int32_t redo_only) {
+    cooperative_groups::grid_group grid = cooperative_groups::this_grid();
+    for (int64_t k = 0; k < S; ++k) {
+        block_share(ntiles, [&](uint32_t l) { kb_lb_tile<BLOCK, Wide, E, R>(v, active_tile<BLOCK>(v.act, l), k); });
         grid.sync();
     }
-    if (S_lb > 0 && !lb_redo_only) {
-        for (uint32_t id = b; id < ninst; id += nb)
-            if (threadIdx.x < 64) kb_lb_finalize_inst(lv.insts, lv.slots, lv.l2ring, lv.ctrl, id);
+    if (redo_only) return;
+    for (uint32_t id = blockIdx.x; id < ninst; id += gridDim.x)
+        if (threadIdx.x < 64) kb_lb_finalize_inst(v.insts, v.slots, v.l2ring, v.ctrl, id);
+}
+
+template <typename W, bool GEN>
+__global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void kb_mp_round(BatchMpView<W> v, int64_t S, uint32_t ntiles,
+                                                                     uint32_t ninst) {
+    cooperative_groups::grid_group grid = cooperative_groups::this_grid();
+    for (int64_t k = 0; k < S; ++k) {
+        block_share(ntiles, [&](uint32_t l) { kb_mp_tile<W, GEN>(v, v.act[l], k, 1); });
         grid.sync();
     }
-    for (int64_t k = 0; k < S_mp; ++k) {
-        for (uint32_t l = t0 + local; l < t1; l += nblk)
-            kb_mp_tile<BLOCK, Wide, W, XR>(mv, active_tile<BLOCK>(mv.act, l), k, 1);
-        grid.sync();
-    }
-    if (S_mp > 0)
-        for (uint32_t id = b; id < ninst; id += nb)
-            kb_mp_reduce_inst<BLOCK, BLOCK>(mv.insts, mv.part0, mv.part1, mv.vtrace, mv.vt_stride, mv.ctrl, id);
+    for (uint32_t id = blockIdx.x; id < ninst; id += gridDim.x) kb_mp_reduce_inst(v, id);
 }
 
 // ------------------------------------------------------------------ host
@@ -373,6 +364,7 @@ struct HostInst {
     double Db = 0, ka = 0, kd = 0, lambda = 0;
     int64_t t = 0, max_lb = 0, switch_step = INT64_MAX, check_after = 2;
     int64_t mp_it = 0, mp_target = 0;
+    bool general = false;           // its MP steps need the general kernel (lbx_mp.h)
     std::vector<uint32_t> nodes_h;  // full-box index | interfacial bit
     std::vector<double> vacf;       // (mp_it+1) x 3
     double deff[3] = {0, 0, 0};
@@ -384,7 +376,7 @@ struct HostInst {
 struct lbxb {
     int32_t prec = LBX_PREC_FP64;
     bool wide = false;       // 64-bit addressing of the population buffers
-    uint32_t n_xrows = 0;    // live instances more than one node wide along x
+    uint32_t n_general = 0;  // live instances whose MP steps need the general kernel
     bool wide_auto = false;  // what the capacity alone selects
     uint64_t Np = 0, cap_box = 0;
     uint32_t cap_inst = 0, ntiles_cap = 0;
@@ -409,20 +401,22 @@ struct lbxb {
     unsigned long long* slots = nullptr;
     double* l2ring = nullptr;
     Ctrl* ctrl = nullptr;
-    double* win = nullptr;
-    float* win32 = nullptr;
-    double* ustar = nullptr;
-    float* ustar32 = nullptr;
-    double* rem = nullptr;
-    double* P[2] = {nullptr, nullptr};
-    double* Pa[2] = {nullptr, nullptr};
+    MpTiles mpt;                 // MP tiles: 2 ntiles_cap
+    uint32_t* mp_tile_inst = nullptr;
+    MpFields<double> mpf;        // FP64 form
+    MpFields<float> mpf32;       // FP32-storage forms
+    uint32_t* walk = nullptr;    // scratch of the layout builds, grown as needed
+    uint64_t walk_cap = 0;
+    MpBuild* builds = nullptr;   // [max instances]
+    MpBuilt* built = nullptr;
+    uint8_t* split = nullptr;
     double* part[2] = {nullptr, nullptr};
     double* vtrace = nullptr;
     // host state
     std::vector<BInst> tab;
     std::vector<Ctrl> ctrl_h;  // per instance slot: what reset_inst_ctrl uploads (kept until the stream syncs)
     std::vector<HostInst> hi;
-    std::vector<uint32_t> tile_inst_h;
+    std::vector<uint32_t> tile_inst_h, mp_tile_inst_h;
     // the tiles of the instances with LB (0) or MP (1) work in the launches
     // about to run (built by upload_active; host copy kept until the stream syncs)
     uint32_t* act[2] = {nullptr, nullptr};
@@ -433,8 +427,8 @@ struct lbxb {
     struct Graph {
         hipGraphExec_t exec = nullptr;
         int32_t block = 0;
-        uint32_t grid_tiles = 0;  // active 256-node tiles of the phase
-        bool xr = false;  // the MP launches' kernel reuses the lanes' z-neighbours
+        uint32_t grid_tiles = 0;  // active tiles of the phase
+        bool general = false;     // the MP launches run the general kernel
     };
     std::map<std::pair<int, int64_t>, Graph> graph_cache;
     // statistics
@@ -455,8 +449,6 @@ void free_all(lbxb* b) {
     for (int k = 0; k < 2; ++k) {
         dfree(b->f[k]);
         dfree(b->g[k]);
-        dfree(b->P[k]);
-        dfree(b->Pa[k]);
         dfree(b->part[k]);
     }
     dfree(b->j32);
@@ -471,11 +463,29 @@ void free_all(lbxb* b) {
     dfree(b->slots);
     dfree(b->l2ring);
     dfree(b->ctrl);
-    dfree(b->win);
-    dfree(b->win32);
-    dfree(b->ustar);
-    dfree(b->ustar32);
-    dfree(b->rem);
+    auto fields = [](auto& f) {
+        dfree(f.rv);
+        dfree(f.win);
+        dfree(f.rem);
+        dfree(f.ustar);
+        for (int k = 0; k < 2; ++k) {
+            dfree(f.P[k]);
+            dfree(f.Pa[k]);
+        }
+    };
+    fields(b->mpf);
+    fields(b->mpf32);
+    dfree(b->mpt.info);
+    dfree(b->mpt.halo);
+    dfree(b->mpt.tab4);
+    dfree(b->mpt.tab2);
+    dfree(b->mpt.perm);
+    dfree(b->mpt.inv);
+    dfree(b->mp_tile_inst);
+    dfree(b->walk);
+    dfree(b->builds);
+    dfree(b->built);
+    dfree(b->split);
     dfree(b->vtrace);
     for (auto& e : b->ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
@@ -500,7 +510,10 @@ int reset_inst_ctrl(lbxb* b, uint32_t id, int64_t check_after) {
     return hip_status(hipMemcpyAsync(b->ctrl + id, &h, sizeof(Ctrl), hipMemcpyHostToDevice, b->stream));
 }
 
-uint32_t grid_of(const lbxb* b, int block, int phase /*0 LB, 1 MP*/) { return b->n_act[phase] * (kTile / block); }
+// blocks of a launch: LB tiles are cut into blocks, MP tiles are one block each
+uint32_t grid_of(const lbxb* b, int block, int phase /*0 LB, 1 MP*/) {
+    return phase == 0 ? b->n_act[0] * (kTile / block) : b->n_act[1];
+}
 
 // The active tile lists of the work table as it stands (lb_on / mp_on), for
 // the launches that follow; call after the table changes which instances take
@@ -508,10 +521,11 @@ uint32_t grid_of(const lbxb* b, int block, int phase /*0 LB, 1 MP*/) { return b-
 int upload_active(lbxb* b) {
     LBX_TRY(hipStreamSynchronize(b->stream));  // the previous lists' uploads have been read
     for (int ph = 0; ph < 2; ++ph) {
-        std::vector<std::pair<uint32_t, uint32_t>> r;  // (tile_first, ntiles) of the phase's instances
+        std::vector<std::pair<uint32_t, uint32_t>> r;  // (first tile, tiles) of the phase's instances
         for (uint32_t id = 0; id < b->cap_inst; ++id) {
             const BInst& in = b->tab[id];
-            if (ph == 0 ? in.lb_on : in.mp_on) r.emplace_back(in.tile_first, in.ntiles);
+            if (ph == 0 && in.lb_on) r.emplace_back(in.tile_first, in.ntiles);
+            if (ph == 1 && in.mp_on) r.emplace_back(in.mp_tile0, in.mp_ntiles);
         }
         std::sort(r.begin(), r.end());
         std::vector<uint32_t>& a = b->act_h[ph];
@@ -551,31 +565,25 @@ BatchView<E, R> lb_view(lbxb* b) {
 }
 
 template <typename W>
+MpFields<W>& mp_fields(lbxb* b) {
+    if constexpr (std::is_same<W, float>::value) return b->mpf32; else return b->mpf;
+}
+
+template <typename W>
 BatchMpView<W> mp_view(lbxb* b) {
     BatchMpView<W> v;
     v.insts = b->insts;
-    v.tile_inst = b->tile_inst;
+    v.tile_inst = b->mp_tile_inst;
     v.act = b->act[1];
-    if constexpr (std::is_same<W, float>::value) {
-        v.win = b->win32;
-        v.ustar = b->ustar32;
-    } else {
-        v.win = b->win;
-        v.ustar = b->ustar;
-    }
-    v.rem = b->rem;
+    v.t = b->mpt;
+    v.f = mp_fields<W>(b);
     v.nodes = b->nodes;
     v.maps = b->maps;
-    v.P0 = b->P[0];
-    v.P1 = b->P[1];
-    v.Pa0 = b->Pa[0];
-    v.Pa1 = b->Pa[1];
-    v.part0 = b->part[0];
-    v.part1 = b->part[1];
+    v.part[0] = b->part[0];
+    v.part[1] = b->part[1];
     v.vtrace = b->vtrace;
     v.vt_stride = b->cap_inst;
     v.ctrl = b->ctrl;
-    v.Np = b->Np;
     return v;
 }
 
@@ -619,24 +627,19 @@ void launch_lb(lbxb* b, int64_t k, int block) {
     });
 }
 
-void launch_mp(lbxb* b, int64_t k, int block, int reduce_prev) {
-    const uint32_t grid = grid_of(b, block, 1);
+void launch_mp(lbxb* b, int64_t k, int reduce_prev) {
+    const uint32_t grid = grid_of(b, kBlock, 1);
     if (!grid) return;
-    const bool xr = b->n_xrows > 0;
-    with_block(block, [&](auto BT) {
-        constexpr int BL = decltype(BT)::value;
-        if (shift(b)) {
-            auto v = mp_view<float>(b);
-            auto kern = b->wide ? (xr ? kb_mp_step<BL, true, float, true> : kb_mp_step<BL, true, float, false>)
-                                : (xr ? kb_mp_step<BL, false, float, true> : kb_mp_step<BL, false, float, false>);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(BL), 0, b->stream, v, k, reduce_prev);
-        } else {
-            auto v = mp_view<double>(b);
-            auto kern = b->wide ? (xr ? kb_mp_step<BL, true, double, true> : kb_mp_step<BL, true, double, false>)
-                                : (xr ? kb_mp_step<BL, false, double, true> : kb_mp_step<BL, false, double, false>);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(BL), 0, b->stream, v, k, reduce_prev);
-        }
-    });
+    const bool gen = b->n_general > 0;
+    auto go = [&](auto wtag) {
+        using W = decltype(wtag);
+        auto kern = gen ? kb_mp_step<W, true> : kb_mp_step<W, false>;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, b->stream, mp_view<W>(b), k, reduce_prev);
+    };
+    if (shift(b))
+        go(float{});
+    else
+        go(double{});
 }
 
 void launch_lb_finalize(lbxb* b) {
@@ -644,30 +647,30 @@ void launch_lb_finalize(lbxb* b) {
                        b->ctrl);
 }
 
-void launch_mp_reduce_last(lbxb* b, int block) {
-    with_block(block, [&](auto BT) {
-        constexpr int BL = decltype(BT)::value;
-        hipLaunchKernelGGL(kb_mp_reduce_last<BL>, dim3(b->cap_inst), dim3(kBlock), 0, b->stream, b->insts,
-                           b->part[0], b->part[1], b->vtrace, b->cap_inst, b->ctrl);
-    });
+void launch_mp_reduce_last(lbxb* b) {
+    if (shift(b))
+        hipLaunchKernelGGL(kb_mp_reduce_last<float>, dim3(b->cap_inst), dim3(kBlock), 0, b->stream, mp_view<float>(b));
+    else
+        hipLaunchKernelGGL(kb_mp_reduce_last<double>, dim3(b->cap_inst), dim3(kBlock), 0, b->stream,
+                           mp_view<double>(b));
 }
 
 // the S launches of one phase of a round (+ its closing reduction), replayed
 // from a captured graph when graphs are on
 int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
     if (S <= 0) return LBX_OK;
-    const int block = phase == 0 ? b->lb_block : b->mp_block;
+    const int block = phase == 0 ? b->lb_block : kBlock;
     auto emit = [&]() {
         for (int64_t k = 0; k < S; ++k) {
             if (phase == 0)
                 launch_lb(b, k, block);
             else
-                launch_mp(b, k, block, 1);
+                launch_mp(b, k, 1);
         }
         if (phase == 0)
             launch_lb_finalize(b);
         else
-            launch_mp_reduce_last(b, block);
+            launch_mp_reduce_last(b);
     };
     if (!b->graphs) {
         emit();
@@ -675,9 +678,9 @@ int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
     }
     auto key = std::make_pair(phase, S);
     auto it = b->graph_cache.find(key);
-    const bool xr = b->n_xrows > 0;
+    const bool gen = phase == 1 && b->n_general > 0;
     if (it != b->graph_cache.end() &&
-        (it->second.block != block || it->second.grid_tiles != b->n_act[phase] || it->second.xr != xr)) {
+        (it->second.block != block || it->second.grid_tiles != b->n_act[phase] || it->second.general != gen)) {
         (void)hipGraphExecDestroy(it->second.exec);
         b->graph_cache.erase(it);
         it = b->graph_cache.end();
@@ -698,49 +701,50 @@ int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
         if (ie != hipSuccess) return hip_status(ie);
         gr.block = block;
         gr.grid_tiles = b->n_act[phase];
-        gr.xr = xr;
+        gr.general = gen;
         it = b->graph_cache.emplace(key, gr).first;
     }
     return hip_status(hipGraphLaunch(it->second.exec, b->stream));
 }
 
-// One phase of a round as a single cooperative launch of kb_round (grid: as
-// many blocks as can be resident at once, at most one per tile)
+// One phase of a round as a single cooperative launch (grid: as many blocks as
+// can be resident at once, at most one per tile)
 int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
     if (S <= 0) return LBX_OK;
-    const int block = b->lb_block;
-    const uint32_t ntiles = grid_of(b, block, phase);
-    if (!ntiles) return LBX_OK;
-    const bool xr = b->n_xrows > 0;
-    auto go = [&](auto etag, auto rtag, auto btag, auto wide) -> int {
+    uint32_t nt = grid_of(b, b->lb_block, phase), ni = b->cap_inst;
+    if (!nt) return LBX_OK;
+    auto launch = [&](auto kern, int block, void** args) -> int {
+        int per_cu = 0;
+        LBX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, 0));
+        if (per_cu <= 0) return LBX_ERR_DEVICE;
+        const uint32_t grid = std::min<uint32_t>(nt, (uint32_t)per_cu * (uint32_t)b->num_cu);
+        return hip_status(hipLaunchCooperativeKernel((const void*)kern, dim3(grid), dim3(block), args, 0, b->stream));
+    };
+    if (phase == 1) {
+        auto go = [&](auto wtag) -> int {
+            using W = decltype(wtag);
+            BatchMpView<W> v = mp_view<W>(b);
+            void* args[] = {&v, &S, &nt, &ni};
+            return launch(b->n_general > 0 ? kb_mp_round<W, true> : kb_mp_round<W, false>, kBlock, args);
+        };
+        return shift(b) ? go(float{}) : go(double{});
+    }
+    auto go = [&](auto etag, auto rtag, auto btag) -> int {
         using E = decltype(etag);  // population storage
         using R = decltype(rtag);  // LB arithmetic
-        using W = E;               // MP probabilities are stored like the populations
         constexpr int BL = decltype(btag)::value;
-        constexpr bool WD = decltype(wide)::value;
-        auto kern = xr ? kb_round<BL, WD, E, R, W, true> : kb_round<BL, WD, E, R, W, false>;
-        int per_cu = 0;
-        LBX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, BL, 0));
-        if (per_cu <= 0) return LBX_ERR_DEVICE;
-        const uint32_t grid = std::min<uint32_t>(ntiles, (uint32_t)per_cu * (uint32_t)b->num_cu);
-        BatchView<E, R> lv = lb_view<E, R>(b);
-        BatchMpView<W> mv = mp_view<W>(b);
-        int64_t S_lb = phase == 0 ? S : 0, S_mp = phase == 1 ? S : 0;
-        uint32_t nt = ntiles, ni = b->cap_inst;
-        int32_t ro = redo_only;
-        void* args[] = {&lv, &mv, &S_lb, &S_mp, &nt, &ni, &ro};
-        return hip_status(hipLaunchCooperativeKernel((const void*)kern, dim3(grid), dim3(BL), args, 0, b->stream));
+        BatchView<E, R> v = lb_view<E, R>(b);
+        void* args[] = {&v, &S, &nt, &ni, &redo_only};
+        return launch(b->wide ? kb_lb_round<BL, true, E, R> : kb_lb_round<BL, false, E, R>, BL, args);
     };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
     int st = LBX_OK;
-    with_block(block, [&](auto BT) {
+    with_block(b->lb_block, [&](auto BT) {
         if (b->prec == LBX_PREC_FP32_SHIFT)
-            st = b->wide ? go(float{}, float{}, BT, T_{}) : go(float{}, float{}, BT, F_{});
+            st = go(float{}, float{}, BT);
         else if (b->prec == LBX_PREC_FP32_STORE)
-            st = b->wide ? go(float{}, double{}, BT, T_{}) : go(float{}, double{}, BT, F_{});
+            st = go(float{}, double{}, BT);
         else
-            st = b->wide ? go(double{}, double{}, BT, T_{}) : go(double{}, double{}, BT, F_{});
+            st = go(double{}, double{}, BT);
     });
     return st;
 }
@@ -751,94 +755,175 @@ int download(lbxb* b, const T* src, uint64_t count, T* dst) {
     return hip_status(hipStreamSynchronize(b->stream));
 }
 
-// extract + MP prep + VACF(0) of instance id, whose LB phase ended at step t
-int mp_setup_inst(lbxb* b, uint32_t id) {
-    HostInst& h = b->hi[id];
-    BInst& in = b->tab[id];
-    const int64_t t = h.t;
-    const uint32_t gt = in.ntiles;
-    const uint32_t* map = b->maps + in.map_off;
-    if (t > 0) {
-        const int src = (t - 1) & 1, dst = t & 1;
-        if (shift(b)) {
-            const double* Ft = t > h.switch_step ? h.F : nullptr;
-            const double fm[3] = {Ft ? Ft[0] / 2.0 : 0.0, Ft ? Ft[1] / 2.0 : 0.0, Ft ? Ft[2] / 2.0 : 0.0};
-            hipLaunchKernelGGL(k_extract_shift, dim3(gt), dim3(kBlock), 0, b->stream, b->g[src], b->g[dst], b->rho,
-                               b->j, b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end, b->Np, in.rho0,
-                               fm[0], fm[1], fm[2]);
-        } else {
-            hipLaunchKernelGGL(k_extract, dim3(gt), dim3(kBlock), 0, b->stream, b->f[src], b->f[dst], b->rho,
-                               b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end, b->Np);
-        }
+// MP layouts of the instances ids, built together (lbx_mp.h; as build_tiles of
+// the single-lattice path, so an instance gets the same tiles there and here)
+int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
+    std::vector<MpBuild> builds(ids.size());
+    std::vector<MpBuilt> built(ids.size());
+    uint64_t walk = 0;
+    for (size_t k = 0; k < ids.size(); ++k) {
+        const HostInst& h = b->hi[ids[k]];
+        const BInst& in = b->tab[ids[k]];
+        MpBuild& d = builds[k];
+        d = MpBuild{};
+        d.b = make_bricks((uint32_t)h.lx, (uint32_t)h.ly, (uint32_t)h.lz);
+        d.nodes = b->nodes;
+        d.map = b->maps + in.map_off;
+        d.dlx = in.dlx;
+        d.dly = in.dly;
+        d.order_off = (uint32_t)walk;
+        d.tile0 = 2 * in.tile_first;
+        d.bound = mp_tile_bound(h.Nf);  // 2 in.ntiles
+        walk += d.b.norder;
     }
-    const double eps = DBL_EPSILON;
-    TracerParams tp{};
-    const double K = (std::fabs(h.kd) <= eps) ? 0.0 : h.ka / h.kd;  // module_moment_propagation.f90:46-50
-    tp.ads[0] = std::fabs(K) > eps;                                 // :52-56
-    tp.bw[0] = 1.0 / ((double)h.Nf + K * (double)h.nfi);            // :97
-    tp.ka[0] = h.ka;
-    tp.kd[0] = h.kd;
-    tp.one_minus_kd[0] = 1.0 - h.kd;
-    in.tp = tp;
-    in.any_ads = tp.ads[0];
-    const uint64_t n = (uint64_t)gt * kTile;
-    // Pa = 0 on the instance's range of both buffers (comp_index layout: pair plane + single plane)
-    for (int k = 0; k < 2; ++k) {
-        LBX_TRY(hipMemsetAsync(b->Pa[k] + 2 * (uint64_t)in.node_off, 0, 2 * n * sizeof(double), b->stream));
-        LBX_TRY(hipMemsetAsync(b->Pa[k] + 2 * b->Np + in.node_off, 0, n * sizeof(double), b->stream));
+    if (walk > b->walk_cap) {  // counts and bases
+        dfree(b->walk);
+        b->walk_cap = 0;
+        LBX_TRY(dalloc(&b->walk, 2 * walk));
+        b->walk_cap = walk;
     }
-    LBX_TRY(reset_inst_ctrl(b, id, 2));
-    auto prep = [&](auto wtag) {
-        using W = decltype(wtag);
-        MpPrepArgs<W> a;
-        a.rho = b->rho;
-        a.j = b->j;
-        a.nodes = b->nodes;
-        a.map = map;
-        if constexpr (std::is_same<W, float>::value) {
-            a.win = b->win32;
-            a.ustar = b->ustar32;
-        } else {
-            a.win = b->win;
-            a.ustar = b->ustar;
+    uint32_t *count = b->walk, *base = b->walk + walk;
+    // one pass over the lattices `which`; general: keep what has an LDS slot
+    auto pass = [&](const std::vector<size_t>& which, bool counted, const uint8_t* by, uint8_t* mark,
+                    bool general) -> int {
+        std::vector<MpBuild> d;
+        uint32_t gw = 0, gt = 0;
+        for (size_t k : which) {
+            d.push_back(builds[k]);
+            gw = std::max(gw, (builds[k].b.norder + kBlock / 64 - 1) / (kBlock / 64));
+            gt = std::max(gt, builds[k].bound);
         }
-        a.rem = b->rem;
-        a.P0 = b->P[0];
-        a.partials = b->part[0];
-        a.ctrl = b->ctrl + id;
-        a.dlx = in.dlx;
-        a.dly = in.dly;
-        a.lz = in.lz;
-        a.Nf = in.node_end;
-        a.Np = b->Np;
-        a.fx = h.F[0];
-        a.fy = h.F[1];
-        a.fz = h.F[2];
-        a.lambda = h.lambda;
-        a.eps = eps;
-        a.tile0 = in.tile_first;
-        a.tp = tp;
-        hipLaunchKernelGGL((k_mp_prep<1, W>), dim3(gt), dim3(kBlock), 0, b->stream, a);
-    };
-    if (shift(b))
-        prep(float{});
-    else
-        prep(double{});
-    hipLaunchKernelGGL(k_mp_reduce<3>, dim3(1), dim3(kBlock), 0, b->stream, b->part[0] + 3 * (uint64_t)in.tile_first,
-                       gt, nullptr, b->ctrl + id, 0, (int64_t)0, 0, 0.0, 0.0);
-    LBX_TRY(hipGetLastError());
-    Ctrl c;
-    LBX_TRY(download(b, b->ctrl + id, 1, &c));
-    if (c.restpart) {
-        h.phase = kFailed;
-        h.status = LBX_ERR_RESTPART;
+        const uint32_t nd = (uint32_t)d.size();
+        LBX_TRY(hipMemcpyAsync(b->builds, d.data(), nd * sizeof(MpBuild), hipMemcpyHostToDevice, b->stream));
+        if (!counted)
+            hipLaunchKernelGGL(k_mpb_count, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, count);
+        hipLaunchKernelGGL(k_mpb_group, dim3(nd), dim3(kBlock), 0, b->stream, b->builds, b->built, count, base,
+                           b->mpt.info, by);
+        hipLaunchKernelGGL(k_mpb_place, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, b->built, base,
+                           b->mpt.perm, b->mpt.inv);
+        hipLaunchKernelGGL((general ? k_mpb_table<true> : k_mpb_table<false>), dim3(gt, nd), dim3(kBlock), 0,
+                           b->stream, b->builds, b->built, b->mpt, mark);
+        LBX_TRY(hipGetLastError());
+        std::vector<MpBuilt> r(nd);
+        LBX_TRY(hipMemcpyAsync(r.data(), b->built, nd * sizeof(MpBuilt), hipMemcpyDeviceToHost, b->stream));
+        LBX_TRY(hipStreamSynchronize(b->stream));
+        for (uint32_t k = 0; k < nd; ++k) built[which[k]] = r[k];
         return LBX_OK;
+    };
+    std::vector<size_t> all, again, gen;
+    for (size_t k = 0; k < ids.size(); ++k) all.push_back(k);
+    LBX_TRY(pass(all, false, nullptr, b->split, false));
+    for (size_t k : all)
+        if (built[k].halo_max > kHaloMax) again.push_back(k);
+    if (!again.empty()) {
+        LBX_TRY(pass(again, true, b->split, nullptr, false));
+        for (size_t k : again)
+            if (built[k].ntiles == 0) gen.push_back(k);
+        if (!gen.empty()) LBX_TRY(pass(gen, true, nullptr, nullptr, true));
     }
-    h.vacf.assign(c.vacf0, c.vacf0 + 3);
-    h.mp_it = 0;
-    h.phase = h.mp_target > 0 ? kMp : kDone;
-    if (h.phase == kDone)
-        for (int a_ = 0; a_ < 3; ++a_) h.deff[a_] = c.deff_s[a_] + c.deff_c[a_];
+    for (size_t k = 0; k < ids.size(); ++k) {
+        BInst& in = b->tab[ids[k]];
+        in.mp_tile0 = 2 * in.tile_first;
+        in.mp_ntiles = built[k].ntiles;
+        for (uint32_t t = 0; t < 2 * in.ntiles; ++t)
+            b->mp_tile_inst_h[in.mp_tile0 + t] = t < in.mp_ntiles ? ids[k] : kNoInst;
+        LBX_TRY(hipMemcpyAsync(b->mp_tile_inst + in.mp_tile0, b->mp_tile_inst_h.data() + in.mp_tile0,
+                               2 * (uint64_t)in.ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
+    }
+    for (size_t k : gen) b->hi[ids[k]].general = true;
+    return LBX_OK;
+}
+
+template <typename W>
+void launch_mp_prep(lbxb* b, uint32_t id, double eps) {
+    const HostInst& h = b->hi[id];
+    const BInst& in = b->tab[id];
+    MpPrepArgs<W> a;
+    a.t = b->mpt;
+    a.f = mp_fields<W>(b);
+    a.rho = b->rho;
+    a.j = b->j;
+    a.nodes = b->nodes;
+    a.map = b->maps + in.map_off;
+    a.partials = b->part[0];
+    a.ctrl = b->ctrl + id;
+    a.dlx = in.dlx;
+    a.dly = in.dly;
+    a.lz = in.lz;
+    a.Np = b->Np;
+    a.fx = h.F[0];
+    a.fy = h.F[1];
+    a.fz = h.F[2];
+    a.lambda = in.lambda;
+    a.eps = eps;
+    a.tp = in.tp;
+    hipLaunchKernelGGL((k_mp_prep<1, W>), dim3(in.mp_ntiles), dim3(kBlock), 0, b->stream, a, in.mp_tile0);
+}
+
+// extract + MP layout + prep + VACF(0) of the instances ids, whose LB phases
+// have ended: launched for all of them, then read back at once
+int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
+    if (ids.empty()) return LBX_OK;
+    LBX_TRY(build_tiles(b, ids));
+    const double eps = DBL_EPSILON;
+    for (uint32_t id : ids) {
+        HostInst& h = b->hi[id];
+        BInst& in = b->tab[id];
+        const int64_t t = h.t;
+        const uint32_t gt = in.ntiles;
+        const uint32_t* map = b->maps + in.map_off;
+        if (t > 0) {
+            const int src = (t - 1) & 1, dst = t & 1;
+            if (shift(b)) {
+                const double* Ft = t > h.switch_step ? h.F : nullptr;
+                const double fm[3] = {Ft ? Ft[0] / 2.0 : 0.0, Ft ? Ft[1] / 2.0 : 0.0, Ft ? Ft[2] / 2.0 : 0.0};
+                hipLaunchKernelGGL(k_extract_shift, dim3(gt), dim3(kBlock), 0, b->stream, b->g[src], b->g[dst],
+                                   b->rho, b->j, b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end,
+                                   b->Np, in.rho0, fm[0], fm[1], fm[2]);
+            } else {
+                hipLaunchKernelGGL(k_extract, dim3(gt), dim3(kBlock), 0, b->stream, b->f[src], b->f[dst], b->rho,
+                                   b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end, b->Np);
+            }
+        }
+        TracerParams tp{};
+        const double K = (std::fabs(h.kd) <= eps) ? 0.0 : h.ka / h.kd;  // module_moment_propagation.f90:46-50
+        tp.ads[0] = std::fabs(K) > eps;                                 // :52-56
+        tp.bw[0] = 1.0 / ((double)h.Nf + K * (double)h.nfi);            // :97
+        tp.ka[0] = h.ka;
+        tp.kd[0] = h.kd;
+        tp.one_minus_kd[0] = 1.0 - h.kd;
+        in.tp = tp;
+        in.any_ads = tp.ads[0];
+        in.lambda = h.lambda;
+        LBX_TRY(reset_inst_ctrl(b, id, 2));
+        if (shift(b))
+            launch_mp_prep<float>(b, id, eps);
+        else
+            launch_mp_prep<double>(b, id, eps);
+        hipLaunchKernelGGL(k_mp_reduce<3>, dim3(1), dim3(kBlock), 0, b->stream,
+                           b->part[0] + 3 * (uint64_t)in.mp_tile0, in.mp_ntiles, nullptr, b->ctrl + id, 0,
+                           (int64_t)0, 0, 0.0, 0.0);
+    }
+    LBX_TRY(hipGetLastError());
+    std::vector<Ctrl> ctrl(b->cap_inst);
+    LBX_TRY(download(b, b->ctrl, b->cap_inst, ctrl.data()));
+    for (uint32_t id : ids) {
+        HostInst& h = b->hi[id];
+        const Ctrl& c = ctrl[id];
+        if (c.restpart) {
+            h.phase = kFailed;
+            h.status = LBX_ERR_RESTPART;
+            h.general = false;  // it takes no step
+            continue;
+        }
+        h.general = h.general || (!shift(b) && c.mp_divide);
+        if (h.general) ++b->n_general;
+        h.vacf.assign(c.vacf0, c.vacf0 + 3);
+        h.mp_it = 0;
+        h.phase = h.mp_target > 0 ? kMp : kDone;
+        if (h.phase == kDone)
+            for (int a_ = 0; a_ < 3; ++a_) h.deff[a_] = c.deff_s[a_] + c.deff_c[a_];
+    }
     return LBX_OK;
 }
 
@@ -855,7 +940,11 @@ int64_t lbxb_footprint_bytes(int32_t precision, int64_t capacity_nodes, int64_t 
     uint64_t by = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + Np * 4 +
                   (uint64_t)capacity_box * 4 + Np / kTile * 4;
     by += (uint64_t)max_instances * (sizeof(BInst) + 3 * kSlots * 8 + kRing * 8 + sizeof(Ctrl));
-    by += (18 + 3) * Np * pop + Np * 8 + 4 * 3 * Np * 8 + 2 * 2 * (Np / 128) * 3 * 8;
+    // MP: twice the nodes' entries (probabilities or (rho, v), rem, u*, P and Pa twice, slot table, node),
+    // halo lists, partials, each node's entry
+    const uint64_t M = 2 * Np;
+    by += M * ((pop == 8 ? 4 * 8 : 18 * 4) + 8 + 3 * pop + 4 * 3 * 8 + 24 + 4) +
+          M / kTile * (kHaloMaxGen * 4 + 2 * 3 * 8 + 3 * 4 + 1) + Np * 4;
     by += (uint64_t)kRoundMax * max_instances * 3 * 8;
     return (int64_t)by;
 }
@@ -891,9 +980,7 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
     for (int k = 0; k < 2; ++k) {
         if (!st && !sh) st = dalloc(&b->f[k], kQ * Np);
         if (!st && sh) st = dalloc(&b->g[k], kQ * Np);
-        if (!st) st = dalloc(&b->P[k], 3 * Np);
-        if (!st) st = dalloc(&b->Pa[k], 3 * Np);
-        if (!st) st = dalloc(&b->part[k], (Np / 64) * 3);  // one VACF partial per 64-node block
+        if (!st) st = dalloc(&b->part[k], 2 * (uint64_t)b->ntiles_cap * 3);
     }
     if (!st && precision == LBX_PREC_FP32_SHIFT) st = dalloc(&b->j32, 3 * Np);
     if (!st) st = dalloc(&b->j, 3 * Np);
@@ -902,16 +989,38 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
     if (!st) st = dalloc(&b->maps, (uint64_t)capacity_box);
     if (!st) st = dalloc(&b->tile_inst, (uint64_t)b->ntiles_cap);
     if (!st) st = dalloc(&b->act[0], (uint64_t)b->ntiles_cap);
-    if (!st) st = dalloc(&b->act[1], (uint64_t)b->ntiles_cap);
+    if (!st) st = dalloc(&b->act[1], 2 * (uint64_t)b->ntiles_cap);
     if (!st) st = dalloc(&b->insts, (uint64_t)max_instances);
     if (!st) st = dalloc(&b->slots, (uint64_t)max_instances * 3 * kSlots);
     if (!st) st = dalloc(&b->l2ring, (uint64_t)max_instances * kRing);
     if (!st) st = dalloc(&b->ctrl, (uint64_t)max_instances);
-    if (!st && !sh) st = dalloc(&b->win, 18 * Np);
-    if (!st && !sh) st = dalloc(&b->ustar, 3 * Np);
-    if (!st && sh) st = dalloc(&b->win32, 18 * Np);
-    if (!st && sh) st = dalloc(&b->ustar32, 3 * Np);
-    if (!st) st = dalloc(&b->rem, Np);
+    const uint64_t M = 2 * Np;  // entries of the MP tiles
+    auto fields = [&](auto& f) {
+        if (!st) st = dalloc(&f.rem, M);
+        if (!st) st = dalloc(&f.ustar, 3 * M);
+        for (int k = 0; k < 2; ++k) {
+            if (!st) st = dalloc(&f.P[k], 3 * M);
+            if (!st) st = dalloc(&f.Pa[k], 3 * M);
+        }
+    };
+    if (sh) {
+        fields(b->mpf32);
+        if (!st) st = dalloc(&b->mpf32.win, 9 * M);
+    } else {
+        fields(b->mpf);
+        if (!st) st = dalloc(&b->mpf.rv, 2 * M);
+    }
+    b->mpt.pitch = kHaloMaxGen;
+    if (!st) st = dalloc(&b->mpt.info, M / kTile);
+    if (!st) st = dalloc(&b->mpt.halo, M / kTile * b->mpt.pitch);
+    if (!st) st = dalloc(&b->mpt.tab4, M);
+    if (!st) st = dalloc(&b->mpt.tab2, M);
+    if (!st) st = dalloc(&b->mpt.perm, M);
+    if (!st) st = dalloc(&b->mpt.inv, Np);
+    if (!st) st = dalloc(&b->mp_tile_inst, M / kTile);
+    if (!st) st = dalloc(&b->split, M / kTile);
+    if (!st) st = dalloc(&b->builds, (uint64_t)max_instances);
+    if (!st) st = dalloc(&b->built, (uint64_t)max_instances);
     if (!st) st = dalloc(&b->vtrace, (uint64_t)kRoundMax * max_instances * 3);
     if (!st && (hipEventCreate(&b->ev[0]) != hipSuccess || hipEventCreate(&b->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
@@ -920,6 +1029,7 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
         b->ctrl_h.assign(max_instances, Ctrl{});
         b->hi.assign(max_instances, HostInst{});
         b->tile_inst_h.assign(b->ntiles_cap, kNoInst);
+        b->mp_tile_inst_h.assign(2 * (size_t)b->ntiles_cap, kNoInst);
         b->node_alloc.init(b->ntiles_cap);
         b->map_alloc.init(b->cap_box);
         st = hip_status(hipMemcpyAsync(b->tile_inst, b->tile_inst_h.data(), b->ntiles_cap * sizeof(uint32_t),
@@ -1058,7 +1168,6 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     }
     b->tab[id] = in;
     b->hi[id] = std::move(h);
-    if (lx > 1) ++b->n_xrows;
     *id_out = (int32_t)id;
     return LBX_OK;
 }
@@ -1072,7 +1181,7 @@ int lbxb_remove(lbxb* b, int32_t id) {
                            in.ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
     b->node_alloc.give(in.tile_first, in.ntiles);
     b->map_alloc.give(in.map_off, b->hi[id].map_n);
-    if (b->hi[id].lx > 1) --b->n_xrows;
+    if (b->hi[id].general) --b->n_general;
     b->hi[id] = HostInst{};
     in = BInst{};
     return hip_status(hipStreamSynchronize(b->stream));
@@ -1230,7 +1339,7 @@ int lbxb_round(lbxb* b, int32_t lb_steps, int32_t mp_steps, int32_t* active) {
     b->lb_fluid_updates += lb_fluid;
     b->mp_box_updates += mp_box;
     b->mp_fluid_updates += mp_fluid;
-    for (uint32_t id : to_mp) LBX_TRY(mp_setup_inst(b, id));
+    LBX_TRY(mp_setup_insts(b, to_mp));
     int32_t n = 0;
     for (uint32_t id = 0; id < ni; ++id) n += b->hi[id].phase >= kLb && b->hi[id].phase <= kMp;
     if (active) *active = n;
@@ -1363,7 +1472,7 @@ int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_bloc
     LBX_TRY(hipMemcpyAsync(b->insts, b->tab.data(), ni * sizeof(BInst), hipMemcpyHostToDevice, b->stream));
     LBX_TRY(upload_active(b));
     auto launch = [&](int phase, int block) {
-        if (phase == 0) launch_lb(b, 0, block); else launch_mp(b, 0, block, 0);
+        if (phase == 0) launch_lb(b, 0, block); else launch_mp(b, 0, 0);
     };
     auto elapsed = [&](double* out) -> int {
         LBX_TRY(hipEventRecord(b->ev[1], b->stream));

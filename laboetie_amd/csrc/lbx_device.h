@@ -220,21 +220,6 @@ struct Plane {
         else
             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, idx * 4u, 0, CP);
     }
-    // elements 2*pidx and 2*pidx+1 in one access (b128 for double, b64 for float)
-    __device__ __forceinline__ Vec2<E> ld2(uint32_t pidx) const {
-        if constexpr (sizeof(E) == 8)
-            return __builtin_bit_cast(Vec2<E>, __builtin_amdgcn_raw_buffer_load_b128(r, pidx * 16u, 0, 0));
-        else
-            return __builtin_bit_cast(Vec2<E>, __builtin_amdgcn_raw_buffer_load_b64(r, pidx * 8u, 0, 0));
-    }
-    __device__ __forceinline__ void st2(uint32_t pidx, Vec2<E> v) const {
-        if constexpr (sizeof(E) == 8)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v),
-                                                   r, pidx * 16u, 0, 0);
-        else
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v),
-                                                  r, pidx * 8u, 0, 0);
-    }
 };
 
 // A set of planes of E addressed by a 32-bit element index.  Narrow: a
@@ -249,8 +234,6 @@ struct View<false, E> {
     __device__ __forceinline__ E ld(uint32_t idx) const { return p.ld(idx); }
     __device__ __forceinline__ void st(uint32_t idx, E v) const { p.st(idx, v); }
     __device__ __forceinline__ void stnt(uint32_t idx, E v) const { p.template st<kNonTemporal>(idx, v); }
-    __device__ __forceinline__ Vec2<E> ld2(uint32_t pidx) const { return p.ld2(pidx); }
-    __device__ __forceinline__ void st2(uint32_t pidx, Vec2<E> v) const { p.st2(pidx, v); }
 };
 template <typename E>
 struct View<true, E> {
@@ -259,39 +242,7 @@ struct View<true, E> {
     __device__ __forceinline__ E ld(uint32_t idx) const { return b[(uint64_t)idx]; }
     __device__ __forceinline__ void st(uint32_t idx, E v) const { b[(uint64_t)idx] = v; }
     __device__ __forceinline__ void stnt(uint32_t idx, E v) const { __builtin_nontemporal_store(v, b + (uint64_t)idx); }
-    __device__ __forceinline__ Vec2<E> ld2(uint32_t pidx) const { return ((const Vec2<E>*)b)[(uint64_t)pidx]; }
-    __device__ __forceinline__ void st2(uint32_t pidx, Vec2<E> v) const { ((Vec2<E>*)b)[(uint64_t)pidx] = v; }
 };
-
-// K per-node values of Np nodes (a moment field, the scattering
-// probabilities) laid out so that one 16-byte (double) or 8-byte (float)
-// access reads two of them: values 2p and 2p+1 (p < K/2) side by side in pair
-// plane p, an odd last value alone in a plane after the pairs.  A node's K
-// values then take ceil(K/2) loads instead of K.
-__host__ __device__ constexpr uint64_t comp_index(int K, int k, uint64_t i, uint64_t Np) {
-    return k < (K & ~1) ? ((uint64_t)(k >> 1) * Np + i) * 2 + (uint64_t)(k & 1) : (uint64_t)(K & ~1) * Np + i;
-}
-
-template <int K, typename V, typename E>
-__device__ __forceinline__ void load_comps(const V& v, uint32_t Np, uint32_t i, E (&out)[K]) {
-    static_for<0, K / 2>([&](auto P) {
-        const Vec2<E> x = v.ld2((uint32_t)P * Np + i);
-        out[2 * P] = x[0];
-        out[2 * P + 1] = x[1];
-    });
-    if constexpr (K & 1) out[K - 1] = v.ld((uint32_t)(K - 1) * Np + i);
-}
-
-template <int K, typename V, typename E>
-__device__ __forceinline__ void store_comps(const V& v, uint32_t Np, uint32_t i, const E (&in)[K]) {
-    static_for<0, K / 2>([&](auto P) {
-        Vec2<E> x;
-        x[0] = in[2 * P];
-        x[1] = in[2 * P + 1];
-        v.st2((uint32_t)P * Np + i, x);
-    });
-    if constexpr (K & 1) v.st((uint32_t)(K - 1) * Np + i, in[K - 1]);
-}
 
 // Periodic neighbour offsets of a node: X[1+d] is the x index of x+d, and Y,
 // Z the row / plane offsets of y+d, z+d (module_system.f90:99-112: only a
@@ -388,38 +339,6 @@ __device__ __forceinline__ double wave_max(double v) {
     v = fmax(v, dpp_row<0x141>(v));
     v = fmax(v, dpp_row<0x140>(v));
     return fmax(fmax(read_lane(v, 0), read_lane(v, 16)), fmax(read_lane(v, 32), read_lane(v, 48)));
-}
-
-// Lane k of the wave receives lane k+1's value (S = +1, DPP wave_shl:1) or
-// lane k-1's (S = -1, wave_shr:1); lane 63 (S = +1) and lane 0 (S = -1), and
-// a lane whose source lane is inactive, receive 0.  Register moves only.
-template <int S>
-__device__ __forceinline__ double lane_shift(double v) {
-    static_assert(S == 1 || S == -1, "one lane up or down");
-    constexpr int ctrl = S > 0 ? 0x130 : 0x138;
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, ctrl, 0xf, 0xf, false);
-    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), ctrl, 0xf, 0xf, false);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// Deterministic block sum of 3 values; the result is valid in thread 0.
-template <int BLOCK>
-__device__ __forceinline__ void block_sum3(double v[3], double* lds /* [BLOCK/64*3] */) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int a = 0; a < 3; ++a) {
-        double s = wave_sum(v[a]);
-        if (lane == 0) lds[w * 3 + a] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int a = 0; a < 3; ++a) {
-            double s = lds[a];
-            for (int k = 1; k < BLOCK / 64; ++k) s = s + lds[k * 3 + a];
-            v[a] = s;
-        }
-    }
-    __syncthreads();
 }
 
 }  // namespace lbx

@@ -1,8 +1,8 @@
 // Device code of liblbx shared by the single-lattice path (lbx.hip) and the
 // multi-instance batch path (lbx_batch.hip): the control block, neighbour
-// lookup, the LB and moment-propagation work of one block of nodes
-// (lb_step_tile, mp_prep_tile, mp_step_tile, parameterised by the block size)
-// and the small kernels both paths launch.  A lattice's nodes are a range of
+// lookup, the LB work of one block of nodes (lb_step_tile, parameterised by
+// the block size), the VACF reduction and the small kernels both paths launch
+// (moment propagation itself: lbx_mp.h).  A lattice's nodes are a range of
 // the packed fluid-node list; both paths run the same per-node arithmetic, so
 // an instance gives the same bits alone or in a batch.
 #pragma once
@@ -39,7 +39,7 @@ struct Ctrl {
     int64_t exit_step;           // LB: that converged step
     int64_t negpop;              // LB: first step with a negative population (-1: none)
     int32_t mp_stop;             // MP: VACF convergence reached
-    int32_t pad;
+    int32_t mp_divide;           // MP: densities or flows outside quotient()'s range (set by mp prep)
     int64_t mp_conv_step;
     int32_t floor_hit;           // LB (FP32-shift): the stop at exit_step was the l2err floor test
     int32_t pad2;
@@ -234,9 +234,6 @@ __device__ __forceinline__ E pull(const View<Wide, E>& fin, uint32_t Np, uint32_
 // density (:254) and flux (:293-300), the l2err contribution (:339-344), then
 // the collision that opens step t+1 (module_collision.f90:87-108).
 // E = float: the FP32-shift form; the l2err is still a max of FP64 values.
-#ifndef LBX_MP_WAVES
-#define LBX_MP_WAVES 1
-#endif
 #ifndef LBX_LB_WAVES
 #define LBX_LB_WAVES 1
 #endif
@@ -642,23 +639,8 @@ __global__ __launch_bounds__(kBlock) void k_init_rest(double* __restrict__ f, fl
 
 // ---------------------------------------------------------------- MP kernels
 
-// packed nodes on either side of an MP block whose P the block stages in LDS
-#ifndef LBX_MP_HALO
-#define LBX_MP_HALO 128
-#endif
-constexpr int kMpHalo = LBX_MP_HALO;
-
-// a block's LDS array with View's element / pair access (load_comps, store_comps)
-struct LdsView {
-    double* b;
-    __device__ __forceinline__ double ld(uint32_t idx) const { return b[idx]; }
-    __device__ __forceinline__ void st(uint32_t idx, double v) const { b[idx] = v; }
-    __device__ __forceinline__ Vec2<double> ld2(uint32_t pidx) const { return ((const Vec2<double>*)b)[pidx]; }
-    __device__ __forceinline__ void st2(uint32_t pidx, Vec2<double> v) const { ((Vec2<double>*)b)[pidx] = v; }
-};
-//
 // Several tracers that share the flow and Db (so the scattering
-// probabilities win, rem and u*) but differ in ka, kd can be propagated in one
+// probabilities, rem and u*) but differ in ka, kd can be propagated in one
 // pass: the shared coefficients are read once per node for all of them.  The
 // arithmetic of each tracer is exactly that of a single-tracer run.
 
@@ -670,10 +652,20 @@ constexpr int kMaxTracers = 4;
 // optionally, the convergence test of module_moment_propagation.f90:284-288
 // (all NV components below both limits).  Called by all BLOCK threads of one
 // block.  mode 0: VACF(0) of mp init; mode 1: VACF(it) of a step.
+// Component a is summed over the waves and kept by thread a, whose loads of the
+// running sums go out with the partials: one thread doing all components paid
+// a memory round trip for each (a 3-tracer step of 2 000 nodes: 11.9 us).
 template <int NV, int BLOCK>
 __device__ __forceinline__ void mp_reduce_block(const double* part, uint32_t nparts, double* vtrace, Ctrl* ctrl,
                                                 int32_t mode, int64_t it, int32_t check_conv, double lim1,
-                                                double lim2, double* lds /* [4*NV] */) {
+                                                double lim2, double* lds /* [BLOCK/64*NV] */) {
+    static_assert(NV <= 64, "one wave keeps the components");
+    const int me = threadIdx.x;
+    double run_s = 0.0, run_c = 0.0;
+    if (mode != 0 && me < NV) {
+        run_s = ctrl->deff_s[me];
+        run_c = ctrl->deff_c[me];
+    }
     double s[NV];
 #pragma unroll
     for (int a = 0; a < NV; ++a) s[a] = 0.0;
@@ -684,44 +676,32 @@ __device__ __forceinline__ void mp_reduce_block(const double* part, uint32_t npa
             s[a] = (k == threadIdx.x) ? x : s[a] + x;
         }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    wave_sums<NV>(s);
+    if (lane == 0)
 #pragma unroll
-    for (int a = 0; a < NV; ++a) {
-        const double t = wave_sum(s[a]);
-        if (lane == 0) lds[w * NV + a] = t;
-    }
+        for (int a = 0; a < NV; ++a) lds[w * NV + a] = s[a];
     __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int a = 0; a < NV; ++a) {
-            double t = lds[a];
-            for (int k = 1; k < BLOCK / 64; ++k) t = t + lds[k * NV + a];
-            s[a] = t;
-        }
-        if (mode == 0) {
-#pragma unroll
-            for (int a = 0; a < NV; ++a) {
-                ctrl->vacf0[a] = s[a];
-                ctrl->deff_s[a] = 0.5 * s[a];
-                ctrl->deff_c[a] = 0.0;
-            }
-        } else {
-#pragma unroll
-            for (int a = 0; a < NV; ++a) {
-                vtrace[a] = s[a];
+    if (w == 0) {
+        bool below = true;
+        if (me < NV) {
+            double t = lds[me];
+            for (int k = 1; k < BLOCK / 64; ++k) t = t + lds[k * NV + me];
+            if (mode == 0) {
+                ctrl->vacf0[me] = t;
+                ctrl->deff_s[me] = 0.5 * t;
+                ctrl->deff_c[me] = 0.0;
+            } else {
+                vtrace[me] = t;
                 // Neumaier update of D = VACF(0)/2 + sum VACF(t)
-                const double d = ctrl->deff_s[a], x = s[a], u = d + x;
-                ctrl->deff_c[a] += (fabs(d) >= fabs(x)) ? (d - u) + x : (x - u) + d;
-                ctrl->deff_s[a] = u;
+                const double u = run_s + t;
+                ctrl->deff_c[me] = run_c + ((fabs(run_s) >= fabs(t)) ? (run_s - u) + t : (t - u) + run_s);
+                ctrl->deff_s[me] = u;
             }
-            if (check_conv && it > 2) {
-                bool conv = true;
-#pragma unroll
-                for (int a = 0; a < NV; ++a) conv = conv && fabs(s[a]) < lim1 && fabs(s[a]) < lim2;
-                if (conv) {
-                    ctrl->mp_conv_step = it;
-                    ctrl->mp_stop = 1;
-                }
-            }
+            below = fabs(t) < lim1 && fabs(t) < lim2;
+        }
+        if (mode != 0 && check_conv && it > 2 && __all(below) && me == 0) {
+            ctrl->mp_conv_step = it;
+            ctrl->mp_stop = 1;
         }
     }
     __syncthreads();
@@ -742,8 +722,8 @@ struct TracerParams {
     int32_t ads[kMaxTracers];  // adsorption on (K = ka/kd > eps, :46-56)
 };
 
-// W is the type the scattering probabilities win and u* are stored in:
-// double, or float in the FP32-shift form.  There each probability is rounded
+// W is the type the scattering probabilities and u* are rounded to (and, where
+// they are kept, stored in): double, or float in the FP32-shift form.  There each probability is rounded
 // to FP32 once, and every quantity built from it (the rest probability
 // rem = 1 - sum s, which stays FP64, u*, P(r,1), VACF(0)) uses the rounded
 // value, so the propagator still conserves sum_r P exactly up to FP64 rounding.
@@ -765,460 +745,25 @@ __device__ __forceinline__ double scatter_prob(double rho, double vx, double vy,
     return as_coef<W>(nt / rho - a0(L) + lambda * a0(L) * 0.5);
 }
 
-// Where the MP step takes the incoming probabilities s(r+c_l, inv l) from
-// (the C-ABI's LBX_MP_STORED / _RECOMPUTED / _MIXED): the 18 stored per node,
-// all 18 recomputed from the neighbours' (rho, v), or the 10 with c_z != 0
-// stored (those neighbours are a plane away, outside the LDS window, where
-// reading (rho, v) costs more than a stored value) and the 8 others
-// recomputed from the window.
-constexpr int kCoefStored = 0, kCoefRecomputed = 1, kCoefMixed = 2;
-constexpr int kZDirs = 10;  // directions with c_z != 0: 5, 6, 11..18
-// index of direction L (c_z != 0) among them, and of its pair (L, L+1 for odd L)
-constexpr int zdir(int L) { return L <= 6 ? L - 5 : L - 9; }
-
-template <typename W>
-struct MpPrepArgs {
-    const double* __restrict__ rho;
-    const double* __restrict__ j;
-    const uint32_t* __restrict__ nodes;
-    const uint32_t* __restrict__ map;
-    W* __restrict__ win = nullptr;       // incoming probabilities (NULL: not kept, the step recomputes them)
-    int32_t win_z = 0;                   // win holds only the kZDirs directions with c_z != 0
-    double* __restrict__ rv = nullptr;   // (rho, v) of each node, 4 doubles (NULL: not kept)
-    double* __restrict__ rem;
-    W* __restrict__ ustar;
-    double* __restrict__ P0;   // [T][3][Np]
-    double* partials;
-    Ctrl* ctrl;
-    FastDiv dlx, dly;
-    uint32_t lz, Nf;
-    uint64_t Np;
-    double fx, fy, fz;   // lb.in f_ext (drop_tracers.f90:92)
-    double lambda, eps;
-    uint32_t tile0;        // first tile of the lattice's node range
-    TracerParams tp;
-};
-
-// update_tracer_population (drop_tracers.f90:97-100) fused with
-// moment_propagation::init (module_moment_propagation.f90:105-137) and the
-// static part of propagate (:218-249): per fluid node, the scattering
-// probabilities s(r,l) = n_l/rho - w_l + lambda w_l / 2 towards fluid
-// neighbours, the rest probability rem, u* = sum s c, the incoming
-// probabilities win(r,l) = s(r+c_l, inv l), and per tracer P(r,1) and the
-// VACF(0) contribution.
-//
-// mp_prep_tile: one block's share; the block's nodes are tile*BLOCK + lane
-// (valid below a.Nf) and its VACF(0) partial goes to a.partials[3T*tile ...].
-template <int BLOCK, int T, typename W>
-__device__ __forceinline__ void mp_prep_tile(const MpPrepArgs<W>& a, uint32_t tile) {
-    __shared__ double lds[BLOCK / 64 * 3 * T];
-    const uint32_t i = tile * BLOCK + threadIdx.x;
-    double vp[3 * T];
-#pragma unroll
-    for (int k = 0; k < 3 * T; ++k) vp[k] = 0.0;
-    if (i < a.Nf) {
-        const uint32_t e = a.nodes[i];
-        Neighbours nb;
-        nb.load(a.map, e & kIndexMask, a.dlx, a.dly, a.lz);
-        const double rr = a.rho[i];
-        const double vx = a.j[i] + a.fx, vy = a.j[a.Np + i] + a.fy, vz = a.j[2 * a.Np + i] + a.fz;
-        if (a.rv) {
-            a.rv[4 * (uint64_t)i] = rr;
-            a.rv[4 * (uint64_t)i + 1] = vx;
-            a.rv[4 * (uint64_t)i + 2] = vy;
-            a.rv[4 * (uint64_t)i + 3] = vz;
-        }
-        double us[3] = {0.0, 0.0, 0.0};
-        double p1[3 * T];
-#pragma unroll
-        for (int k = 0; k < 3 * T; ++k) p1[k] = 0.0;
-        double remv = 1.0;
-        static_for<1, kQ>([&](auto I) {
-            constexpr int L = I;
-            constexpr int Li = kInv[L];
-            constexpr int cx = kCX[L], cy = kCY[L], cz = kCZ[L];
-            const uint32_t q = nb.q[L];
-            if (q != kSolidSlot) {
-                const double s = scatter_prob<L, W>(rr, vx, vy, vz, a.lambda);
-                remv = remv - s;
-                if constexpr (cx != 0) us[0] = us[0] + sgn<cx>(s);
-                if constexpr (cy != 0) us[1] = us[1] + sgn<cy>(s);
-                if constexpr (cz != 0) us[2] = us[2] + sgn<cz>(s);
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    if constexpr (cx != 0) vp[3 * t + 0] = vp[3 * t + 0] + a.tp.bw[t] * s;
-                    if constexpr (cy != 0) vp[3 * t + 1] = vp[3 * t + 1] + a.tp.bw[t] * s;
-                    if constexpr (cz != 0) vp[3 * t + 2] = vp[3 * t + 2] + a.tp.bw[t] * s;
-                }
-                const double rn = a.rho[q];
-                const double wx = a.j[q] + a.fx, wy = a.j[a.Np + q] + a.fy, wz = a.j[2 * a.Np + q] + a.fz;
-                const double sp = scatter_prob<Li, W>(rn, wx, wy, wz, a.lambda);
-                if (a.win) {
-                    if (!a.win_z)
-                        a.win[comp_index(18, L - 1, i, a.Np)] = (W)sp;
-                    else if constexpr (cz != 0)
-                        a.win[comp_index(kZDirs, zdir(L), i, a.Np)] = (W)sp;
-                }
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-                    if constexpr (cx != 0) p1[3 * t + 0] = p1[3 * t + 0] + sgn<-cx>(sp) * a.tp.bw[t];
-                    if constexpr (cy != 0) p1[3 * t + 1] = p1[3 * t + 1] + sgn<-cy>(sp) * a.tp.bw[t];
-                    if constexpr (cz != 0) p1[3 * t + 2] = p1[3 * t + 2] + sgn<-cz>(sp) * a.tp.bw[t];
-                }
-            } else if (a.win) {
-                if (!a.win_z)
-                    a.win[comp_index(18, L - 1, i, a.Np)] = W(0);
-                else if constexpr (cz != 0)
-                    a.win[comp_index(kZDirs, zdir(L), i, a.Np)] = W(0);
-            }
-        });
-        a.rem[i] = remv;
-        bool low = false;
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const double rt = (a.tp.ads[t] && (e & kNodeInterfacial)) ? remv - a.tp.ka[t] : remv;
-            low = low || rt < a.eps;
-        }
-        if (low) a.ctrl->restpart = 1;
-        for (int c = 0; c < 3; ++c) a.ustar[comp_index(3, c, i, a.Np)] = (W)us[c];
-#pragma unroll
-        for (int k = 0; k < 3 * T; ++k) a.P0[comp_index(3 * T, k, i, a.Np)] = p1[k];
-    }
-    block_partial<3 * T, BLOCK>(vp, a.partials + 3 * T * (uint64_t)tile, lds);
+// x / y rounded correctly from r = 1/y rounded correctly (y shared by many
+// quotients, so its division is done once): after one correction q is within
+// an ulp of x/y, and then q + r (x - y q), its remainder exact in one fused
+// multiply-add, rounds to x/y rounded correctly (Markstein, "Computation of
+// elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34, 1990, theorem on the last step of a division).  For y in [2^-400,
+// 2^400] and x = 0 or in [2^-900, 2^900] nothing over- or underflows on the way.
+__device__ __forceinline__ double quotient(double x, double y, double r) {
+    double q = x * r;
+    q = __builtin_fma(__builtin_fma(-y, q, x), r, q);
+    return __builtin_fma(__builtin_fma(-y, q, x), r, q);
 }
 
-template <int T, typename W>
-__global__ __launch_bounds__(kBlock) void k_mp_prep(MpPrepArgs<W> a) {
-    mp_prep_tile<kBlock, T, W>(a, a.tile0 + xcd_tile());
-}
-
-template <typename W>
-struct MpStepArgs {
-    const W* __restrict__ win;
-    const double* __restrict__ rem;
-    const W* __restrict__ ustar;
-    const uint32_t* __restrict__ nodes;
-    const uint32_t* __restrict__ map;
-    const double* __restrict__ Pn;   // [T][3][Np]
-    double* __restrict__ Px;
-    const double* __restrict__ Pan;
-    double* __restrict__ Pax;
-    double* partials;                // this step's per-block VACF partials
-    const double* prev_partials;     // the previous step's, reduced by block 0 (NULL: none)
-    int32_t check_conv = 0;          // block 0 also applies the convergence test to VACF(it-1)
-    double lim1 = 0.0, lim2 = 0.0;   // its limits (module_moment_propagation.f90:284)
-    // RV steps: (rho, v) of each node, 4 doubles, and lambda, from which the
-    // incoming probabilities are recomputed instead of read from win
-    const double* rv = nullptr;
-    double lambda = 0.0;
-    double* prev_vtrace;             // where VACF(it-1) goes
-    int64_t it;
-    Ctrl* ctrl;
-    FastDiv dlx, dly;
-    uint32_t lz, Nf;
-    uint64_t Np;
-    int32_t any_ads;                 // some tracer of the batch adsorbs (Pan, Pax allocated)
-    TracerParams tp;
-    const uint32_t* tile_order = nullptr;  // tile of each logical tile (NULL: the same)
-};
-
-// One moment-propagation step of T tracers, module_moment_propagation.f90:207-253:
-// P(r,t+1) = sum_l P(r+c_l,t) s(r+c_l, inv l) + rem(r) P(r,t) [+ kd Pa],
-// Pa(r,t+1) = (1-kd) Pa(r,t) + ka P(r,t) at adsorbing interfacial nodes,
-// VACF(t) = sum_r P(r,t) . u*(r).
-//
-// mp_step_tile: one block's share; nodes tile*BLOCK + lane (valid below a.Nf),
-// VACF partial to a.partials[K*tile ...]; first_block also reduces the
-// previous step's nparts partials (a.prev_partials) into VACF(it-1).
-//
-// XR: directions 11..14 may reuse the z-neighbours of the lanes beside (below).
-// CF (kCoef*): recomputed probabilities come from the neighbours' (rho, v)
-// (scatter_prob, the set-up's own arithmetic: the same bits): 32 bytes per
-// node kept and staged in the LDS window beside P; stored ones from win (18 or,
-// mixed, kZDirs per node, read in pairs).
-template <int BLOCK, bool Wide, int T, typename W, int CF = kCoefStored, bool XR = true>
-__device__ __forceinline__ void mp_step_tile(const MpStepArgs<W>& a, uint32_t tile, bool first_block,
-                                             uint32_t nparts) {
-    constexpr bool RV = CF != kCoefStored;  // (rho, v) staged in the window
-    constexpr bool RVZ = CF == kCoefRecomputed;  // the directions with c_z != 0 recomputed too
-    constexpr int K = 3 * T;  // moment components of the batch
-    // The edge-lane records and the early gathers of the neighbours along 5
-    // and 6 (below) serve the forms that store the z-directions'
-    // probabilities.  With those recomputed (RVZ) the added loads and (rho, v)
-    // work before the window barrier cost more than the records save
-    // (measured), so RVZ leaves both out.
-    constexpr bool XCH = !RVZ && XR;
-    // the mixed form with three tracers: 4 fewer halo nodes a side keep the
-    // records within a third of the CU's LDS (three blocks per CU)
-    constexpr int HALO = (XCH && RV && T == 3) ? kMpHalo - 4 : kMpHalo;
-    constexpr int WIN = BLOCK + 2 * HALO;
-    constexpr int NW = BLOCK / 64;  // waves per block
-    // Edge-lane records, [wave boundary][side][plane][RW]: P of a wave's first
-    // (side 0) or last (side 1) lane's neighbour along 5 (plane 0) or 6
-    // (plane 1), for the lane beside it in the adjacent wave.  The array
-    // holds the VACF partial's wave sums after the step's last record read.
-    constexpr int RW = K;  // doubles per record
-    constexpr int XN = (XCH && NW > 1) ? (NW - 1) * 4 * RW : 0;
-    constexpr int LN = NW * K > XN ? NW * K : XN;
-    __shared__ double lds[LN];
-    __shared__ double pwin[K * WIN];  // P(now) of packed nodes [w0, w0 + WIN), comp_index layout
-    __shared__ double rvwin[RV ? 4 * WIN : 2];  // RV: (rho, v) of the same nodes
-    const uint32_t i = tile * BLOCK + threadIdx.x;
-    const bool valid = i < a.Nf;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    // Each wave's work is a chain of dependent memory round trips (stop flag,
-    // node word, neighbour indices, neighbour values), so independent
-    // requests are issued together: the node word with the stop flag, the
-    // neighbour indices and the node's coefficients with the LDS window.
-    const uint32_t e = valid ? ld(a.nodes, i) : 0u;
-    if (block_flag(vload(&a.ctrl->mp_stop) != 0)) return;
-    // VACF(it-1) from the previous step's partials and, with check_conv, the
-    // convergence test: a stop set here ends the run at step it-1 (this
-    // launch's other blocks may have started step it already; they write only
-    // the other buffer of P, and every later launch returns at once)
-    if (a.prev_partials && first_block) {
-        mp_reduce_block<K, BLOCK>(a.prev_partials, nparts, a.prev_vtrace, a.ctrl, 1, a.it - 1, a.check_conv, a.lim1,
-                                  a.lim2, lds);
-        if constexpr (XCH && NW > 1) __syncthreads();  // its last read of lds before the records are written there
-    }
-    const uint32_t Np = (uint32_t)a.Np;
-    const View<Wide> Pn(a.Pn, K * a.Np);
-    const View<Wide, W> win(a.win, (CF == kCoefMixed ? kZDirs : 18) * a.Np), us(a.ustar, 3 * a.Np);
-    const View<Wide> rem(a.rem, a.Np);
-    Neighbours nb;
-    W uw[3] = {W(0), W(0), W(0)};
-    double rm = 0.0;
-    if (valid) {
-        nb.load(a.map, e & kIndexMask, a.dlx, a.dly, a.lz);
-        load_comps<3>(us, Np, i, uw);
-        rm = rem.ld(i);
-    }
-    // The block's nodes and HALO on either side: neighbours along x, and
-    // along y where a row holds fewer fluid nodes than that, are read from LDS
-    const int64_t w0 = (int64_t)tile * BLOCK - HALO;
-    const LdsView pw{pwin};
-    const View<Wide> rvv(a.rv, 4 * a.Np);
-    // The node's neighbours along 5 (0,0,1) and 6 (0,0,-1), whose values the
-    // directions 11..14 reuse (below): gathered here, with the window, where
-    // they lie outside it or the lane is a wave's first or last.
-    // A lattice one node wide along x (the 2-D instances) has no x-neighbour
-    // in another lane: it skips all of this (the same for every lane of a
-    // block, whose nodes belong to one lattice), and XR = false compiles it
-    // out (a batch of such lattices only: the registers it holds cost them
-    // occupancy).
-    const bool xreuse = XR && a.dlx.d > 1u;
-    double zc[2][K];         // their P (0 if solid)
-    Vec2<double> zr[2][2];   // RVZ: their (rho, v), kept in the direction loop
-    bool zearly[2] = {false, false};
-    const bool edge_lane = XCH && NW > 1 && xreuse && (lane == 0u || lane == 63u);
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) zc[s][k] = 0.0;
-        zr[s][0] = Vec2<double>{0.0, 0.0};
-        zr[s][1] = Vec2<double>{0.0, 0.0};
-        if (valid) {
-            const uint32_t q = nb.q[5 + s];
-            zearly[s] = XCH && xreuse && q != kSolidSlot && ((uint32_t)((int64_t)q - w0) >= (uint32_t)WIN || edge_lane);
-            if (zearly[s]) load_comps<K>(Pn, Np, q, zc[s]);
-        }
-    }
-    {
-        // every slot's loads go out before the first LDS write waits on them
-        constexpr int NIT = (WIN + BLOCK - 1) / BLOCK;
-        double fv[NIT][K];
-        Vec2<double> fr[NIT][2];
-        bool in[NIT];
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int n = (int)threadIdx.x + it * BLOCK;
-            const int64_t g = w0 + n;
-            in[it] = n < WIN && g >= 0 && g < (int64_t)Np;
-            if (in[it]) {
-                load_comps<K>(Pn, Np, (uint32_t)g, fv[it]);
-                if constexpr (RV) {
-                    fr[it][0] = rvv.ld2(2 * (uint32_t)g);
-                    fr[it][1] = rvv.ld2(2 * (uint32_t)g + 1);
-                }
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < NIT; ++it) {
-            const int n = (int)threadIdx.x + it * BLOCK;
-            if (in[it]) {
-                store_comps<K>(pw, WIN, (uint32_t)n, fv[it]);
-                if constexpr (RV) {
-                    ((Vec2<double>*)rvwin)[2 * n] = fr[it][0];
-                    ((Vec2<double>*)rvwin)[2 * n + 1] = fr[it][1];
-                }
-            }
-        }
-    }
-    // records of the lanes at the block's inner wave boundaries: lane 0 of
-    // wave w serves lane 63 of wave w-1 (directions 11, 13), lane 63 of wave w
-    // serves lane 0 of wave w+1 (12, 14)
-    if constexpr (XCH && NW > 1) {
-        if (valid && xreuse && ((lane == 0u && wave > 0u) || (lane == 63u && wave + 1u < (uint32_t)NW))) {
-            const uint32_t side = lane == 0u ? 0u : 1u, bnd = lane == 0u ? wave - 1u : wave;
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                double* r = lds + ((bnd * 2u + side) * 2u + (uint32_t)s) * RW;
-#pragma unroll
-                for (int k = 0; k < K; ++k) r[k] = zc[s][k];
-            }
-        }
-    }
-    __syncthreads();
-    double vp[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) vp[k] = 0.0;
-    if (valid) {
-        const View<Wide> Px(a.Px, K * a.Np);
-        double p[K], acc[K];
-        load_comps<K>(pw, WIN, (uint32_t)(HALO + threadIdx.x), p);
-#pragma unroll
-        for (int k = 0; k < K; ++k) acc[k] = 0.0;
-        // The node's x-neighbour in its row is packed node i+1 (i-1) whenever
-        // that neighbour is fluid and not across the periodic wrap: held by the
-        // next (previous) lane of the wave, or by the first (last) lane of the
-        // next (previous) wave of the block.  Its neighbour one plane up (down)
-        // is then the node's neighbour along (+-1, 0, +-1): directions 11..14
-        // take P (and the probability from (rho, v)) of that lane's neighbour
-        // along 5 or 6, moved across the wave or from its edge-lane record,
-        // instead of gathering them again; the sum keeps its order and bits.
-        const bool adj_r = nb.q[1] == i + 1u;
-        const bool adj_l = i > 0u && nb.q[2] == i - 1u;
-        Vec2<W> wp;  // the probabilities of directions L, L+1 (L odd) from one paired load
-        static_for<1, kQ>([&](auto I) {
-            constexpr int L = I;
-            constexpr bool stored = CF == kCoefStored || (CF == kCoefMixed && kCZ[L] != 0);
-            // 11, 12 from 5 of lane +-1; 13, 14 from 6 of lane +-1; 5, 6 kept
-            constexpr int zsrc = (L >= 11 && L <= 14) ? (kCZ[L] > 0 ? 0 : 1) : -1;
-            constexpr int zkeep = L == 5 ? 0 : (L == 6 ? 1 : -1);
-            if constexpr (CF == kCoefStored && (L & 1)) wp = win.ld2((uint32_t)((L - 1) / 2) * Np + i);
-            if constexpr (CF == kCoefMixed && stored && (L & 1)) wp = win.ld2((uint32_t)(zdir(L) / 2) * Np + i);
-            double sh[K];          // moved across the wave while every valid lane is active
-            Vec2<double> sr[2];
-            if constexpr (zsrc >= 0) {
-                if (xreuse) {
-#pragma unroll
-                    for (int k = 0; k < K; ++k) sh[k] = lane_shift<kCX[L]>(zc[zsrc][k]);
-                    if constexpr (!stored)
-                        for (int h = 0; h < 2; ++h)
-                            sr[h] = Vec2<double>{lane_shift<kCX[L]>(zr[zsrc][h][0]),
-                                                 lane_shift<kCX[L]>(zr[zsrc][h][1])};
-                }
-            }
-            const uint32_t q = nb.q[L];
-            if (q != kSolidSlot) {
-                double pq[K];
-                double w = 0.0;
-                Vec2<double> r0, r1;  // (rho, vx), (vy, vz) of the neighbour (RV directions)
-                int how = 0;          // 0: gather, 1: from the lane beside, 2: from an edge-lane record
-                if constexpr (zsrc >= 0) {
-                    constexpr bool right = kCX[L] > 0;
-                    if (xreuse && (right ? adj_r : adj_l)) {  // else gathered (sh is not set)
-                        if (!(right ? lane == 63u : lane == 0u))
-                            how = 1;
-                        else if (XCH && (right ? wave + 1u < (uint32_t)NW : wave > 0u))
-                            how = 2;
-                    }
-                    if (how == 1) {
-#pragma unroll
-                        for (int k = 0; k < K; ++k) pq[k] = sh[k];
-                        if constexpr (!stored) {
-                            r0 = sr[0];
-                            r1 = sr[1];
-                        }
-                    } else if (how == 2) {  // XCH: these directions' probabilities are stored
-                        const double* r = lds + (((right ? wave : wave - 1u) * 2u + (right ? 0u : 1u)) * 2u +
-                                                 (uint32_t)zsrc) * RW;
-#pragma unroll
-                        for (int k = 0; k < K; ++k) pq[k] = r[k];
-                    }
-                }
-                if constexpr (zkeep >= 0) {
-                    if (zearly[zkeep]) {
-#pragma unroll
-                        for (int k = 0; k < K; ++k) pq[k] = zc[zkeep][k];
-                        if constexpr (!stored) {
-                            r0 = zr[zkeep][0];
-                            r1 = zr[zkeep][1];
-                        }
-                        how = 1;
-                    }
-                }
-                if (how == 0) {
-                    const uint32_t d = (uint32_t)((int64_t)q - w0);
-                    if (d < (uint32_t)WIN) {
-                        load_comps<K>(pw, WIN, d, pq);
-                        if constexpr (!stored) {
-                            r0 = ((const Vec2<double>*)rvwin)[2 * d];
-                            r1 = ((const Vec2<double>*)rvwin)[2 * d + 1];
-                        }
-                    } else {
-                        load_comps<K>(Pn, Np, q, pq);
-                        if constexpr (!stored) {
-                            r0 = rvv.ld2(2 * q);
-                            r1 = rvv.ld2(2 * q + 1);
-                        }
-                    }
-                }
-                if constexpr (zkeep >= 0) {
-#pragma unroll
-                    for (int k = 0; k < K; ++k) zc[zkeep][k] = pq[k];
-                    if constexpr (!stored) {
-                        zr[zkeep][0] = r0;
-                        zr[zkeep][1] = r1;
-                    }
-                }
-                if constexpr (!stored)
-                    w = scatter_prob<kInv[L], W>(r0[0], r0[1], r1[0], r1[1], a.lambda);
-                else
-                    w = (double)wp[(L - 1) & 1];
-#pragma unroll
-                for (int k = 0; k < K; ++k) acc[k] = acc[k] + pq[k] * w;
-            }
-        });
-#pragma unroll
-        for (int t = 0; t < T; ++t)
-            for (int c = 0; c < 3; ++c) vp[3 * t + c] = p[3 * t + c] * (double)uw[c];
-        double px[K];
-        if (!(a.any_ads && (e & kNodeInterfacial))) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) px[k] = acc[k] + rm * p[k];
-            store_comps<K>(Px, Np, i, px);
-        } else {
-            const View<Wide> Pan(a.Pan, K * a.Np), Pax(a.Pax, K * a.Np);
-            double pa[K], pax[K];
-            load_comps<K>(Pan, Np, i, pa);
-#pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const double rt = rm - a.tp.ka[t];
-                for (int c = 0; c < 3; ++c) {
-                    const int k = 3 * t + c;
-                    if (a.tp.ads[t]) {
-                        px[k] = (acc[k] + rt * p[k]) + pa[k] * a.tp.kd[t];
-                        pax[k] = pa[k] * a.tp.one_minus_kd[t] + p[k] * a.tp.ka[t];
-                    } else {  // a tracer without adsorption keeps Pa = 0
-                        px[k] = acc[k] + rm * p[k];
-                        pax[k] = pa[k];
-                    }
-                }
-            }
-            store_comps<K>(Px, Np, i, px);
-            store_comps<K>(Pax, Np, i, pax);
-        }
-    }
-    if constexpr (XCH && NW > 1)
-        if (xreuse) __syncthreads();  // every wave's last edge-lane record read is over
-    block_partial<K, BLOCK>(vp, a.partials + (uint64_t)K * tile, lds);
-}
-
-template <bool Wide, int T, typename W, int CF>
-__global__ __launch_bounds__(kBlock, LBX_MP_WAVES) void k_mp_step(MpStepArgs<W> a) {
-    mp_step_tile<kBlock, Wide, T, W, CF>(a, a.tile_order ? a.tile_order[xcd_tile()] : xcd_tile(), blockIdx.x == 0,
-                                         gridDim.x);
+// scatter_prob with 1/rho given: the same bits
+template <int L, typename W>
+__device__ __forceinline__ double scatter_prob(double rho, double rinv, double vx, double vy, double vz, double lambda) {
+    constexpr int cx = kCX[L], cy = kCY[L], cz = kCZ[L];
+    const double nt = a0(L) * rho + a1(L) * dot3<cx, cy, cz>(vx, vy, vz);
+    return as_coef<W>(quotient(nt, rho, rinv) - a0(L) + lambda * a0(L) * 0.5);
 }
 
 // Plain streaming copy (16 B per lane per iteration, grid-stride): the

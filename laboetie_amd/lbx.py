@@ -362,9 +362,8 @@ class Lattice:
     def set_mp_coefficients(self, form):
         """MP_RECOMPUTED: the MP step recomputes the incoming scattering
         probabilities from each node's density and flow; MP_STORED: keeps them
-        (18 per node); MP_MIXED: keeps the 10 with c_z != 0 and recomputes the
-        others; MP_AUTO (default): recomputed for several FP64 tracers, stored
-        otherwise.  Same bits; from the next mp_init."""
+        (18 per node); MP_MIXED: as MP_RECOMPUTED; MP_AUTO (default): by the
+        size of the step's arrays.  Same bits; from the next mp_init."""
         _check(lib().lbx_set_mp_coefficients(self._h, int(form)), "set_mp_coefficients")
 
     @property
