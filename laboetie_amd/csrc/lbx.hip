@@ -130,6 +130,8 @@ struct lbx_ctx {
     std::vector<double> jpart_h;
     std::vector<double> jsum_trace;   // sum of j over the fluid nodes, 3 per step
     double* jflow = nullptr;          // lbx_flow: the flux of the last step
+    double* box = nullptr;            // full-box copies: the values of a run of box nodes
+    uint32_t box_n = 0;               // ... and how many it holds
 };
 
 // the forms that store populations as FP32 deviations (FP32-shift: FP32
@@ -237,6 +239,7 @@ void free_all(lbx_ctx* c) {
     dfree(c->l2ring);
     dfree(c->jpart);
     dfree(c->jflow);
+    dfree(c->box);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream), c->stream = nullptr;
@@ -364,49 +367,109 @@ void launch_lb_step(lbx_ctx* c, int64_t t, const double fm[3], const double fc[3
     }
 }
 
-// packed <-> full-box copies on the host (not on the hot path)
+// ---- full-box host arrays <-> packed device planes
+// A plane of the full box passes through a device buffer, a run of box nodes
+// at a time: the kernel below spreads (gathers) the packed values, and the copy
+// goes straight to (from) the caller's array.  One host thread doing this per
+// node through a temporary took 160 ms for the density and flux of a 256^3
+// medium; now it is the copy.
+
+// The buffer's nodes (*run), kept until the context goes.  32 MB, or as much
+// of it as the device still has.
+int box_buffer(lbx_ctx* c, double** box, uint32_t* run) {
+    for (uint32_t n = std::max(3u, std::min(c->N, 1u << 22)); !c->box;) {
+        const int st = dalloc(&c->box, n);
+        c->box_n = st ? 0 : n;
+        if (!st) break;
+        if (st != LBX_ERR_NOMEM || n <= 4096) return st;
+        n /= 4;
+    }
+    *box = c->box;
+    *run = c->box_n;
+    return LBX_OK;
+}
+
+// a packed plane of E as FP64 values of the box nodes [r0, r0 + n), 0 at
+// solids; FP32 deviations become rest + g
+template <typename E>
+__global__ __launch_bounds__(kBlock) void k_spread(const E* __restrict__ src, const uint32_t* __restrict__ map,
+                                                   double* __restrict__ box, uint32_t r0, uint32_t n, double rest) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t q = map[r0 + k];
+    double v = 0.0;
+    if (q != kSolidSlot) {
+        if constexpr (std::is_same<E, float>::value) v = rest + (double)src[q]; else v = src[q];
+    }
+    box[k] = v;
+}
+
+// the inverse: the fluid nodes of the run into their packed places
+template <typename E>
+__global__ __launch_bounds__(kBlock) void k_gather(E* __restrict__ dst, const uint32_t* __restrict__ map,
+                                                   const double* __restrict__ box, uint32_t r0, uint32_t n,
+                                                   double rest) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t q = map[r0 + k];
+    if (q == kSolidSlot) return;
+    if constexpr (std::is_same<E, float>::value) dst[q] = (float)(box[k] - rest); else dst[q] = box[k];
+}
+
+template <typename E>
+int download_plane(lbx_ctx* c, const E* src, double rest, double* host) {
+    double* box;
+    uint32_t run;
+    LBX_TRY(box_buffer(c, &box, &run));
+    for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
+        const uint32_t n = std::min(run, c->N - r0);
+        hipLaunchKernelGGL(k_spread<E>, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, src, c->map, box, r0, n, rest);
+        LBX_TRY(hipGetLastError());
+        LBX_TRY(hipMemcpyAsync(host + r0, box, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        LBX_TRY(hipStreamSynchronize(c->stream));
+    }
+    return LBX_OK;
+}
+
+template <typename E>
+int upload_plane(lbx_ctx* c, const double* host, double rest, E* dst) {
+    double* box;
+    uint32_t run;
+    LBX_TRY(box_buffer(c, &box, &run));
+    // the padding after the last node is 0
+    LBX_TRY(hipMemsetAsync(dst + c->Nf, 0, (c->Np - c->Nf) * sizeof(E), c->stream));
+    for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
+        const uint32_t n = std::min(run, c->N - r0);
+        LBX_TRY(hipMemcpyAsync(box, host + r0, (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+        hipLaunchKernelGGL(k_gather<E>, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, dst, c->map, box, r0, n, rest);
+        LBX_TRY(hipGetLastError());
+        LBX_TRY(hipStreamSynchronize(c->stream));
+    }
+    return LBX_OK;
+}
+
 int download_full(lbx_ctx* c, const double* dsrc, int planes, double* host_full) {
-    std::vector<double> tmp((size_t)planes * c->Np);
-    LBX_TRY(hipMemcpyAsync(tmp.data(), dsrc, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    LBX_TRY(hipStreamSynchronize(c->stream));
-    std::memset(host_full, 0, (size_t)planes * c->N * sizeof(double));
     for (int p = 0; p < planes; ++p)
-        for (uint32_t i = 0; i < c->Nf; ++i)
-            host_full[(size_t)p * c->N + (c->nodes_h[i] & kIndexMask)] = tmp[(size_t)p * c->Np + i];
+        LBX_TRY(download_plane(c, dsrc + (size_t)p * c->Np, 0.0, host_full + (size_t)p * c->N));
     return LBX_OK;
 }
 
 int upload_full(lbx_ctx* c, const double* const* host_planes, int planes, double* ddst) {
-    std::vector<double> tmp((size_t)planes * c->Np, 0.0);
-    for (int p = 0; p < planes; ++p)
-        for (uint32_t i = 0; i < c->Nf; ++i) tmp[(size_t)p * c->Np + i] = host_planes[p][c->nodes_h[i] & kIndexMask];
-    LBX_TRY(hipMemcpyAsync(ddst, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    return hip_status(hipStreamSynchronize(c->stream));
+    for (int p = 0; p < planes; ++p) LBX_TRY(upload_plane(c, host_planes[p], 0.0, ddst + (size_t)p * c->Np));
+    return LBX_OK;
 }
 
 // FP32-shift populations <-> full-box FP64 n = a0 rho0 + g (0 at solid nodes)
 int download_shift(lbx_ctx* c, const float* gsrc, double* n_full) {
-    std::vector<float> tmp((size_t)kQ * c->Np);
-    LBX_TRY(hipMemcpyAsync(tmp.data(), gsrc, tmp.size() * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    LBX_TRY(hipStreamSynchronize(c->stream));
-    std::memset(n_full, 0, (size_t)kQ * c->N * sizeof(double));
-    for (int l = 0; l < kQ; ++l) {
-        const double rest = a0(l) * c->rho0;
-        for (uint32_t i = 0; i < c->Nf; ++i)
-            n_full[(size_t)l * c->N + (c->nodes_h[i] & kIndexMask)] = rest + (double)tmp[(size_t)l * c->Np + i];
-    }
+    for (int l = 0; l < kQ; ++l)
+        LBX_TRY(download_plane(c, gsrc + (size_t)l * c->Np, a0(l) * c->rho0, n_full + (size_t)l * c->N));
     return LBX_OK;
 }
 
 int upload_shift(lbx_ctx* c, const double* n_full, float* gdst) {
-    std::vector<float> tmp((size_t)kQ * c->Np, 0.0f);
-    for (int l = 0; l < kQ; ++l) {
-        const double rest = a0(l) * c->rho0;
-        for (uint32_t i = 0; i < c->Nf; ++i)
-            tmp[(size_t)l * c->Np + i] = (float)(n_full[(size_t)l * c->N + (c->nodes_h[i] & kIndexMask)] - rest);
-    }
-    LBX_TRY(hipMemcpyAsync(gdst, tmp.data(), tmp.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    return hip_status(hipStreamSynchronize(c->stream));
+    for (int l = 0; l < kQ; ++l)
+        LBX_TRY(upload_plane(c, n_full + (size_t)l * c->N, a0(l) * c->rho0, gdst + (size_t)l * c->Np));
+    return LBX_OK;
 }
 
 // The MP tiles of the context's geometry: counted, grouped, placed and
@@ -643,7 +706,7 @@ int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precisio
     const uint64_t N = (uint64_t)lx * ly * lz, Np = (N + 63) / 64 * 64;
     const uint64_t pop = f32_storage(precision) ? 4 : 8;  // populations; also win and u* of moment propagation
     uint64_t b = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + N * 8 +
-                 sizeof(Ctrl) + kRing * 8;
+                 std::min<uint64_t>(N, 1u << 22) * 8 + sizeof(Ctrl) + kRing * 8;
     if (with_mp > 0) {  // with_mp tracers, each with adsorption (the upper bound)
         const uint64_t T = (uint64_t)std::min(with_mp, kMaxTracers);
         const Bricks br = make_bricks((uint32_t)lx, (uint32_t)ly, (uint32_t)lz);
@@ -1240,20 +1303,20 @@ int lbx_mp_get_tracer(lbx_ctx* c, int32_t tracer, double* P, double* Pa) {
     if (!c) return LBX_ERR_ARG;
     if (!c->mp_ready || c->mpp.active) return LBX_ERR_STATE;  // a begun chunk is waited for first
     if (tracer < 0 || tracer >= c->ntr) return LBX_ERR_ARG;
-    // the tracer's three components into (3,lx,ly,lz), 0 at solids, a run of
-    // box nodes at a time through a device buffer
-    constexpr uint32_t kRun = 1u << 22;
-    double* box = nullptr;
-    LBX_TRY(dalloc(&box, 3 * (uint64_t)std::min(c->N, kRun)));
+    // the tracer's three components into (3,lx,ly,lz), 0 at solids, a run of box nodes at a time
+    double* box;
+    uint32_t run;
+    LBX_TRY(box_buffer(c, &box, &run));
+    run /= 3;
     auto fetch = [&](const double* src, double* dst) -> int {
-        for (uint64_t r0 = 0; r0 < c->N; r0 += kRun) {
-            const uint32_t n = (uint32_t)std::min<uint64_t>(kRun, c->N - r0);
+        for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
+            const uint32_t n = std::min(run, c->N - r0);
             LBX_TRY(hipMemsetAsync(box, 0, 3 * (uint64_t)n * sizeof(double), c->stream));
             hipLaunchKernelGGL(k_mp_box, dim3(c->mp_ntiles), dim3(kBlock), 0, c->stream, src, c->mpt, 0u, c->nodes,
-                               c->ntr, tracer, box, (uint32_t)r0, n);
+                               c->ntr, tracer, box, r0, n);
             LBX_TRY(hipGetLastError());
-            LBX_TRY(hipMemcpyAsync(dst + 3 * r0, box, 3 * (uint64_t)n * sizeof(double), hipMemcpyDeviceToHost,
-                                   c->stream));
+            LBX_TRY(hipMemcpyAsync(dst + 3 * (size_t)r0, box, 3 * (uint64_t)n * sizeof(double),
+                                   hipMemcpyDeviceToHost, c->stream));
             LBX_TRY(hipStreamSynchronize(c->stream));
         }
         return LBX_OK;
@@ -1266,7 +1329,6 @@ int lbx_mp_get_tracer(lbx_ctx* c, int32_t tracer, double* P, double* Pa) {
         else
             std::memset(Pa, 0, 3 * (size_t)c->N * sizeof(double));
     }
-    dfree(box);
     return st;
 }
 

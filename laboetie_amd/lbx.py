@@ -415,9 +415,9 @@ class Lattice:
 
     def flow(self):
         """(rho, j) after the last step taken (also during a paused run)."""
-        rho, jx, jy, jz = (np.zeros(self.N) for _ in range(4))
-        _check(lib().lbx_flow(self._h, _ptr(rho), _ptr(jx), _ptr(jy), _ptr(jz)), "flow")
-        return rho, np.stack([jx, jy, jz])
+        rho, j = np.zeros(self.N), np.zeros((3, self.N))
+        _check(lib().lbx_flow(self._h, _ptr(rho), *[_ptr(a) for a in j]), "flow")
+        return rho, j
 
     def l2err_trace(self):
         """Every l2err of the last equilibrate call."""
@@ -431,10 +431,10 @@ class Lattice:
     def get_state(self, populations=True):
         """(n, rho, j) on the full box; n is None with populations=False."""
         n = np.zeros(19 * self.N) if populations else None
-        rho, jx, jy, jz = (np.zeros(self.N) for _ in range(4))
-        _check(lib().lbx_get_state(self._h, _ptr(n) if populations else None, _ptr(rho), _ptr(jx), _ptr(jy),
-                                   _ptr(jz)), "get_state")
-        return n, rho, np.stack([jx, jy, jz])
+        rho, j = np.zeros(self.N), np.zeros((3, self.N))
+        _check(lib().lbx_get_state(self._h, _ptr(n) if populations else None, _ptr(rho), *[_ptr(a) for a in j]),
+               "get_state")
+        return n, rho, j
 
     def mp_init(self, fext, Db, ka=0.0, kd=0.0, flow=None):
         fe = np.ascontiguousarray(fext, np.float64)
@@ -599,12 +599,12 @@ class Batch:
         v = np.zeros(3 * max(vacf_rows, 1))
         lx, ly, lz = self.dims[iid]
         N = lx * ly * lz
-        fl = [np.zeros(N) for _ in range(4)] if flow else [None] * 4
+        rho, j = (np.zeros(N), np.zeros((3, N))) if flow else (None, [None] * 3)
         _check(lib().lbxb_result(self._h, int(iid), _ptr(d), _ptr(v) if vacf_rows else None, int(vacf_rows),
-                                 *[_ptr(a) for a in fl]), "lbxb_result")
+                                 _ptr(rho), *[_ptr(a) for a in j]), "lbxb_result")
         out = dict(deff=d, vacf=v[:3 * vacf_rows].reshape(-1, 3))
         if flow:
-            out["rho"], out["j"] = fl[0], np.stack(fl[1:])
+            out["rho"], out["j"] = rho, j
         return out
 
     def set_block(self, lb_block, mp_block):
