@@ -85,6 +85,7 @@ struct lbx_ctx {
     double* rho = nullptr;
     uint32_t* nodes = nullptr;
     uint32_t* map = nullptr;
+    uint32_t* pulls = nullptr;   // LB pull sources (small lattices; else NULL)
     uint32_t ntiles = 0;
     unsigned long long* slots = nullptr;  // [3][kSlots] l2err slots
     Ctrl* ctrl = nullptr;
@@ -234,6 +235,7 @@ void free_all(lbx_ctx* c) {
     dfree(c->rho);
     dfree(c->nodes);
     dfree(c->map);
+    dfree(c->pulls);
     dfree(c->slots);
     dfree(c->ctrl);
     dfree(c->l2ring);
@@ -291,6 +293,14 @@ void timer_end(lbx_ctx* c, int which, int64_t launches) {
     }
 }
 
+// Up to this many fluid nodes the LB step takes its pull sources from a table
+// (StepArgs::pulls, 72 bytes a node): while everything a step reads sits in L2
+// its time is the chain of round trips, not the bytes.  us per step without /
+// with it, FP64, FP32-shift, FP32-store: 2 185 nodes 5.88 / 5.54, 5.79 / 5.36,
+// 5.83 / 5.37; 85 056 nodes 9.14 / 8.90, 7.53 / 6.80, 7.71 / 7.11.  Asking for
+// the flags late without the table lost at 128^3 and above (registers).
+constexpr uint32_t kTabNodes = 131072;
+
 template <typename E>
 E* pop_buf(lbx_ctx* c, int b) {
     if constexpr (std::is_same<E, float>::value) return c->g[b]; else return c->f[b];
@@ -305,6 +315,7 @@ StepArgs<E, R> step_args(lbx_ctx* c, int64_t t, const double fm[3], const double
     if constexpr (std::is_same<R, float>::value) a.j = c->j32; else a.j = c->j;
     a.nodes = c->nodes;
     a.map = c->map;
+    a.pulls = c->pulls;
     a.slots = c->slots;
     a.l2ring = c->l2ring;
     a.ctrl = c->ctrl;
@@ -349,20 +360,23 @@ void launch_lb_step(lbx_ctx* c, int64_t t, const double fm[3], const double fc[3
         StepArgs<float> a = step_args<float>(c, t, fm, fc, check_after, target, write_l2, check_every, check_base);
         a.have_prev = have_prev;
         auto kern = c->wide ? (c->nt ? k_lb_step<true, float, float, true> : k_lb_step<true, float>)
-                            : (c->nt ? k_lb_step<false, float, float, true> : k_lb_step<false, float>);
+                    : c->pulls ? k_lb_step<false, float, float, false, true>
+                               : (c->nt ? k_lb_step<false, float, float, true> : k_lb_step<false, float>);
         hipLaunchKernelGGL(kern, dim3(gt), dim3(kBlock), 0, c->stream, a);
     } else if (c->prec == LBX_PREC_FP32_STORE) {
         StepArgs<float, double> a =
             step_args<float, double>(c, t, fm, fc, check_after, target, write_l2, check_every, check_base);
         a.have_prev = have_prev;
         auto kern = c->wide ? (c->nt ? k_lb_step<true, float, double, true> : k_lb_step<true, float, double>)
-                            : (c->nt ? k_lb_step<false, float, double, true> : k_lb_step<false, float, double>);
+                    : c->pulls ? k_lb_step<false, float, double, false, true>
+                               : (c->nt ? k_lb_step<false, float, double, true> : k_lb_step<false, float, double>);
         hipLaunchKernelGGL(kern, dim3(gt), dim3(kBlock), 0, c->stream, a);
     } else {
         StepArgs<double> a = step_args<double>(c, t, fm, fc, check_after, target, write_l2, check_every, check_base);
         a.have_prev = have_prev;
         auto kern = c->wide ? (c->nt ? k_lb_step<true, double, double, true> : k_lb_step<true, double>)
-                            : (c->nt ? k_lb_step<false, double, double, true> : k_lb_step<false, double>);
+                    : c->pulls ? k_lb_step<false, double, double, false, true>
+                               : (c->nt ? k_lb_step<false, double, double, true> : k_lb_step<false, double>);
         hipLaunchKernelGGL(kern, dim3(gt), dim3(kBlock), 0, c->stream, a);
     }
 }
@@ -706,6 +720,7 @@ int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precisio
     const uint64_t N = (uint64_t)lx * ly * lz, Np = (N + 63) / 64 * 64;
     const uint64_t pop = f32_storage(precision) ? 4 : 8;  // populations; also win and u* of moment propagation
     uint64_t b = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + N * 8 +
+                 18 * 4 * std::min<uint64_t>(Np, (kTabNodes + 63) / 64 * 64) +
                  std::min<uint64_t>(N, 1u << 22) * 8 + sizeof(Ctrl) + kRing * 8;
     if (with_mp > 0) {  // with_mp tracers, each with adsorption (the upper bound)
         const uint64_t T = (uint64_t)std::min(with_mp, kMaxTracers);
@@ -781,6 +796,7 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     if (!st) st = dalloc(&c->rho, c->Np);
     if (!st) st = dalloc(&c->nodes, (uint64_t)c->Nf);
     if (!st) st = dalloc(&c->map, (uint64_t)c->N);
+    if (!st && c->Nf <= kTabNodes) st = dalloc(&c->pulls, 18 * c->Np);
     if (!st) st = dalloc(&c->slots, 3 * kSlots);
     if (!st) st = dalloc(&c->ctrl, 1);
     if (!st) st = dalloc(&c->l2ring, kRing);
@@ -790,6 +806,11 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
                                             hipMemcpyHostToDevice, c->stream));
     if (!st) st = hip_status(hipMemcpyAsync(c->map, map.data(), c->N * sizeof(uint32_t), hipMemcpyHostToDevice,
                                             c->stream));
+    if (!st && c->pulls) {
+        hipLaunchKernelGGL(k_pull_table, dim3(c->ntiles), dim3(kBlock), 0, c->stream, c->pulls, c->nodes, c->map, c->dlx,
+                           c->dly, c->lz, c->Nf, (uint32_t)c->Np);
+        st = hip_status(hipGetLastError());
+    }
     for (int b = 0; b < 2; ++b) {
         if (!st && !shift) st = hip_status(hipMemsetAsync(c->f[b], 0, kQ * c->Np * sizeof(double), c->stream));
         if (!st && shift) st = hip_status(hipMemsetAsync(c->g[b], 0, kQ * c->Np * sizeof(float), c->stream));

@@ -121,6 +121,8 @@ struct StepArgs {
     int32_t pad_ = 0;
     int64_t check_base = 0;
     R check_inv = R(1);     // 1 / check_every
+    // TAB steps: element of the populations that direction l of node i pulls, at [(l-1) Np + i]
+    const uint32_t* pulls = nullptr;
     // non-NULL: each block writes the sum of j(t) over its nodes (3 doubles,
     // in a fixed order) to jpart[3 * tile ...] (the per-step total mass flux)
     double* jpart = nullptr;
@@ -219,14 +221,29 @@ __device__ __forceinline__ void block_partial(const double (&v)[NV], double* out
 // node is solid, left i itself in direction inv(L).
 // The two candidate sources differ only in the lane's element index, so one
 // load per direction serves both.
-template <int L, bool Wide, typename E>
-__device__ __forceinline__ E pull(const View<Wide, E>& fin, uint32_t Np, uint32_t i, const Neighbours& nb) {
+template <int L>
+__device__ __forceinline__ uint32_t pull_source(uint32_t Np, uint32_t i, const Neighbours& nb) {
     if constexpr (L == 0) {
-        return fin.ld(i);
+        return i;
     } else {
         const uint32_t q = nb.q[kInv[L]];  // r - c_L = r + c_inv(L)
-        return fin.ld(q != kSolidSlot ? (uint32_t)L * Np + q : (uint32_t)kInv[L] * Np + i);
+        return q != kSolidSlot ? (uint32_t)L * Np + q : (uint32_t)kInv[L] * Np + i;
     }
+}
+template <int L, bool Wide, typename E>
+__device__ __forceinline__ E pull(const View<Wide, E>& fin, uint32_t Np, uint32_t i, const Neighbours& nb) {
+    return fin.ld(pull_source<L>(Np, i, nb));
+}
+
+// the pull sources of every node (StepArgs::pulls)
+__global__ __launch_bounds__(kBlock) void k_pull_table(uint32_t* __restrict__ pulls, const uint32_t* __restrict__ nodes,
+                                                       const uint32_t* __restrict__ map, FastDiv dlx, FastDiv dly,
+                                                       uint32_t lz, uint32_t Nf, uint32_t Np) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= Nf) return;
+    Neighbours nb;
+    nb.load(map, nodes[i] & kIndexMask, dlx, dly, lz);
+    static_for<1, kQ>([&](auto I) { pulls[(uint64_t)(I - 1) * Np + i] = pull_source<I>(Np, i, nb); });
 }
 
 // One time step, fused: pull-streaming with bounce-back of the post-collision
@@ -242,7 +259,12 @@ __device__ __forceinline__ E pull(const View<Wide, E>& fin, uint32_t Np, uint32_
 // consecutive packed nodes, i = tile*BLOCK + lane, valid below a.Nf), `stripe`
 // picks its l2err slot, and `first_block` is the one block of the lattice that
 // writes the step's control fields and clears the next step's slots.
-template <int BLOCK, bool Wide, typename E, typename R = E, bool NT = false>
+//
+// TAB (small lattices, whose step is a chain of round trips to memory and not
+// bytes): the pull sources come from a table in place of node word and map,
+// and the stop flags are looked at after the populations have been asked for:
+// two round trips instead of four.
+template <int BLOCK, bool Wide, typename E, typename R = E, bool NT = false, bool TAB = false>
 __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t tile, uint32_t stripe,
                                              bool first_block) {
     constexpr bool kShift = std::is_same<E, float>::value;  // deviations stored in FP32
@@ -250,13 +272,28 @@ __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t t
     // Each wave's work is a chain of dependent memory round trips, so
     // independent requests go out together: the node word, the stop flags
     // and the previous step's l2err slots (read whether or not a flag is set).
-    const uint32_t node = i < a.Nf ? ld(a.nodes, i) : 0u;
+    const uint32_t node = !TAB && i < a.Nf ? ld(a.nodes, i) : 0u;
     __shared__ int32_t stop_flag;
     __shared__ unsigned long long prev_bits;
     __syncthreads();  // a previous step of this block (persistent launches) has read both
+    bool stop = false;
+    unsigned long long prev = 0ull;
     if (threadIdx.x < 64) {
-        const bool stop = ((int)(vload(&a.ctrl->stop) != 0) | (int)(vload(&a.ctrl->negpop) >= 0)) != 0;
-        const unsigned long long v = a.have_prev ? slots_max(a.slots + ((a.t - 1) % 3) * kSlots) : 0ull;
+        stop = ((int)(vload(&a.ctrl->stop) != 0) | (int)(vload(&a.ctrl->negpop) >= 0)) != 0;
+        if (a.have_prev) prev = vload(a.slots + ((a.t - 1) % 3) * kSlots + (threadIdx.x & (kSlots - 1)));
+    }
+    E early[TAB ? kQ : 1];  // TAB: the populations
+    if constexpr (TAB)
+        if (i < a.Nf) {
+            const uint32_t Np = (uint32_t)a.Np;
+            const View<Wide, E> fin(a.fin, kQ * a.Np);
+            uint32_t src[kQ];
+            static_for<1, kQ>([&](auto I) { src[I] = ld(a.pulls, (I - 1) * Np + i); });
+            early[0] = fin.ld(i);
+            static_for<1, kQ>([&](auto I) { early[I] = fin.ld(src[I]); });
+        }
+    if (threadIdx.x < 64) {
+        const unsigned long long v = wave_max_u64(prev);
         if (threadIdx.x == 0) {
             stop_flag = stop ? 1 : 0;
             prev_bits = v;
@@ -320,7 +357,7 @@ __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t t
         const View<Wide, E> fin(a.fin, kQ * a.Np), fout(a.fout, kQ * a.Np);
         const View<Wide, R> jv(a.j, 3 * a.Np);
         Neighbours nb;
-        nb.load(a.map, node & kIndexMask, a.dlx, a.dly, a.lz);
+        if constexpr (!TAB) nb.load(a.map, node & kIndexMask, a.dlx, a.dly, a.lz);
         // l2err of this step is measured: always in FP64; in the FP32 storage
         // forms only at the check steps, the only ones that read and keep j
         const bool chk = a.write_l2 && is_check(a.t, a.check_base, a.check_every);
@@ -331,7 +368,9 @@ __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t t
             jo[2] = jv.ld(2 * Np + i);
         }
         R f[kQ];
-        static_for<0, kQ>([&](auto I) { f[I] = (R)pull<I, Wide, E>(fin, Np, i, nb); });
+        static_for<0, kQ>([&](auto I) {
+            if constexpr (TAB) f[I] = (R)early[I]; else f[I] = (R)pull<I, Wide, E>(fin, Np, i, nb);
+        });
         if constexpr (kShift)  // n < 0  <=>  g < -a0 rho0
             static_for<0, kQ>([&](auto I) { neg = neg || (f[I] < -((R)a0(I) * a.rho0)); });
         else
@@ -422,9 +461,9 @@ constexpr int kLbMinWaves = (std::is_same<E, float>::value && std::is_same<R, do
 #ifndef LBX_NT_MIN_BYTES  // population footprint (both sets) above which LB stores stream
 #define LBX_NT_MIN_BYTES (256ull << 20)
 #endif
-template <bool Wide, typename E, typename R = E, bool NT = false>
-__global__ __launch_bounds__(kBlock, (kLbMinWaves<E, R>)) void k_lb_step(StepArgs<E, R> a) {
-    lb_step_tile<kBlock, Wide, E, R, NT>(a, xcd_tile(), blockIdx.x, blockIdx.x == 0);
+template <bool Wide, typename E, typename R = E, bool NT = false, bool TAB = false>
+__global__ __launch_bounds__(kBlock, (TAB ? 2 : kLbMinWaves<E, R>)) void k_lb_step(StepArgs<E, R> a) {
+    lb_step_tile<kBlock, Wide, E, R, NT, TAB>(a, xcd_tile(), blockIdx.x, blockIdx.x == 0);
 }
 
 // l2err of the last step of a launch run, which no later step kernel reads
