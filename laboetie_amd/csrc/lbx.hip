@@ -600,6 +600,11 @@ int alloc_fields(lbx_ctx* c, int ntr, bool any_ads, bool stored) {
     return st;
 }
 
+template <int T, typename W>
+__global__ __launch_bounds__(kBlock) void k_mp_prep(MpPrepArgs<W> a) {
+    mp_prep_tile<T, W>(a, xcd_tile());
+}
+
 // k_mp_prep + the VACF(0) reduction for the context's tracers
 template <typename W>
 void launch_mp_prep(lbx_ctx* c, const double fext[3], double eps) {
@@ -625,7 +630,7 @@ void launch_mp_prep(lbx_ctx* c, const double fext[3], double eps) {
     const uint32_t gt = c->mp_ntiles;
     with_tracers(c->ntr, [&](auto TT) {
         constexpr int T = TT;
-        hipLaunchKernelGGL((k_mp_prep<T, W>), dim3(gt), dim3(kBlock), 0, c->stream, a, 0u);
+        hipLaunchKernelGGL((k_mp_prep<T, W>), dim3(gt), dim3(kBlock), 0, c->stream, a);
         hipLaunchKernelGGL(k_mp_reduce<3 * T>, dim3(1), dim3(kBlock), 0, c->stream, c->part, gt, nullptr, c->ctrl, 0,
                            (int64_t)0, 0, 0.0, 0.0);
     });
@@ -843,7 +848,7 @@ int lbx_init_rest(lbx_ctx* c, double rho0) {
     c->eq.active = false;  // a paused run is abandoned
     if (f32_storage(c->prec)) c->rho0 = rho0;  // the deviations follow the rest state
     hipLaunchKernelGGL(k_init_rest, dim3(c->ntiles), dim3(kBlock), 0, c->stream, c->f[0], c->g[0], c->j32, c->rho,
-                       c->j, 0u, c->Nf, c->Np, rho0);
+                       c->j, c->Nf, c->Np, rho0);
     c->pre = 0;
     LBX_TRY(hipGetLastError());
     return hip_status(hipStreamSynchronize(c->stream));
@@ -912,11 +917,11 @@ int end_run(lbx_ctx* c) {
             // carries F(t)/2 as in the step kernel
             const double* Ft = t > q.switch_step ? q.F : zero;
             hipLaunchKernelGGL(k_extract_shift, dim3(gt), dim3(kBlock), 0, c->stream, c->g[src], c->g[dst], c->rho,
-                               c->j, c->nodes, c->map, c->dlx, c->dly, c->lz, 0u, c->Nf, c->Np, c->rho0,
+                               c->j, c->nodes, c->map, c->dlx, c->dly, c->lz, c->Nf, c->Np, c->rho0,
                                Ft[0] / 2.0, Ft[1] / 2.0, Ft[2] / 2.0);
         } else {
             hipLaunchKernelGGL(k_extract, dim3(gt), dim3(kBlock), 0, c->stream, c->f[src], c->f[dst], c->rho,
-                               c->nodes, c->map, c->dlx, c->dly, c->lz, 0u, c->Nf, c->Np);
+                               c->nodes, c->map, c->dlx, c->dly, c->lz, c->Nf, c->Np);
         }
         LBX_TRY(hipGetLastError());
         c->pre = dst;
@@ -943,14 +948,14 @@ int lbx_equilibrate_begin(lbx_ctx* c, double target_error, const double fext[3],
                                c->stream));
     if (c->prec == LBX_PREC_FP32_SHIFT) {
         hipLaunchKernelGGL(k_collide_packed_shift<float>, dim3(gt), dim3(kBlock), 0, c->stream, c->g[0], c->rho,
-                           c->j, c->j32, 0.0f, 0.0f, 0.0f, 0u, c->Nf, c->Np, c->A32, c->B32, (float)c->C,
+                           c->j, c->j32, 0.0f, 0.0f, 0.0f, c->Nf, c->Np, c->A32, c->B32, (float)c->C,
                            c->rho0);
     } else if (c->prec == LBX_PREC_FP32_STORE) {  // j_old is j itself
         hipLaunchKernelGGL(k_collide_packed_shift<double>, dim3(gt), dim3(kBlock), 0, c->stream, c->g[0], c->rho,
-                           c->j, c->j, 0.0, 0.0, 0.0, 0u, c->Nf, c->Np, c->A, c->B, c->C, c->rho0);
+                           c->j, c->j, 0.0, 0.0, 0.0, c->Nf, c->Np, c->A, c->B, c->C, c->rho0);
     } else {
         hipLaunchKernelGGL(k_collide_packed, dim3(gt), dim3(kBlock), 0, c->stream, c->f[0], c->rho, c->j, 0.0, 0.0,
-                           0.0, 0u, c->Nf, c->Np, c->A, c->B, c->C);
+                           0.0, c->Nf, c->Np, c->A, c->B, c->C);
     }
     LBX_TRY(hipGetLastError());
     LBX_TRY(reset_ctrl(c));

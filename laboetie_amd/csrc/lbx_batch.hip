@@ -50,6 +50,7 @@ namespace {
 constexpr int kTile = 256;                 // allocation unit (nodes) of an instance's range
 constexpr uint32_t kNoInst = 0xFFFFFFFFu;
 constexpr int kRoundMax = 1024;            // launches per phase per round (vtrace rows)
+constexpr size_t kStage = 1u << 20;
 constexpr size_t kGraphCacheMax = 64;      // captured round graphs kept at once
 
 struct BInst {
@@ -74,7 +75,21 @@ struct BInst {
     uint32_t mp_tile0, mp_ntiles; // its MP tiles
     double lambda;
     TracerParams tp;
+    // set-up of its moment propagation: the end of its LB phase (step, F/2), lb.in's f_ext
+    int64_t end_t;
+    double end_fm[3], F[3];
 };
+
+// the control block of an instance at the start of a stage or phase
+__device__ __forceinline__ void reset_ctrl(Ctrl* c, int64_t check_after) {
+    Ctrl h{};
+    h.negpop = -1;
+    for (int k = 0; k < 2; ++k) {
+        h.l2min[k] = HUGE_VAL;
+        h.l2min_step[k] = check_after;
+    }
+    *c = h;
+}
 
 template <typename E, typename R = E>
 struct BatchView {
@@ -236,6 +251,107 @@ __device__ __forceinline__ void kb_mp_reduce_inst(const BatchMpView<W>& v, uint3
 template <typename W>
 __global__ __launch_bounds__(kBlock) void kb_mp_reduce_last(BatchMpView<W> v) {
     kb_mp_reduce_inst(v, blockIdx.x);
+}
+
+// Admission of one instance in one launch: its nodes at rest and through the
+// opening collision of step 1 (k_init_rest, k_collide_packed*: the same
+// operations), its tiles' owner, and (first block) its control block, l2err
+// slots and ring.
+template <typename E, typename R>
+__global__ __launch_bounds__(kBlock) void kb_admit(E* f, R* jold, double* __restrict__ rho, double* __restrict__ j,
+                                                   BInst in, uint32_t id, uint32_t* __restrict__ tile_inst,
+                                                   unsigned long long* __restrict__ slots, double* __restrict__ l2ring,
+                                                   Ctrl* ctrl, uint64_t Np) {
+    if (threadIdx.x == 0) tile_inst[in.tile_first + blockIdx.x] = id;
+    if (blockIdx.x == 0) {
+        for (uint32_t k = threadIdx.x; k < 3 * kSlots; k += kBlock) slots[(uint64_t)id * 3 * kSlots + k] = 0ull;
+        for (uint32_t k = threadIdx.x; k < (uint32_t)kRing; k += kBlock) l2ring[(uint64_t)id * kRing + k] = 0.0;
+        if (threadIdx.x == 0) reset_ctrl(ctrl + id, 2);
+    }
+    const uint32_t i = in.node_off + blockIdx.x * kBlock + threadIdx.x;
+    if (i >= in.node_end) return;
+    const R z = R(0);
+    rho[i] = in.rho0;
+    for (int c = 0; c < 3; ++c) {
+        j[c * Np + i] = 0.0;
+        jold[c * Np + i] = z;
+    }
+    const R A = (R)in.A, B = (R)in.B, C = (R)in.C;
+    static_for<0, kQ>([&](auto I) {
+        constexpr int L = I;
+        if constexpr (std::is_same<E, float>::value) {
+            const R drho = (R)(in.rho0 - in.rho0), full = (R)in.rho0 + drho;
+            R ux, uy, uz;
+            shift_velocity<R>(z, z, z, full, ux, uy, uz);
+            f[(uint64_t)L * Np + i] = (float)collide_shift<L, R>(z, drho, z, z, z, ux, uy, uz, z, z, z, A, B, C);
+        } else {
+            const double d = in.rho0, u = 0.0 / d;
+            f[(uint64_t)L * Np + i] = collide_pop<L>(d * a0(L), d, 0.0, 0.0, 0.0, u, u, u, 0.0, 0.0, 0.0, A, B, C);
+        }
+    });
+}
+
+// The post-streaming state, density and flux at the end of the LB phase of
+// the instances whose 256-node tiles are listed in v.act
+template <typename E>
+__global__ __launch_bounds__(kBlock) void kb_extract(BatchView<E, E> v, double* rho, double* j) {
+    const uint32_t tile = v.act[blockIdx.x];
+    const BInst& in = v.insts[v.tile_inst[tile]];
+    const uint32_t i = tile * kTile + threadIdx.x;
+    if (i >= in.node_end || in.end_t <= 0) return;
+    Neighbours nb;
+    nb.load(v.maps + in.map_off, v.nodes[i] & kIndexMask, in.dlx, in.dly, in.lz);
+    const E* src = (in.end_t - 1) & 1 ? v.f1 : v.f0;
+    E* dst = in.end_t & 1 ? v.f1 : v.f0;
+    if constexpr (std::is_same<E, float>::value)
+        extract_node_shift(src, dst, rho, j, nb, i, v.Np, in.rho0, in.end_fm[0], in.end_fm[1], in.end_fm[2]);
+    else
+        extract_node(src, dst, rho, nb, i, v.Np);
+}
+
+// control blocks of the instances ids, as their moment propagation starts
+__global__ __launch_bounds__(64) void kb_reset_ctrl(Ctrl* ctrl, const uint32_t* __restrict__ ids, uint32_t n) {
+    const uint32_t k = blockIdx.x * 64 + threadIdx.x;
+    if (k < n) reset_ctrl(ctrl + ids[k], 2);
+}
+
+// mp_prep_tile on the MP tiles listed in v.act
+template <typename W>
+__global__ __launch_bounds__(kBlock) void kb_mp_prep(BatchMpView<W> v, const double* rho, const double* j, uint64_t Np,
+                                                     double eps) {
+    const uint32_t tile = v.act[xcd_tile()];
+    const uint32_t id = v.tile_inst[tile];
+    const BInst& in = v.insts[id];
+    MpPrepArgs<W> a;
+    a.t = v.t;
+    a.f = v.f;
+    a.rho = rho;
+    a.j = j;
+    a.nodes = v.nodes;
+    a.map = v.maps + in.map_off;
+    a.partials = v.part[0];
+    a.ctrl = v.ctrl + id;
+    a.dlx = in.dlx;
+    a.dly = in.dly;
+    a.lz = in.lz;
+    a.Np = Np;
+    a.fx = in.F[0];
+    a.fy = in.F[1];
+    a.fz = in.F[2];
+    a.lambda = in.lambda;
+    a.eps = eps;
+    a.tp = in.tp;
+    mp_prep_tile<1, W>(a, tile);
+}
+
+// VACF(0) of the instances ids (one block each)
+template <typename W>
+__global__ __launch_bounds__(kBlock) void kb_mp_vacf0(BatchMpView<W> v, const uint32_t* __restrict__ ids) {
+    __shared__ double lds[kBlock / 64 * 3];
+    const uint32_t id = ids[blockIdx.x];
+    const BInst& in = v.insts[id];
+    mp_reduce_block<3, kBlock>(v.part[0] + 3 * (uint64_t)in.mp_tile0, in.mp_ntiles, nullptr, v.ctrl + id, 0, 0, 0, 0.0,
+                               0.0, lds);
 }
 
 // The steps of one phase of a round in one cooperative launch: every block
@@ -407,6 +523,11 @@ struct lbxb {
     MpFields<float> mpf32;       // FP32-storage forms
     uint32_t* walk = nullptr;    // scratch of the layout builds, grown as needed
     uint64_t walk_cap = 0;
+    uint32_t* ids = nullptr;     // [max instances]
+    // admissions go through two pinned buffers in turn (kStage bytes each)
+    char* stage[2] = {nullptr, nullptr};
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    int stage_at = 0;
     MpBuild* builds = nullptr;   // [max instances]
     MpBuilt* built = nullptr;
     uint8_t* split = nullptr;
@@ -486,6 +607,13 @@ void free_all(lbxb* b) {
     dfree(b->builds);
     dfree(b->built);
     dfree(b->split);
+    dfree(b->ids);
+    for (int k = 0; k < 2; ++k) {
+        if (b->stage[k]) (void)hipHostFree(b->stage[k]);
+        if (b->stage_ev[k]) (void)hipEventDestroy(b->stage_ev[k]);
+        b->stage[k] = nullptr;
+        b->stage_ev[k] = nullptr;
+    }
     dfree(b->vtrace);
     for (auto& e : b->ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
@@ -827,64 +955,24 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         in.mp_ntiles = built[k].ntiles;
         for (uint32_t t = 0; t < 2 * in.ntiles; ++t)
             b->mp_tile_inst_h[in.mp_tile0 + t] = t < in.mp_ntiles ? ids[k] : kNoInst;
-        LBX_TRY(hipMemcpyAsync(b->mp_tile_inst + in.mp_tile0, b->mp_tile_inst_h.data() + in.mp_tile0,
-                               2 * (uint64_t)in.ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
     }
+    LBX_TRY(hipMemcpyAsync(b->mp_tile_inst, b->mp_tile_inst_h.data(), b->mp_tile_inst_h.size() * sizeof(uint32_t),
+                           hipMemcpyHostToDevice, b->stream));
     for (size_t k : gen) b->hi[ids[k]].general = true;
     return LBX_OK;
 }
 
-template <typename W>
-void launch_mp_prep(lbxb* b, uint32_t id, double eps) {
-    const HostInst& h = b->hi[id];
-    const BInst& in = b->tab[id];
-    MpPrepArgs<W> a;
-    a.t = b->mpt;
-    a.f = mp_fields<W>(b);
-    a.rho = b->rho;
-    a.j = b->j;
-    a.nodes = b->nodes;
-    a.map = b->maps + in.map_off;
-    a.partials = b->part[0];
-    a.ctrl = b->ctrl + id;
-    a.dlx = in.dlx;
-    a.dly = in.dly;
-    a.lz = in.lz;
-    a.Np = b->Np;
-    a.fx = h.F[0];
-    a.fy = h.F[1];
-    a.fz = h.F[2];
-    a.lambda = in.lambda;
-    a.eps = eps;
-    a.tp = in.tp;
-    hipLaunchKernelGGL((k_mp_prep<1, W>), dim3(in.mp_ntiles), dim3(kBlock), 0, b->stream, a, in.mp_tile0);
-}
-
 // extract + MP layout + prep + VACF(0) of the instances ids, whose LB phases
-// have ended: launched for all of them, then read back at once
+// have ended: one launch of each for all of them (one per instance, a few
+// blocks at a time, took 50 ms for 1024 2-D instances)
 int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
     if (ids.empty()) return LBX_OK;
     LBX_TRY(build_tiles(b, ids));
     const double eps = DBL_EPSILON;
+    for (BInst& in : b->tab) in.lb_on = in.mp_on = 0;
     for (uint32_t id : ids) {
         HostInst& h = b->hi[id];
         BInst& in = b->tab[id];
-        const int64_t t = h.t;
-        const uint32_t gt = in.ntiles;
-        const uint32_t* map = b->maps + in.map_off;
-        if (t > 0) {
-            const int src = (t - 1) & 1, dst = t & 1;
-            if (shift(b)) {
-                const double* Ft = t > h.switch_step ? h.F : nullptr;
-                const double fm[3] = {Ft ? Ft[0] / 2.0 : 0.0, Ft ? Ft[1] / 2.0 : 0.0, Ft ? Ft[2] / 2.0 : 0.0};
-                hipLaunchKernelGGL(k_extract_shift, dim3(gt), dim3(kBlock), 0, b->stream, b->g[src], b->g[dst],
-                                   b->rho, b->j, b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end,
-                                   b->Np, in.rho0, fm[0], fm[1], fm[2]);
-            } else {
-                hipLaunchKernelGGL(k_extract, dim3(gt), dim3(kBlock), 0, b->stream, b->f[src], b->f[dst], b->rho,
-                                   b->nodes, map, in.dlx, in.dly, in.lz, in.node_off, in.node_end, b->Np);
-            }
-        }
         TracerParams tp{};
         const double K = (std::fabs(h.kd) <= eps) ? 0.0 : h.ka / h.kd;  // module_moment_propagation.f90:46-50
         tp.ads[0] = std::fabs(K) > eps;                                 // :52-56
@@ -895,15 +983,31 @@ int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
         in.tp = tp;
         in.any_ads = tp.ads[0];
         in.lambda = h.lambda;
-        LBX_TRY(reset_inst_ctrl(b, id, 2));
-        if (shift(b))
-            launch_mp_prep<float>(b, id, eps);
-        else
-            launch_mp_prep<double>(b, id, eps);
-        hipLaunchKernelGGL(k_mp_reduce<3>, dim3(1), dim3(kBlock), 0, b->stream,
-                           b->part[0] + 3 * (uint64_t)in.mp_tile0, in.mp_ntiles, nullptr, b->ctrl + id, 0,
-                           (int64_t)0, 0, 0.0, 0.0);
+        in.end_t = h.t;
+        for (int a = 0; a < 3; ++a) {
+            in.F[a] = h.F[a];
+            in.end_fm[a] = h.t > h.switch_step ? h.F[a] / 2.0 : 0.0;
+        }
+        in.lb_on = in.mp_on = 1;  // the tiles of both lists
     }
+    LBX_TRY(hipMemcpyAsync(b->insts, b->tab.data(), b->tab.size() * sizeof(BInst), hipMemcpyHostToDevice, b->stream));
+    LBX_TRY(hipMemcpyAsync(b->ids, ids.data(), ids.size() * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
+    LBX_TRY(upload_active(b));
+    const uint32_t n = (uint32_t)ids.size();
+    auto go = [&](auto wtag) {
+        using W = decltype(wtag);
+        const BatchMpView<W> v = mp_view<W>(b);
+        BatchView<W, W> lv = lb_view<W, W>(b);
+        hipLaunchKernelGGL(kb_extract<W>, dim3(b->n_act[0]), dim3(kBlock), 0, b->stream, lv, b->rho, b->j);
+        hipLaunchKernelGGL(kb_reset_ctrl, dim3((n + 63) / 64), dim3(64), 0, b->stream, b->ctrl, b->ids, n);
+        hipLaunchKernelGGL(kb_mp_prep<W>, dim3(b->n_act[1]), dim3(kBlock), 0, b->stream, v, b->rho, b->j, b->Np, eps);
+        hipLaunchKernelGGL(kb_mp_vacf0<W>, dim3(n), dim3(kBlock), 0, b->stream, v, b->ids);
+    };
+    if (shift(b))
+        go(float{});
+    else
+        go(double{});
+    for (BInst& in : b->tab) in.lb_on = in.mp_on = 0;
     LBX_TRY(hipGetLastError());
     std::vector<Ctrl> ctrl(b->cap_inst);
     LBX_TRY(download(b, b->ctrl, b->cap_inst, ctrl.data()));
@@ -1021,6 +1125,11 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
     if (!st) st = dalloc(&b->split, M / kTile);
     if (!st) st = dalloc(&b->builds, (uint64_t)max_instances);
     if (!st) st = dalloc(&b->built, (uint64_t)max_instances);
+    if (!st) st = dalloc(&b->ids, (uint64_t)max_instances);
+    for (int k = 0; k < 2; ++k) {
+        if (!st) st = hip_status(hipHostMalloc((void**)&b->stage[k], kStage));
+        if (!st) st = hip_status(hipEventCreateWithFlags(&b->stage_ev[k], hipEventDisableTiming));
+    }
     if (!st) st = dalloc(&b->vtrace, (uint64_t)kRoundMax * max_instances * 3);
     if (!st && (hipEventCreate(&b->ev[0]) != hipSuccess || hipEventCreate(&b->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
@@ -1072,6 +1181,7 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     HostInst h;
     std::vector<int8_t> itf(N);
     lbx_detect_interfacial(lx, ly, lz, nature, itf.data());
+    h.nodes_h.reserve(N);
     for (uint32_t r = 0; r < N; ++r)
         if (nature[r] == 0) {
             h.nodes_h.push_back(r | (itf[r] ? kNodeInterfacial : 0u));
@@ -1123,43 +1233,42 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     in.rho0 = rho0;
     in.target = target_error;
     in.floor_window = shift(b) ? b->floor_window : 0;
-    // nodes (global packed indices of the instance's fluid nodes) and its map
-    std::vector<uint32_t> gnodes(h.nodes_h);
-    std::vector<uint32_t> map(N, kSolidSlot);
+    // nodes (global packed indices of the instance's fluid nodes) and its map:
+    // through a pinned buffer where they fit, so that the call needs no wait
+    const size_t bytes = (h.Nf + (size_t)N) * sizeof(uint32_t);
+    const bool staged = bytes <= kStage;
+    const int at = b->stage_at;
+    std::vector<uint32_t> own(staged ? 0 : h.Nf + (size_t)N);
+    int st = staged ? hip_status(hipEventSynchronize(b->stage_ev[at])) : LBX_OK;
+    uint32_t* gnodes = staged ? (uint32_t*)b->stage[at] : own.data();
+    uint32_t* map = gnodes + h.Nf;
+    std::memcpy(gnodes, h.nodes_h.data(), h.Nf * sizeof(uint32_t));
+    std::fill(map, map + N, kSolidSlot);
     for (uint32_t i = 0; i < h.Nf; ++i) map[h.nodes_h[i] & kIndexMask] = in.node_off + i;
-    int st = hip_status(hipMemcpyAsync(b->nodes + in.node_off, gnodes.data(), h.Nf * sizeof(uint32_t),
-                                       hipMemcpyHostToDevice, b->stream));
-    if (!st) st = hip_status(hipMemcpyAsync(b->maps + map0, map.data(), N * sizeof(uint32_t), hipMemcpyHostToDevice,
+    if (!st) st = hip_status(hipMemcpyAsync(b->nodes + in.node_off, gnodes, h.Nf * sizeof(uint32_t),
+                                            hipMemcpyHostToDevice, b->stream));
+    if (!st) st = hip_status(hipMemcpyAsync(b->maps + map0, map, N * sizeof(uint32_t), hipMemcpyHostToDevice,
                                             b->stream));
     // rest state and the opening collision of step 1 (no force)
     if (!st) {
-        if (shift(b)) {
-            hipLaunchKernelGGL(k_init_rest, dim3(ntiles), dim3(kBlock), 0, b->stream, nullptr, b->g[0], b->j32,
-                               b->rho, b->j, in.node_off, in.node_end, b->Np, rho0);
-            if (b->prec == LBX_PREC_FP32_SHIFT)
-                hipLaunchKernelGGL(k_collide_packed_shift<float>, dim3(ntiles), dim3(kBlock), 0, b->stream, b->g[0],
-                                   b->rho, b->j, b->j32, 0.0f, 0.0f, 0.0f, in.node_off, in.node_end, b->Np,
-                                   (float)in.A, (float)in.B, (float)in.C, rho0);
-            else  // FP32-store: j_old is j itself
-                hipLaunchKernelGGL(k_collide_packed_shift<double>, dim3(ntiles), dim3(kBlock), 0, b->stream, b->g[0],
-                                   b->rho, b->j, b->j, 0.0, 0.0, 0.0, in.node_off, in.node_end, b->Np, in.A, in.B,
-                                   in.C, rho0);
-        } else {
-            hipLaunchKernelGGL(k_init_rest, dim3(ntiles), dim3(kBlock), 0, b->stream, b->f[0], nullptr, nullptr,
-                               b->rho, b->j, in.node_off, in.node_end, b->Np, rho0);
-            hipLaunchKernelGGL(k_collide_packed, dim3(ntiles), dim3(kBlock), 0, b->stream, b->f[0], b->rho, b->j,
-                               0.0, 0.0, 0.0, in.node_off, in.node_end, b->Np, in.A, in.B, in.C);
-        }
+        auto admit = [&](auto* f, auto* jold) {
+            using E = std::remove_pointer_t<decltype(f)>;
+            using R = std::remove_pointer_t<decltype(jold)>;
+            hipLaunchKernelGGL((kb_admit<E, R>), dim3(ntiles), dim3(kBlock), 0, b->stream, f, jold, b->rho, b->j, in, id,
+                               b->tile_inst, b->slots, b->l2ring, b->ctrl, b->Np);
+        };
+        if (b->prec == LBX_PREC_FP32_SHIFT)
+            admit(b->g[0], b->j32);
+        else if (b->prec == LBX_PREC_FP32_STORE)
+            admit(b->g[0], b->j);  // j_old is j itself
+        else
+            admit(b->f[0], b->j);
         st = hip_status(hipGetLastError());
     }
-    if (!st) st = reset_inst_ctrl(b, id, 2);
-    if (!st) st = hip_status(hipMemsetAsync(b->slots + (uint64_t)id * 3 * kSlots, 0,
-                                            3 * kSlots * sizeof(unsigned long long), b->stream));
-    if (!st) st = hip_status(hipMemsetAsync(b->l2ring + (uint64_t)id * kRing, 0, kRing * sizeof(double), b->stream));
+    if (!st && staged) st = hip_status(hipEventRecord(b->stage_ev[at], b->stream));
+    if (staged) b->stage_at ^= 1;
     for (uint64_t t = 0; t < ntiles; ++t) b->tile_inst_h[tile0 + t] = id;
-    if (!st) st = hip_status(hipMemcpyAsync(b->tile_inst + tile0, b->tile_inst_h.data() + tile0,
-                                            ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
-    if (!st) st = hip_status(hipStreamSynchronize(b->stream));
+    if (!st && !staged) st = hip_status(hipStreamSynchronize(b->stream));  // own is a local
     if (st) {
         for (uint64_t t = 0; t < ntiles; ++t) b->tile_inst_h[tile0 + t] = kNoInst;
         b->node_alloc.give(tile0, ntiles);

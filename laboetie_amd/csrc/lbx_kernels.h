@@ -487,15 +487,10 @@ __global__ __launch_bounds__(64) void k_lb_finalize(const unsigned long long* sl
 }
 
 // Streaming only: the post-streaming state f_s(t) of the step whose input is
-// fin, and its density SUM(n,4) (equilibration.f90:254).
-__global__ __launch_bounds__(kBlock) void k_extract(const double* __restrict__ fin, double* __restrict__ nout,
-                                                    double* __restrict__ rho_out, const uint32_t* __restrict__ nodes,
-                                                    const uint32_t* __restrict__ map, FastDiv dlx, FastDiv dly,
-                                                    uint32_t lz, uint32_t i0, uint32_t Nf, uint64_t Np) {
-    const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
-    if (i >= Nf) return;
-    Neighbours nb;
-    nb.load(map, nodes[i] & kIndexMask, dlx, dly, lz);
+// fin, and its density SUM(n,4) (equilibration.f90:254), of packed node i.
+__device__ __forceinline__ void extract_node(const double* __restrict__ fin, double* __restrict__ nout,
+                                             double* __restrict__ rho_out, const Neighbours& nb, uint32_t i,
+                                             uint64_t Np) {
     const View<true> fv(fin, kQ * Np);
     double rho = 0.0;
     static_for<0, kQ>([&](auto I) {
@@ -510,16 +505,10 @@ __global__ __launch_bounds__(kBlock) void k_extract(const double* __restrict__ f
 // The same for the FP32-shift form: the post-streaming deviations g into
 // gout, and the FP64 density rho0 + sum g and flux F/2 + sum g c, summed in
 // FP64 from the FP32 deviations (the flow that moment propagation reads).
-__global__ __launch_bounds__(kBlock) void k_extract_shift(const float* __restrict__ gin, float* __restrict__ gout,
-                                                          double* __restrict__ rho_out, double* __restrict__ j_out,
-                                                          const uint32_t* __restrict__ nodes,
-                                                          const uint32_t* __restrict__ map, FastDiv dlx, FastDiv dly,
-                                                          uint32_t lz, uint32_t i0, uint32_t Nf, uint64_t Np,
-                                                          double rho0, double fmx, double fmy, double fmz) {
-    const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
-    if (i >= Nf) return;
-    Neighbours nb;
-    nb.load(map, nodes[i] & kIndexMask, dlx, dly, lz);
+__device__ __forceinline__ void extract_node_shift(const float* __restrict__ gin, float* __restrict__ gout,
+                                                   double* __restrict__ rho_out, double* __restrict__ j_out,
+                                                   const Neighbours& nb, uint32_t i, uint64_t Np, double rho0,
+                                                   double fmx, double fmy, double fmz) {
     const View<true, float> gv(gin, kQ * Np);
     double drho = 0.0, jx = fmx, jy = fmy, jz = fmz;
     static_for<0, kQ>([&](auto I) {
@@ -536,6 +525,30 @@ __global__ __launch_bounds__(kBlock) void k_extract_shift(const float* __restric
     j_out[i] = jx;
     j_out[Np + i] = jy;
     j_out[2 * Np + i] = jz;
+}
+
+__global__ __launch_bounds__(kBlock) void k_extract(const double* __restrict__ fin, double* __restrict__ nout,
+                                                    double* __restrict__ rho_out, const uint32_t* __restrict__ nodes,
+                                                    const uint32_t* __restrict__ map, FastDiv dlx, FastDiv dly,
+                                                    uint32_t lz, uint32_t Nf, uint64_t Np) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= Nf) return;
+    Neighbours nb;
+    nb.load(map, nodes[i] & kIndexMask, dlx, dly, lz);
+    extract_node(fin, nout, rho_out, nb, i, Np);
+}
+
+__global__ __launch_bounds__(kBlock) void k_extract_shift(const float* __restrict__ gin, float* __restrict__ gout,
+                                                          double* __restrict__ rho_out, double* __restrict__ j_out,
+                                                          const uint32_t* __restrict__ nodes,
+                                                          const uint32_t* __restrict__ map, FastDiv dlx, FastDiv dly,
+                                                          uint32_t lz, uint32_t Nf, uint64_t Np, double rho0,
+                                                          double fmx, double fmy, double fmz) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= Nf) return;
+    Neighbours nb;
+    nb.load(map, nodes[i] & kIndexMask, dlx, dly, lz);
+    extract_node_shift(gin, gout, rho_out, j_out, nb, i, Np, rho0, fmx, fmy, fmz);
 }
 
 // The density SUM(n,4) (equilibration.f90:254) and flux F(t)/2 + sum n c
@@ -598,9 +611,9 @@ __global__ __launch_bounds__(kBlock) void k_flow_shift(const float* __restrict__
 // of a run), in place: module_collision.f90:87-108.
 __global__ __launch_bounds__(kBlock) void k_collide_packed(double* f, const double* __restrict__ rho,
                                                            const double* __restrict__ j, double fx, double fy,
-                                                           double fz, uint32_t i0, uint32_t Nf, uint64_t Np,
-                                                           double A, double B, double C) {
-    const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
+                                                           double fz, uint32_t Nf, uint64_t Np, double A, double B,
+                                                           double C) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= Nf) return;
     const double d = rho[i], jx = j[i], jy = j[Np + i], jz = j[2 * Np + i];
     const double ux = jx / d, uy = jy / d, uz = jz / d;
@@ -618,9 +631,9 @@ __global__ __launch_bounds__(kBlock) void k_collide_packed(double* f, const doub
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_collide_packed_shift(float* g, const double* __restrict__ rho,
                                                                  const double* j, R* jold, R fx, R fy, R fz,
-                                                                 uint32_t i0, uint32_t Nf, uint64_t Np, R A, R B,
-                                                                 R C, double rho0) {
-    const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
+                                                                 uint32_t Nf, uint64_t Np, R A, R B, R C,
+                                                                 double rho0) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= Nf) return;
     const R drho = (R)(rho[i] - rho0), full = (R)rho0 + drho;
     const R jx = (R)j[i], jy = (R)j[Np + i], jz = (R)j[2 * Np + i];
@@ -660,9 +673,9 @@ __global__ __launch_bounds__(kBlock) void k_collide_box(double* f, const double*
 // FP32-shift form (g != NULL) the deviations g = 0 and the FP32 flux j32 = 0.
 __global__ __launch_bounds__(kBlock) void k_init_rest(double* __restrict__ f, float* __restrict__ g,
                                                       float* __restrict__ j32, double* __restrict__ rho,
-                                                      double* __restrict__ j, uint32_t i0, uint32_t Nf, uint64_t Np,
+                                                      double* __restrict__ j, uint32_t Nf, uint64_t Np,
                                                       double rho0) {
-    const uint32_t i = i0 + blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= Nf) return;
     static_for<0, kQ>([&](auto I) {
         constexpr int L = I;

@@ -443,9 +443,8 @@ struct MpPrepArgs {
 // neighbours, the rest probability rem, u* = sum s c, and per tracer P(r,1)
 // and the VACF(0) contribution; Pa = 0.
 template <int T, typename W>
-__global__ __launch_bounds__(kBlock) void k_mp_prep(MpPrepArgs<W> a, uint32_t tile0) {
+__device__ __forceinline__ void mp_prep_tile(const MpPrepArgs<W>& a, uint32_t tile) {
     __shared__ double lds[kBlock / 64 * 3 * T];
-    const uint32_t tile = tile0 + xcd_tile();
     const uint32_t e = tile * kMpTile + threadIdx.x;
     double vp[3 * T];
 #pragma unroll
