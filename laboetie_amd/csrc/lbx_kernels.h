@@ -282,13 +282,18 @@ __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t t
         stop = ((int)(vload(&a.ctrl->stop) != 0) | (int)(vload(&a.ctrl->negpop) >= 0)) != 0;
         if (a.have_prev) prev = vload(a.slots + ((a.t - 1) % 3) * kSlots + (threadIdx.x & (kSlots - 1)));
     }
-    E early[TAB ? kQ : 1];  // TAB: the populations
+    E early[TAB ? kQ : 1];  // TAB: the populations and j_old
+    R jearly[3] = {R(0), R(0), R(0)};
     if constexpr (TAB)
         if (i < a.Nf) {
             const uint32_t Np = (uint32_t)a.Np;
             const View<Wide, E> fin(a.fin, kQ * a.Np);
             uint32_t src[kQ];
             static_for<1, kQ>([&](auto I) { src[I] = ld(a.pulls, (I - 1) * Np + i); });
+            if (a.write_l2 && is_check(a.t, a.check_base, a.check_every)) {
+                const View<Wide, R> jv(a.j, 3 * a.Np);
+                for (int c = 0; c < 3; ++c) jearly[c] = jv.ld(c * Np + i);
+            }
             early[0] = fin.ld(i);
             static_for<1, kQ>([&](auto I) { early[I] = fin.ld(src[I]); });
         }
@@ -361,8 +366,8 @@ __device__ __forceinline__ void lb_step_tile(const StepArgs<E, R>& a, uint32_t t
         // l2err of this step is measured: always in FP64; in the FP32 storage
         // forms only at the check steps, the only ones that read and keep j
         const bool chk = a.write_l2 && is_check(a.t, a.check_base, a.check_every);
-        R jo[3] = {R(0), R(0), R(0)};
-        if (chk) {  // j_old, issued before the populations so its latency overlaps theirs
+        R jo[3] = {jearly[0], jearly[1], jearly[2]};
+        if (!TAB && chk) {  // j_old, issued before the populations so its latency overlaps theirs
             jo[0] = jv.ld(i);
             jo[1] = jv.ld(Np + i);
             jo[2] = jv.ld(2 * Np + i);
