@@ -646,9 +646,9 @@ __global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void k_mp_step(MpStepArgs<W>
         mp_step_tile<T, W, RV, GEN>(a, xcd_tile() - 1);
 }
 
-// one k_mp_step launch
+// the arguments of step `it` (the chunk's k-th), whose input is buffer `now`
 template <typename W>
-void launch_mp_step(lbx_ctx* c, int now, int64_t it, int64_t k, int32_t stop_on_convergence, double lim1,
+MpStepArgs<W> mp_step_args(lbx_ctx* c, int now, int64_t it, int64_t k, int32_t stop_on_convergence, double lim1,
                            double lim2) {
     const uint32_t gt = c->mp_ntiles;
     const int nv = 3 * c->ntr;
@@ -672,13 +672,31 @@ void launch_mp_step(lbx_ctx* c, int now, int64_t it, int64_t k, int32_t stop_on_
     a.dlx = c->dlx;
     a.dly = c->dly;
     a.lz = c->lz;
+    return a;
+}
+
+// one k_mp_step launch
+template <typename W>
+void launch_mp_step(lbx_ctx* c, int now, int64_t it, int64_t k, int32_t stop_on_convergence, double lim1,
+                    double lim2) {
+    const MpStepArgs<W> a = mp_step_args<W>(c, now, it, k, stop_on_convergence, lim1, lim2);
     with_tracers(c->ntr, [&](auto TT) {
         constexpr int T = TT;
         const bool gen = c->mp_general || c->mp_divide;
         auto kern = a.rv ? (gen ? k_mp_step<T, W, true, true> : k_mp_step<T, W, true, false>)
-                           : (c->mp_general ? k_mp_step<T, W, false, true> : k_mp_step<T, W, false, false>);
-        hipLaunchKernelGGL(kern, dim3(gt + 1), dim3(kBlock), 0, c->stream, a);
+                         : (c->mp_general ? k_mp_step<T, W, false, true> : k_mp_step<T, W, false, false>);
+        hipLaunchKernelGGL(kern, dim3(c->mp_ntiles + 1), dim3(kBlock), 0, c->stream, a);
     });
+}
+
+// a chunk of S steps of a lattice of a few tiles: one launch of one block
+template <typename W>
+void launch_mp_run(lbx_ctx* c, int64_t S, int32_t stop_on_convergence, double lim1, double lim2) {
+    const MpFields<W>& f = mp_fields<W>(c);
+    const int n = c->mp_now;
+    hipLaunchKernelGGL(k_mp_run<W>, dim3(1), dim3(c->mp_ntiles * kMpTile), 0, c->stream,
+                       mp_step_args<W>(c, n, c->mp_it + 1, 0, stop_on_convergence, lim1, lim2), S, c->mp_ntiles,
+                       f.P[n], f.P[n ^ 1], f.Pa[n], f.Pa[n ^ 1], c->vtrace);
 }
 
 }  // namespace
@@ -1221,22 +1239,29 @@ static int mp_chunk_launch(lbx_ctx* c, int64_t S, int32_t stop, double* vt_h, Ct
     double lim1, lim2;
     mp_limits(c, &lim1, &lim2);
     timer_begin(c);
-    for (int64_t k = 0; k < S; ++k) {
-        const int now = c->mp_now ^ (int)(k & 1);
-        const int64_t it = c->mp_it + k + 1;
+    if (c->ntr == 1 && c->mp_ntiles <= kRunTiles) {
         if (f32_storage(c->prec))
-            launch_mp_step<float>(c, now, it, k, stop, lim1, lim2);
+            launch_mp_run<float>(c, S, stop, lim1, lim2);
         else
-            launch_mp_step<double>(c, now, it, k, stop, lim1, lim2);
-    }
-    timer_stop(c);
-    {  // the last step's VACF (and convergence test)
+            launch_mp_run<double>(c, S, stop, lim1, lim2);
+        timer_stop(c);
+    } else {
+        for (int64_t k = 0; k < S; ++k) {
+            const int now = c->mp_now ^ (int)(k & 1);
+            const int64_t it = c->mp_it + k + 1;
+            if (f32_storage(c->prec))
+                launch_mp_step<float>(c, now, it, k, stop, lim1, lim2);
+            else
+                launch_mp_step<double>(c, now, it, k, stop, lim1, lim2);
+        }
+        timer_stop(c);
+        // the last step's VACF (and convergence test)
         const int64_t it = c->mp_it + S;
         with_tracers(c->ntr, [&](auto TT) {
             constexpr int T = TT;
             hipLaunchKernelGGL(k_mp_reduce<3 * T>, dim3(1), dim3(kBlock), 0, c->stream,
-                               c->part + (uint64_t)nv * c->mp_ntiles * (it & 1), c->mp_ntiles, c->vtrace + nv * (S - 1),
-                               c->ctrl, 1, it, stop, lim1, lim2);
+                               c->part + (uint64_t)nv * c->mp_ntiles * (it & 1), c->mp_ntiles,
+                               c->vtrace + nv * (S - 1), c->ctrl, 1, it, stop, lim1, lim2);
         });
     }
     LBX_TRY(hipGetLastError());

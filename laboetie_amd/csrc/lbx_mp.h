@@ -803,6 +803,154 @@ __device__ __forceinline__ void mp_step_tile(const MpStepArgs<W>& a, uint32_t ti
     tile_partial<3 * T>(vp, a.partials + (uint64_t)(3 * T) * tile, (double*)smem);
 }
 
+// A whole chunk of steps of one tracer in one launch of one block, for a
+// lattice of at most kRunTiles tiles: P stays in LDS, the probabilities, Pa and
+// everything else of a node in its thread's registers, and a step costs two
+// barriers in place of a launch.  The sums are those of mp_step_tile,
+// tile_partial and mp_reduce_block in their order, so the bits are the same.
+// us per step launched / here: 60 nodes 3.6 / 1.5, 512 (a 4x4x34 slit) 3.8 / 1.7,
+// 768 (three tiles) 3.7 / 1.75, 1024 (four, all a block's threads) 3.8 / 2.0.
+constexpr uint32_t kRunTiles = 4;
+
+// lane k of wave 0 holds component k of the running sums
+template <typename W>
+__global__ __launch_bounds__(1024) void k_mp_run(MpStepArgs<W> a, int64_t S, uint32_t ntiles, double* P0, double* P1,
+                                                 double* Pa0, double* Pa1, double* vtrace) {
+    constexpr uint32_t E = kRunTiles * kMpTile, kNone = E;  // kNone: a solid neighbour's slot
+    __shared__ Vec2<double> pA[E + 1];
+    __shared__ double pB[E + 1];
+    __shared__ double vs[3 * E];              // P . u* by component and entry
+    __shared__ double part[3 * kRunTiles];    // tile sums
+    __shared__ int32_t stop;
+    if (block_flag(vload(&a.ctrl->mp_stop) != 0)) return;
+    const uint32_t e = threadIdx.x, lane = e & 63u, wave = e >> 6, nwaves = blockDim.x >> 6;
+    const bool valid = e % kMpTile < a.t.info[e / kMpTile];
+    uint16_t slot[kQ];
+    double w[kQ], p[3] = {0.0, 0.0, 0.0}, pa[3] = {0.0, 0.0, 0.0}, rm = 0.0;
+    W us[3] = {W(0), W(0), W(0)};
+    bool ads = false;
+    if (valid) {
+        const uint32_t word = a.nodes[a.t.perm[e]];
+        Neighbours nb;
+        nb.load(a.map, word & kIndexMask, a.dlx, a.dly, a.lz);
+        static_for<1, kQ>([&](auto I) {
+            constexpr int L = I;
+            slot[L] = (uint16_t)kNone;
+            w[L] = 0.0;
+            if (nb.q[L] != kSolidSlot) {
+                const uint32_t q = a.t.inv[nb.q[L]];
+                slot[L] = (uint16_t)q;
+                if (a.rv) {
+                    const Vec2<double> r0 = a.rv[rv_index(q)], r1 = a.rv[rv_index(q) + 1];
+                    w[L] = scatter_prob<kInv[L], W>(r0[0], r0[1], r1[0], r1[1], a.lambda);
+                } else {
+                    w[L] = (double)a.win[win_index(e, (L - 1) / 2)][(L - 1) & 1];
+                }
+            }
+        });
+        Trio<double>::load(a.Pn, e, 1, 0, p);
+        rm = a.rem[e];
+        Trio<W>::load(a.ustar, e, 1, 0, us);
+        ads = a.any_ads && (word & kNodeInterfacial) != 0;
+        if (ads) Trio<double>::load(a.Pan, e, 1, 0, pa);
+        pA[e] = Vec2<double>{p[0], p[1]};
+        pB[e] = p[2];
+    }
+    const double ka = a.tp.ka[0], kd = a.tp.kd[0], keep = a.tp.one_minus_kd[0];
+    double run_s = 0.0, run_c = 0.0;
+    if (e < 3) {
+        run_s = a.ctrl->deff_s[e];
+        run_c = a.ctrl->deff_c[e];
+    }
+    if (e == 0) {
+        pA[kNone] = Vec2<double>{0.0, 0.0};
+        pB[kNone] = 0.0;
+        stop = 0;
+    }
+    // VACF of the chunk's step k from the tile sums (wave 0), and the convergence test
+    const auto reduce = [&](int64_t k) {
+        double s[3];
+        for (int c = 0; c < 3; ++c) s[c] = lane < ntiles ? part[3 * lane + c] : 0.0;
+        wave_sums<3>(s);
+        bool below = true;
+        if (lane < 3) {
+            const double t = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
+            vtrace[3 * k + lane] = t;
+            const double u = run_s + t;
+            run_c = run_c + ((fabs(run_s) >= fabs(t)) ? (run_s - u) + t : (t - u) + run_s);
+            run_s = u;
+            below = fabs(t) < a.lim1 && fabs(t) < a.lim2;
+        }
+        return a.check_conv && a.it + k > 2 && __all(below);
+    };
+    __syncthreads();
+    int64_t ran = 0;
+    bool conv = false;
+    for (int64_t k = 0; k < S; ++k) {
+        if (k > 0 && wave == 0) {
+            const bool c = reduce(k - 1);
+            if (lane == 0 && c) stop = 1;
+        }
+        double px[3] = {0.0, 0.0, 0.0}, vp[3] = {0.0, 0.0, 0.0};
+        if (valid) {
+            double acc[3] = {0.0, 0.0, 0.0};
+            static_for<1, kQ>([&](auto I) {
+                constexpr int L = I;
+                if constexpr (L % kPace == 0) __builtin_amdgcn_sched_barrier(0);
+                const Vec2<double> x = pA[slot[L]];
+                const double y = pB[slot[L]];
+                acc[0] = acc[0] + x[0] * w[L];
+                acc[1] = acc[1] + x[1] * w[L];
+                acc[2] = acc[2] + y * w[L];
+            });
+            for (int c = 0; c < 3; ++c) {
+                vp[c] = p[c] * (double)us[c];
+                px[c] = acc[c] + rm * p[c];
+                if (ads) px[c] = (acc[c] + (rm - ka) * p[c]) + pa[c] * kd;
+            }
+        }
+        for (int c = 0; c < 3; ++c) vs[c * E + e] = vp[c];
+        __syncthreads();  // every read of P and of the tile sums is over
+        conv = stop != 0;
+        if (conv) break;
+        if (valid) {
+            pA[e] = Vec2<double>{px[0], px[1]};
+            pB[e] = px[2];
+            for (int c = 0; c < 3; ++c) {
+                if (ads) pa[c] = pa[c] * keep + p[c] * ka;
+                p[c] = px[c];
+            }
+        }
+        // tile_partial's sums, one (tile, component) a wave
+        for (uint32_t q = wave; q < 3 * ntiles; q += nwaves) {
+            const double* v = vs + (q % 3) * E + (q / 3) * kMpTile + lane;
+            double s = v[0];
+            for (int x = 1; x < 4; ++x) s = s + v[64 * x];
+            s = wave_sum(s);
+            if (lane == 0) part[q] = s;
+        }
+        ran = k + 1;
+        __syncthreads();
+    }
+    if (!conv && wave == 0) {
+        const bool c = reduce(S - 1);
+        if (lane == 0 && c) stop = 1;
+    }
+    if (e < 3) {
+        a.ctrl->deff_s[e] = run_s;
+        a.ctrl->deff_c[e] = run_c;
+    }
+    if (e == 0 && stop) {
+        a.ctrl->mp_conv_step = a.it + ran - 1;
+        a.ctrl->mp_stop = 1;
+    }
+    if (valid) {  // the buffer that `ran` launched steps would have left
+        const bool other = (ran & 1) != 0;
+        Trio<double>::store(other ? P1 : P0, e, 1, 0, p);
+        if (ads) Trio<double>::store(other ? Pa1 : Pa0, e, 1, 0, pa);
+    }
+}
+
 // P or Pa of tracer t of T into the full box, (3, box nodes): the nodes with
 // box index in [r0, r0 + n)
 __global__ __launch_bounds__(kBlock) void k_mp_box(const double* __restrict__ p, MpTiles t, uint32_t tile0,
