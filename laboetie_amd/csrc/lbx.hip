@@ -296,8 +296,8 @@ void timer_end(lbx_ctx* c, int which, int64_t launches) {
 // Up to this many fluid nodes the LB step takes its pull sources from a table
 // (StepArgs::pulls, 72 bytes a node): while everything a step reads sits in L2
 // its time is the chain of round trips, not the bytes.  us per step without /
-// with it, FP64, FP32-shift, FP32-store: 2 185 nodes 5.88 / 5.54, 5.79 / 5.36,
-// 5.83 / 5.37; 85 056 nodes 9.14 / 8.90, 7.53 / 6.80, 7.71 / 7.11.  Asking for
+// with it, FP64, FP32-shift, FP32-store: 2 185 nodes 5.88 / 5.26, 5.79 / 5.13,
+// 5.83 / 5.31; 85 056 nodes 9.14 / 8.77, 7.53 / 6.82, 7.71 / 7.19.  Asking for
 // the flags late without the table lost at 128^3 and above (registers).
 constexpr uint32_t kTabNodes = 131072;
 
@@ -379,6 +379,25 @@ void launch_lb_step(lbx_ctx* c, int64_t t, const double fm[3], const double fc[3
                                : (c->nt ? k_lb_step<false, double, double, true> : k_lb_step<false, double>);
         hipLaunchKernelGGL(kern, dim3(gt), dim3(kBlock), 0, c->stream, a);
     }
+}
+
+// steps t0+1 .. t0+S of a lattice of a few nodes in one launch
+void launch_lb_run(lbx_ctx* c, int64_t t0, int64_t S, const double F[3], int64_t check_after, double target,
+                   int32_t check_every, int64_t check_base) {
+    auto go = [&](auto a, auto kern, auto* f0, auto* f1) {
+        a.t = t0;
+        const uint32_t threads = (c->Nf + 63u) / 64u * 64u;
+        hipLaunchKernelGGL(kern, dim3(1), dim3(threads), 0, c->stream, a, f0, f1, S);
+    };
+    if (c->prec == LBX_PREC_FP32_SHIFT)
+        go(step_args<float>(c, t0 + 1, F, F, check_after, target, 1, check_every, check_base), k_lb_run<float, float>,
+           c->g[0], c->g[1]);
+    else if (c->prec == LBX_PREC_FP32_STORE)
+        go(step_args<float, double>(c, t0 + 1, F, F, check_after, target, 1, check_every, check_base),
+           k_lb_run<float, double>, c->g[0], c->g[1]);
+    else
+        go(step_args<double>(c, t0 + 1, F, F, check_after, target, 1, check_every, check_base),
+           k_lb_run<double, double>, c->f[0], c->f[1]);
 }
 
 // ---- full-box host arrays <-> packed device planes
@@ -1022,8 +1041,11 @@ int lbx_equilibrate_advance(lbx_ctx* c, int64_t until_step, int64_t* steps_done,
         const int64_t base = q.stage == 1 ? 0 : q.switch_step;
         const int64_t t = q.t;
         timer_begin(c);
-        for (int64_t k = 1; k <= S; ++k)
-            launch_lb_step(c, t + k, Fs, Fs, q.check_after, q.target, 1, t + k > 1, every, base);
+        if (c->pulls && c->Nf <= kRunNodes && !c->wide && !q.flux_sums)
+            launch_lb_run(c, t, S, Fs, q.check_after, q.target, every, base);
+        else
+            for (int64_t k = 1; k <= S; ++k)
+                launch_lb_step(c, t + k, Fs, Fs, q.check_after, q.target, 1, t + k > 1, every, base);
         timer_stop(c);
         hipLaunchKernelGGL(k_lb_finalize, dim3(1), dim3(kSlots), 0, c->stream, c->slots, c->l2ring, c->ctrl, t + S,
                            base, every);

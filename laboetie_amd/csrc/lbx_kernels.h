@@ -491,6 +491,170 @@ __global__ __launch_bounds__(64) void k_lb_finalize(const unsigned long long* sl
     lb_finalize(slots, l2ring, ctrl, t, check_base, check_every);
 }
 
+// A whole launch run of steps t0+1 .. t0+S (a.t = t0) in one launch of one
+// block, for a lattice of at most kRunNodes nodes: one node a thread, the
+// post-collision populations in LDS and j_old in registers, two barriers a
+// step in place of a launch.  The last step's two population sets, the flags,
+// l2err record and slots are left as the launches leave them; arithmetic and
+// verdicts are lb_step_tile's.  One CU does the work of all, so it pays while
+// few waves share its SIMDs: us per step launched / here, FP64 and FP32-shift,
+// 60 nodes 4.8 / 1.5 and 4.7 / 1.5, 256 nodes 5.1 / 1.9 and 4.8 / 1.8, 512 nodes
+// 5.3 / 3.1 and 5.2 / 2.8; a second node a thread would double the last.
+constexpr uint32_t kRunNodes = 512;
+
+template <typename E, typename R>
+__global__ __launch_bounds__(kRunNodes) void k_lb_run(StepArgs<E, R> a, E* f0, E* f1, int64_t S) {
+    constexpr bool kShift = std::is_same<E, float>::value;
+    __shared__ E pop[kQ * kRunNodes];
+    __shared__ double red[kRunNodes / 64];
+    __shared__ unsigned long long first_bits;
+    const uint32_t i = threadIdx.x, Np = (uint32_t)a.Np, nwaves = blockDim.x >> 6;
+    const bool valid = i < a.Nf, first = i == 0;
+    const int64_t t0 = a.t;
+    if (block_flag((int)(vload(&a.ctrl->stop) != 0) | (int)(vload(&a.ctrl->negpop) >= 0))) return;
+    // the record of the stage up to step t0 - 1, in every thread
+    double lmin = a.ctrl->l2min[(t0 - 1) & 1], lmax = a.ctrl->l2max[(t0 - 1) & 1];
+    int64_t lstep = a.ctrl->l2min_step[(t0 - 1) & 1];
+    // the verdicts on step t, which step t+1 takes in lb_step_tile: true ends the run
+    const auto ends = [&](int64_t t, unsigned long long bits) {
+        if (bits == kNegMark) {
+            if (first) a.ctrl->negpop = t;
+            return true;
+        }
+        const bool chk = is_check(t, a.check_base, a.check_every);
+        const double prev = chk ? __longlong_as_double((long long)bits) : __builtin_nan("");
+        if (first) a.l2ring[t % kRing] = prev;
+        bool floor = false;
+        if (a.floor_window > 0 && t > a.check_after) {
+            if (chk) {
+                if (prev < lmin) {
+                    lmin = prev;
+                    lstep = t;
+                }
+                lmax = fmax(lmax, prev);
+            }
+            floor = chk && t - lstep >= a.floor_window && lmin <= kFloorDrop * lmax;
+        }
+        if (!(chk && t > a.check_after && (prev <= a.target || floor))) return false;
+        if (first) {
+            a.ctrl->exit_step = t;
+            a.ctrl->floor_hit = prev <= a.target ? 0 : 1;
+            a.ctrl->stop = 1;
+        }
+        return true;
+    };
+    if (t0 > 0) {
+        if (i < 64) {
+            const unsigned long long v = slots_max(a.slots + (t0 % 3) * kSlots);
+            if (first) first_bits = v;
+        }
+        __syncthreads();
+        if (ends(t0, first_bits)) return;
+    }
+    uint16_t src[kQ];
+    R jo[3] = {R(0), R(0), R(0)};
+    if (valid) {
+        const E* fin = t0 & 1 ? f1 : f0;
+        src[0] = (uint16_t)i;
+        static_for<1, kQ>([&](auto I) {
+            const uint32_t v = a.pulls[(uint64_t)(I - 1) * Np + i];
+            src[I] = (uint16_t)(v / Np * kRunNodes + v % Np);
+        });
+        static_for<0, kQ>([&](auto I) { pop[I * kRunNodes + i] = fin[(uint64_t)I * Np + i]; });
+        for (int c = 0; c < 3; ++c) jo[c] = a.j[c * (uint64_t)Np + i];
+    }
+    __syncthreads();
+    for (int64_t t = t0 + 1;; ++t) {
+        const bool chk = is_check(t, a.check_base, a.check_every);
+        double l2 = 0.0;
+        bool neg = false;
+        E out[kQ];
+        if (valid) {
+            R f[kQ];
+            static_for<0, kQ>([&](auto I) { f[I] = (R)pop[src[I]]; });
+            if constexpr (kShift)
+                static_for<0, kQ>([&](auto I) { neg = neg || (f[I] < -((R)a0(I) * a.rho0)); });
+            else
+                static_for<0, kQ>([&](auto I) { neg = neg || (f[I] < 0.0); });
+            R rho = f[0];
+            static_for<1, kQ>([&](auto I) { rho = rho + f[I]; });
+            R jx = a.fmx, jy = a.fmy, jz = a.fmz;
+            static_for<0, kQ>([&](auto I) {
+                constexpr int L = I;
+                if constexpr (kCX[L] != 0) jx = jx + sgn<kCX[L]>(f[L]);
+                if constexpr (kCY[L] != 0) jy = jy + sgn<kCY[L]>(f[L]);
+                if constexpr (kCZ[L] != 0) jz = jz + sgn<kCZ[L]>(f[L]);
+            });
+            if (chk) {
+                R dx = fabs(jx - jo[0]), dy = fabs(jy - jo[1]), dz = fabs(jz - jo[2]);
+                if constexpr (kShift) {
+                    dx = dx * a.check_inv;
+                    dy = dy * a.check_inv;
+                    dz = dz * a.check_inv;
+                }
+                l2 = (double)fmax(fmax(dx, dy), dz);
+            }
+            if (!kShift || chk) {
+                jo[0] = jx;
+                jo[1] = jy;
+                jo[2] = jz;
+            }
+            if constexpr (kShift) {
+                const R drho = rho, full = a.rho0 + drho;
+                R ux, uy, uz;
+                shift_velocity<R>(jx, jy, jz, full, ux, uy, uz);
+                static_for<0, kQ>([&](auto I) {
+                    constexpr int L = I;
+                    out[L] = (E)collide_shift<L, R>(f[L], drho, jx, jy, jz, ux, uy, uz, a.fcx, a.fcy, a.fcz, a.A, a.B,
+                                                    a.C);
+                });
+            } else {
+                const double ux = jx / rho, uy = jy / rho, uz = jz / rho;
+                static_for<0, kQ>([&](auto I) {
+                    constexpr int L = I;
+                    out[L] = collide_pop<L>(f[L], rho, jx, jy, jz, ux, uy, uz, a.fcx, a.fcy, a.fcz, a.A, a.B, a.C);
+                });
+            }
+        }
+        l2 = wave_max(l2);
+        const bool wneg = __ballot(neg) != 0ull;
+        if ((i & 63u) == 0) red[i >> 6] = wneg ? -1.0 : l2;
+        __syncthreads();  // every read of the populations is over
+        double m = red[0];
+        bool bneg = m < 0.0;
+        for (uint32_t w = 1; w < nwaves; ++w) {
+            bneg = bneg || red[w] < 0.0;
+            m = fmax(m, red[w]);
+        }
+        const unsigned long long bits =
+            bneg ? kNegMark : (m > 0.0 ? (unsigned long long)__double_as_longlong(m) : 0ull);
+        if (t == t0 + S || ends(t, bits)) {
+            if (valid) {
+                E *fin = t & 1 ? f0 : f1, *fout = t & 1 ? f1 : f0;
+                static_for<0, kQ>([&](auto I) {
+                    fin[(uint64_t)I * Np + i] = pop[I * kRunNodes + i];
+                    fout[(uint64_t)I * Np + i] = out[I];
+                });
+                for (int c = 0; c < 3; ++c) a.j[c * (uint64_t)Np + i] = jo[c];
+            }
+            if (i < kSlots) {
+                a.slots[(t % 3) * kSlots + i] = i == 0 ? bits : 0ull;
+                a.slots[((t + 1) % 3) * kSlots + i] = 0ull;
+            }
+            break;
+        }
+        if (valid) static_for<0, kQ>([&](auto I) { pop[I * kRunNodes + i] = out[I]; });
+        __syncthreads();
+    }
+    if (first) {
+        for (int k = 0; k < 2; ++k) {
+            a.ctrl->l2min[k] = lmin;
+            a.ctrl->l2min_step[k] = lstep;
+            a.ctrl->l2max[k] = lmax;
+        }
+    }
+}
+
 // Streaming only: the post-streaming state f_s(t) of the step whose input is
 // fin, and its density SUM(n,4) (equilibration.f90:254), of packed node i.
 __device__ __forceinline__ void extract_node(const double* __restrict__ fin, double* __restrict__ nout,

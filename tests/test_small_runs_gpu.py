@@ -1,6 +1,8 @@
-"""Lattices small enough that one block takes a whole chunk of MP steps: the
-same bits as one launch a step, which a pair of equal tracers still takes.
-Node counts around the edges of waves, tiles and the rule."""
+"""Lattices small enough that one block takes a whole run of steps: the same
+bits as one launch a step, which a run with flux sums (LB) and a pair of equal
+tracers (MP) still take.  Node counts around the edges of waves, tiles and the
+rule; runs paused at odd steps, stopped by the target, by the floor of l2err,
+by a negative population and by the cap."""
 import numpy as np
 import pytest
 
@@ -18,6 +20,45 @@ def lattice(nf):
     nat = np.ones(int(np.prod(dims)), np.int8)
     nat[np.random.default_rng(nf).permutation(nat.size)[:nf]] = 0
     return dims, nat
+
+
+def lb_run(L, launched, fext, target, cap, pauses):
+    L.init_rest(1.0)
+    L.equilibrate_begin(fext, target, max_steps=cap, flux_sums=launched)
+    for t in pauses:
+        r = L.equilibrate_advance(t, check=False)
+        if r["status"] or r["exit_reason"]:
+            break
+        flow = L.flow()
+    else:
+        r = L.equilibrate_advance(check=False)
+        flow = L.flow()
+    out = [np.array([r["status"], r["steps"], r["exit_reason"]]), L.l2err_trace()]
+    if r["status"] == lbx.OK:
+        out += [*flow, *L.get_state()]
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", PRECS)
+@pytest.mark.parametrize("nf", [1, 63, 64, 65, 257, 511, 512])
+def test_lb_run_in_one_block(nf, prec):
+    dims, nat = lattice(nf)
+    print("lb run", nf, prec, flush=True)
+    fext = [1e-4, -2e-4, 3e-4]
+    with lbx.Lattice(dims, nat, 0.8, precision=prec) as L:
+        for what, f, target, cap, pauses, window, every in [
+                ("capped", fext, 0.0, 70, (1, 2, 4, 9, 10, 41), 0, 1),
+                ("target", fext, 1e-7, 4000, (5, 77), 0, 4),
+                ("floor", fext, 0.0, 6000, (), 40, 1),
+                ("negative", [0.9, 0.0, 0.0], 0.0, 400, (3,), 0, 1)]:
+            if prec != lbx.PREC_FP64:  # FP64 measures l2err at every step and has no floor
+                L.set_floor_window(window)
+                L.set_check_interval(every)
+            a, b = (lb_run(L, launched, f, target, cap, pauses) for launched in (False, True))
+            assert len(a) == len(b), (what, a[0], b[0])
+            for x, y in zip(a, b):
+                assert np.array_equal(x, y, equal_nan=True), (what, a[0], b[0])
 
 
 @pytest.mark.gpu
