@@ -34,6 +34,7 @@
 #include "lbx_device.h"
 #include "lbx_kernels.h"
 #include "lbx_mp.h"
+#include "lbx_nodes.h"
 #include "lbx_tables.h"
 
 #pragma clang fp contract(off)
@@ -92,7 +93,7 @@ struct lbx_ctx {
     Ctrl ctrl_h{};               // host copy that reset_ctrl uploads from (read by the stream's next copy)
     double* l2ring = nullptr;
     int pre = 0;                 // buffer holding the post-streaming state
-    std::vector<uint32_t> nodes_h;
+    uint32_t first_node = 0;  // box index of the first fluid node
     // moment propagation
     bool mp_ready = false;
     MpTiles mpt;                 // the geometry's tiles (built by the first MP set-up, kept)
@@ -398,6 +399,48 @@ void launch_lb_run(lbx_ctx* c, int64_t t0, int64_t S, const double F[3], int64_t
     else
         go(step_args<double>(c, t0 + 1, F, F, check_after, target, 1, check_every, check_base),
            k_lb_run<double, double>, c->f[0], c->f[1]);
+}
+
+__global__ __launch_bounds__(kNodeThreads) void k_nodes(const int8_t* __restrict__ nature, uint32_t N,
+                                                        const uint32_t* __restrict__ counts, uint32_t* nodes,
+                                                        uint32_t* map, uint32_t* nfi, FastDiv dlx, FastDiv dly,
+                                                        uint32_t lz) {
+    node_chunk(nature, N, counts, blockIdx.x, 0, nodes, map, nfi, dlx, dly, lz);
+}
+
+// Node list and map of a new context; *nfi holds the interfacial nodes once the
+// stream has synchronised.  The nature and the counts lie in a population set,
+// which holds nothing yet, or, where that is too small (a box of nearly no
+// fluid), in memory of their own.
+int build_nodes(lbx_ctx* c, const int8_t* nature, uint32_t* nfi) {
+    const uint64_t nat = ((uint64_t)c->N + 255) / 256 * 256;
+    const uint32_t chunks = node_chunks(c->N);
+    const uint64_t need = nat + (chunks + 1) * sizeof(uint32_t);
+    const bool shift = f32_storage(c->prec);
+    char* own = nullptr;
+    char* at = shift ? (char*)c->g[1] : (char*)c->f[1];
+    if (kQ * c->Np * (shift ? sizeof(float) : sizeof(double)) < need) {
+        LBX_TRY(dalloc(&own, need));
+        at = own;
+    }
+    int8_t* nd = (int8_t*)at;
+    uint32_t *counts = (uint32_t*)(at + nat), *total = counts + chunks;
+    int st = hip_status(hipMemcpyAsync(nd, nature, c->N, hipMemcpyHostToDevice, c->stream));
+    if (!st) st = hip_status(hipMemsetAsync(total, 0, sizeof(uint32_t), c->stream));
+    if (!st) {
+        if (chunks > kNodeCountChunks)
+            hipLaunchKernelGGL(k_node_count, dim3(chunks), dim3(kNodeThreads), 0, c->stream, nd, c->N, counts);
+        hipLaunchKernelGGL(k_nodes, dim3(chunks), dim3(kNodeThreads), 0, c->stream, nd, c->N,
+                           chunks > kNodeCountChunks ? counts : nullptr, c->nodes, c->map, total, c->dlx, c->dly,
+                           c->lz);
+        st = hip_status(hipGetLastError());
+    }
+    if (!st) st = hip_status(hipMemcpyAsync(nfi, total, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    if (own) {
+        if (!st) st = hip_status(hipStreamSynchronize(c->stream));
+        dfree(own);
+    }
+    return st;
 }
 
 // ---- full-box host arrays <-> packed device planes
@@ -800,20 +843,12 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     relaxation_coeffs(tau, &c->A, &c->B, &c->C);
     fp32_relaxation(tau, &c->A32, &c->B32);
     (void)hipGetDevice(&c->device);
-    std::vector<int8_t> itf(c->N);
-    lbx_detect_interfacial(lx, ly, lz, nature, itf.data());
-    std::vector<uint32_t> map(c->N, kSolidSlot);
-    for (uint32_t r = 0; r < c->N; ++r)
-        if (nature[r] == 0) {
-            map[r] = (uint32_t)c->nodes_h.size();
-            c->nodes_h.push_back(r | (itf[r] ? kNodeInterfacial : 0u));
-            c->nfi += itf[r] != 0;
-        }
-    c->Nf = (uint32_t)c->nodes_h.size();
+    c->Nf = count_fluid(nature, c->N);
     if (c->Nf == 0) {
         delete c;
         return LBX_ERR_ARG;
     }
+    c->first_node = (uint32_t)((const int8_t*)std::memchr(nature, 0, c->N) - nature);
     c->Np = ((uint64_t)c->Nf + 63) / 64 * 64;
     // element indices of the population set (19*Np) are 32-bit
     if (kQ * c->Np >= (1ull << 32)) {
@@ -844,10 +879,8 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     if (!st) st = dalloc(&c->l2ring, kRing);
     if (!st && (hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
-    if (!st) st = hip_status(hipMemcpyAsync(c->nodes, c->nodes_h.data(), c->Nf * sizeof(uint32_t),
-                                            hipMemcpyHostToDevice, c->stream));
-    if (!st) st = hip_status(hipMemcpyAsync(c->map, map.data(), c->N * sizeof(uint32_t), hipMemcpyHostToDevice,
-                                            c->stream));
+    uint32_t nfi = 0;
+    if (!st) st = build_nodes(c, nature, &nfi);
     if (!st && c->pulls) {
         hipLaunchKernelGGL(k_pull_table, dim3(c->ntiles), dim3(kBlock), 0, c->stream, c->pulls, c->nodes, c->map, c->dlx,
                            c->dly, c->lz, c->Nf, (uint32_t)c->Np);
@@ -867,6 +900,7 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
         delete c;
         return st;
     }
+    c->nfi = nfi;
     c->l2host.resize(kRing);
     *out = c;
     return LBX_OK;
@@ -898,7 +932,7 @@ int lbx_set_state(lbx_ctx* c, const double* n, const double* rho, const double* 
     if (f32_storage(c->prec)) {
         // the rest density of the deviations: the density of the first fluid
         // node (the uniform rest density when the state is a rest state)
-        c->rho0 = rho[c->nodes_h[0] & kIndexMask];
+        c->rho0 = rho[c->first_node];
         LBX_TRY(upload_shift(c, n, c->g[0]));
     } else {
         const double* planes[kQ];

@@ -39,6 +39,7 @@
 #include "lbx_device.h"
 #include "lbx_kernels.h"
 #include "lbx_mp.h"
+#include "lbx_nodes.h"
 #include "lbx_tables.h"
 
 #pragma clang fp contract(off)
@@ -261,7 +262,15 @@ template <typename E, typename R>
 __global__ __launch_bounds__(kBlock) void kb_admit(E* f, R* jold, double* __restrict__ rho, double* __restrict__ j,
                                                    BInst in, uint32_t id, uint32_t* __restrict__ tile_inst,
                                                    unsigned long long* __restrict__ slots, double* __restrict__ l2ring,
-                                                   Ctrl* ctrl, uint64_t Np) {
+                                                   Ctrl* ctrl, uint64_t Np, const int8_t* __restrict__ nature,
+                                                   uint32_t N, const uint32_t* __restrict__ counts,
+                                                   uint32_t* __restrict__ nodes, uint32_t* __restrict__ maps,
+                                                   uint32_t* nfi) {
+    static_assert(kBlock == kNodeThreads, "one block size");
+    if (blockIdx.x * kNodeChunk < N)
+        node_chunk(nature, N, counts, blockIdx.x, in.node_off, nodes, maps + in.map_off, nfi + id, in.dlx, in.dly,
+                   in.lz);
+    if (blockIdx.x >= in.ntiles) return;
     if (threadIdx.x == 0) tile_inst[in.tile_first + blockIdx.x] = id;
     if (blockIdx.x == 0) {
         for (uint32_t k = threadIdx.x; k < 3 * kSlots; k += kBlock) slots[(uint64_t)id * 3 * kSlots + k] = 0ull;
@@ -289,6 +298,20 @@ __global__ __launch_bounds__(kBlock) void kb_admit(E* f, R* jold, double* __rest
             f[(uint64_t)L * Np + i] = collide_pop<L>(d * a0(L), d, 0.0, 0.0, 0.0, u, u, u, 0.0, 0.0, 0.0, A, B, C);
         }
     });
+}
+
+// A removed instance's tiles and interfacial count.
+__global__ __launch_bounds__(kBlock) void kb_release(uint32_t* __restrict__ tile_inst, uint32_t n, uint32_t* nfi) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) tile_inst[i] = kNoInst;
+    if (i == 0) *nfi = 0;
+}
+
+// out[k] = l2ring[at[k]]
+__global__ __launch_bounds__(kBlock) void kb_pick_l2(const double* __restrict__ l2ring, const uint64_t* __restrict__ at,
+                                                     uint32_t n, double* __restrict__ out) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < n) out[k] = l2ring[at[k]];
 }
 
 // The post-streaming state, density and flux at the end of the LB phase of
@@ -481,10 +504,8 @@ struct HostInst {
     int64_t t = 0, max_lb = 0, switch_step = INT64_MAX, check_after = 2;
     int64_t mp_it = 0, mp_target = 0;
     bool general = false;           // its MP steps need the general kernel (lbx_mp.h)
-    std::vector<uint32_t> nodes_h;  // full-box index | interfacial bit
     std::vector<double> vacf;       // (mp_it+1) x 3
     double deff[3] = {0, 0, 0};
-    int64_t nfi = 0;
 };
 
 }  // namespace
@@ -513,6 +534,9 @@ struct lbxb {
     uint32_t* nodes = nullptr;
     uint32_t* maps = nullptr;
     uint32_t* tile_inst = nullptr;
+    int8_t* nature = nullptr;    // of the instance being admitted
+    uint32_t* counts = nullptr;  // its fluid nodes by chunk (lbx_nodes.h)
+    uint32_t* nfi = nullptr;     // interfacial nodes of each instance
     BInst* insts = nullptr;
     unsigned long long* slots = nullptr;
     double* l2ring = nullptr;
@@ -537,7 +561,7 @@ struct lbxb {
     std::vector<BInst> tab;
     std::vector<Ctrl> ctrl_h;  // per instance slot: what reset_inst_ctrl uploads (kept until the stream syncs)
     std::vector<HostInst> hi;
-    std::vector<uint32_t> tile_inst_h, mp_tile_inst_h;
+    std::vector<uint32_t> mp_tile_inst_h;
     // the tiles of the instances with LB (0) or MP (1) work in the launches
     // about to run (built by upload_active; host copy kept until the stream syncs)
     uint32_t* act[2] = {nullptr, nullptr};
@@ -578,6 +602,9 @@ void free_all(lbxb* b) {
     dfree(b->nodes);
     dfree(b->maps);
     dfree(b->tile_inst);
+    dfree(b->nature);
+    dfree(b->counts);
+    dfree(b->nfi);
     dfree(b->act[0]);
     dfree(b->act[1]);
     dfree(b->insts);
@@ -969,6 +996,8 @@ int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
     if (ids.empty()) return LBX_OK;
     LBX_TRY(build_tiles(b, ids));
     const double eps = DBL_EPSILON;
+    std::vector<uint32_t> nfi(b->cap_inst);
+    LBX_TRY(download(b, b->nfi, b->cap_inst, nfi.data()));
     for (BInst& in : b->tab) in.lb_on = in.mp_on = 0;
     for (uint32_t id : ids) {
         HostInst& h = b->hi[id];
@@ -976,7 +1005,7 @@ int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
         TracerParams tp{};
         const double K = (std::fabs(h.kd) <= eps) ? 0.0 : h.ka / h.kd;  // module_moment_propagation.f90:46-50
         tp.ads[0] = std::fabs(K) > eps;                                 // :52-56
-        tp.bw[0] = 1.0 / ((double)h.Nf + K * (double)h.nfi);            // :97
+        tp.bw[0] = 1.0 / ((double)h.Nf + K * (double)nfi[id]);            // :97
         tp.ka[0] = h.ka;
         tp.kd[0] = h.kd;
         tp.one_minus_kd[0] = 1.0 - h.kd;
@@ -1042,8 +1071,8 @@ int64_t lbxb_footprint_bytes(int32_t precision, int64_t capacity_nodes, int64_t 
     const uint64_t Np = ((uint64_t)capacity_nodes + kTile - 1) / kTile * kTile;
     const uint64_t pop = (precision == LBX_PREC_FP32_SHIFT || precision == LBX_PREC_FP32_STORE) ? 4 : 8;
     uint64_t by = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + Np * 4 +
-                  (uint64_t)capacity_box * 4 + Np / kTile * 4;
-    by += (uint64_t)max_instances * (sizeof(BInst) + 3 * kSlots * 8 + kRing * 8 + sizeof(Ctrl));
+                  (uint64_t)capacity_box * 5 + node_chunks((uint64_t)capacity_box) * 4ull + Np / kTile * 4;
+    by += (uint64_t)max_instances * (4 + sizeof(BInst) + 3 * kSlots * 8 + kRing * 8 + sizeof(Ctrl));
     // MP: twice the nodes' entries (probabilities or (rho, v), rem, u*, P and Pa twice, slot table, node),
     // halo lists, partials, each node's entry
     const uint64_t M = 2 * Np;
@@ -1092,6 +1121,9 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
     if (!st) st = dalloc(&b->nodes, Np);
     if (!st) st = dalloc(&b->maps, (uint64_t)capacity_box);
     if (!st) st = dalloc(&b->tile_inst, (uint64_t)b->ntiles_cap);
+    if (!st) st = dalloc(&b->nature, ((uint64_t)capacity_box + 15) / 16 * 16);
+    if (!st) st = dalloc(&b->counts, (uint64_t)node_chunks((uint64_t)capacity_box));
+    if (!st) st = dalloc(&b->nfi, (uint64_t)max_instances);
     if (!st) st = dalloc(&b->act[0], (uint64_t)b->ntiles_cap);
     if (!st) st = dalloc(&b->act[1], 2 * (uint64_t)b->ntiles_cap);
     if (!st) st = dalloc(&b->insts, (uint64_t)max_instances);
@@ -1137,12 +1169,11 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
         b->tab.assign(max_instances, BInst{});
         b->ctrl_h.assign(max_instances, Ctrl{});
         b->hi.assign(max_instances, HostInst{});
-        b->tile_inst_h.assign(b->ntiles_cap, kNoInst);
         b->mp_tile_inst_h.assign(2 * (size_t)b->ntiles_cap, kNoInst);
         b->node_alloc.init(b->ntiles_cap);
         b->map_alloc.init(b->cap_box);
-        st = hip_status(hipMemcpyAsync(b->tile_inst, b->tile_inst_h.data(), b->ntiles_cap * sizeof(uint32_t),
-                                       hipMemcpyHostToDevice, b->stream));
+        st = hip_status(hipMemsetAsync(b->tile_inst, 0xFF, b->ntiles_cap * sizeof(uint32_t), b->stream));  // kNoInst
+        if (!st) st = hip_status(hipMemsetAsync(b->nfi, 0, b->cap_inst * sizeof(uint32_t), b->stream));
     }
     if (!st) st = hip_status(hipMemcpyAsync(b->insts, b->tab.data(), b->tab.size() * sizeof(BInst),
                                             hipMemcpyHostToDevice, b->stream));
@@ -1179,15 +1210,7 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     while (id < b->cap_inst && b->hi[id].phase != kFree) ++id;
     if (id == b->cap_inst) return LBX_ERR_NOMEM;
     HostInst h;
-    std::vector<int8_t> itf(N);
-    lbx_detect_interfacial(lx, ly, lz, nature, itf.data());
-    h.nodes_h.reserve(N);
-    for (uint32_t r = 0; r < N; ++r)
-        if (nature[r] == 0) {
-            h.nodes_h.push_back(r | (itf[r] ? kNodeInterfacial : 0u));
-            h.nfi += itf[r] != 0;
-        }
-    h.Nf = (uint32_t)h.nodes_h.size();
+    h.Nf = count_fluid(nature, N);
     if (h.Nf == 0) return LBX_ERR_ARG;
     const uint64_t ntiles = (h.Nf + kTile - 1) / kTile;
     uint64_t tile0 = 0, map0 = 0;
@@ -1233,29 +1256,26 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     in.rho0 = rho0;
     in.target = target_error;
     in.floor_window = shift(b) ? b->floor_window : 0;
-    // nodes (global packed indices of the instance's fluid nodes) and its map:
-    // through a pinned buffer where they fit, so that the call needs no wait
-    const size_t bytes = (h.Nf + (size_t)N) * sizeof(uint32_t);
-    const bool staged = bytes <= kStage;
+    // the nature, through a pinned buffer where it fits, so that the call needs no wait
+    const bool staged = N <= kStage;
     const int at = b->stage_at;
-    std::vector<uint32_t> own(staged ? 0 : h.Nf + (size_t)N);
     int st = staged ? hip_status(hipEventSynchronize(b->stage_ev[at])) : LBX_OK;
-    uint32_t* gnodes = staged ? (uint32_t*)b->stage[at] : own.data();
-    uint32_t* map = gnodes + h.Nf;
-    std::memcpy(gnodes, h.nodes_h.data(), h.Nf * sizeof(uint32_t));
-    std::fill(map, map + N, kSolidSlot);
-    for (uint32_t i = 0; i < h.Nf; ++i) map[h.nodes_h[i] & kIndexMask] = in.node_off + i;
-    if (!st) st = hip_status(hipMemcpyAsync(b->nodes + in.node_off, gnodes, h.Nf * sizeof(uint32_t),
+    if (staged) std::memcpy(b->stage[at], nature, N);
+    if (!st) st = hip_status(hipMemcpyAsync(b->nature, staged ? (const void*)b->stage[at] : (const void*)nature, N,
                                             hipMemcpyHostToDevice, b->stream));
-    if (!st) st = hip_status(hipMemcpyAsync(b->maps + map0, map, N * sizeof(uint32_t), hipMemcpyHostToDevice,
-                                            b->stream));
-    // rest state and the opening collision of step 1 (no force)
+    const uint32_t chunks = node_chunks(N);
+    if (!st && chunks > kNodeCountChunks)
+        hipLaunchKernelGGL(k_node_count, dim3(chunks), dim3(kNodeThreads), 0, b->stream, b->nature, (uint32_t)N,
+                           b->counts);
+    // node list, map (global packed indices), rest state and the opening collision of step 1 (no force)
     if (!st) {
         auto admit = [&](auto* f, auto* jold) {
             using E = std::remove_pointer_t<decltype(f)>;
             using R = std::remove_pointer_t<decltype(jold)>;
-            hipLaunchKernelGGL((kb_admit<E, R>), dim3(ntiles), dim3(kBlock), 0, b->stream, f, jold, b->rho, b->j, in, id,
-                               b->tile_inst, b->slots, b->l2ring, b->ctrl, b->Np);
+            hipLaunchKernelGGL((kb_admit<E, R>), dim3(std::max<uint32_t>((uint32_t)ntiles, chunks)), dim3(kBlock), 0,
+                               b->stream, f, jold, b->rho, b->j, in, id, b->tile_inst, b->slots, b->l2ring, b->ctrl,
+                               b->Np, b->nature, (uint32_t)N, chunks > kNodeCountChunks ? b->counts : nullptr,
+                               b->nodes, b->maps, b->nfi);
         };
         if (b->prec == LBX_PREC_FP32_SHIFT)
             admit(b->g[0], b->j32);
@@ -1267,10 +1287,8 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
     }
     if (!st && staged) st = hip_status(hipEventRecord(b->stage_ev[at], b->stream));
     if (staged) b->stage_at ^= 1;
-    for (uint64_t t = 0; t < ntiles; ++t) b->tile_inst_h[tile0 + t] = id;
-    if (!st && !staged) st = hip_status(hipStreamSynchronize(b->stream));  // own is a local
+    if (!st && !staged) st = hip_status(hipStreamSynchronize(b->stream));  // the nature is the caller's
     if (st) {
-        for (uint64_t t = 0; t < ntiles; ++t) b->tile_inst_h[tile0 + t] = kNoInst;
         b->node_alloc.give(tile0, ntiles);
         b->map_alloc.give(map0, N);
         return st;
@@ -1283,17 +1301,16 @@ int lbxb_add(lbxb* b, int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
 
 int lbxb_remove(lbxb* b, int32_t id) {
     if (!b || id < 0 || (uint32_t)id >= b->cap_inst || b->hi[id].phase == kFree) return LBX_ERR_ARG;
-    (void)hipStreamSynchronize(b->stream);
+    // no wait: what follows on the stream finds the tiles free
     BInst& in = b->tab[id];
-    for (uint32_t t = 0; t < in.ntiles; ++t) b->tile_inst_h[in.tile_first + t] = kNoInst;
-    LBX_TRY(hipMemcpyAsync(b->tile_inst + in.tile_first, b->tile_inst_h.data() + in.tile_first,
-                           in.ntiles * sizeof(uint32_t), hipMemcpyHostToDevice, b->stream));
+    hipLaunchKernelGGL(kb_release, dim3((in.ntiles + kBlock - 1) / kBlock), dim3(kBlock), 0, b->stream, b->tile_inst + in.tile_first,
+                       in.ntiles, b->nfi + id);
     b->node_alloc.give(in.tile_first, in.ntiles);
     b->map_alloc.give(in.map_off, b->hi[id].map_n);
     if (b->hi[id].general) --b->n_general;
     b->hi[id] = HostInst{};
     in = BInst{};
-    return hip_status(hipStreamSynchronize(b->stream));
+    return hip_status(hipGetLastError());
 }
 
 // One round: redo launches of instances whose stage 1 ended, lb_steps LB
@@ -1397,7 +1414,7 @@ int lbxb_round(lbxb* b, int32_t lb_steps, int32_t mp_steps, int32_t* active) {
         vt.resize((size_t)S_mp * ni * 3);
         LBX_TRY(download(b, b->vtrace, vt.size(), vt.data()));
     }
-    std::vector<uint32_t> to_mp;
+    std::vector<uint32_t> to_mp, capped;
     for (uint32_t id = 0; id < ni; ++id) {
         BInst& in = b->tab[id];
         HostInst& h = b->hi[id];
@@ -1423,10 +1440,7 @@ int lbxb_round(lbxb* b, int32_t lb_steps, int32_t mp_steps, int32_t* active) {
             } else {
                 h.t = last;
                 if (h.max_lb > 0 && h.t >= h.max_lb) {
-                    double l2 = 0.0;
-                    LBX_TRY(download(b, b->l2ring + (uint64_t)id * kRing + (h.t % kRing), 1, &l2));
-                    h.exit_reason = (h.stage == 2 && h.t > h.check_after && l2 <= in.target) ? LBX_EXIT_CONVERGED
-                                                                                             : LBX_EXIT_CAP;
+                    capped.push_back(id);
                     h.phase = kLbDone;
                 }
             }
@@ -1443,6 +1457,23 @@ int lbxb_round(lbxb* b, int32_t lb_steps, int32_t mp_steps, int32_t* active) {
             }
         }
         in.lb_on = in.mp_on = 0;
+    }
+    if (!capped.empty()) {  // l2err of their last step, all in one copy (one per instance took 15 ms for 1024)
+        const uint32_t n = (uint32_t)capped.size();
+        std::vector<uint64_t> at;
+        for (uint32_t id : capped) at.push_back((uint64_t)id * kRing + (uint64_t)(b->hi[id].t % kRing));
+        uint64_t* at_d = (uint64_t*)b->vtrace + n;  // of kRoundMax x 3 per instance, read above
+        std::vector<double> l2(n);
+        LBX_TRY(hipMemcpyAsync(at_d, at.data(), n * sizeof(uint64_t), hipMemcpyHostToDevice, b->stream));
+        hipLaunchKernelGGL(kb_pick_l2, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, b->stream, b->l2ring, at_d, n, b->vtrace);
+        LBX_TRY(hipGetLastError());
+        LBX_TRY(download(b, b->vtrace, n, l2.data()));
+        for (uint32_t k = 0; k < n; ++k) {
+            HostInst& h = b->hi[capped[k]];
+            h.exit_reason = (h.stage == 2 && h.t > h.check_after && l2[k] <= b->tab[capped[k]].target)
+                                ? LBX_EXIT_CONVERGED
+                                : LBX_EXIT_CAP;
+        }
     }
     b->lb_box_updates += lb_box;
     b->lb_fluid_updates += lb_fluid;
@@ -1480,13 +1511,18 @@ int lbxb_result(lbxb* b, int32_t id, double deff[3], double* vacf, int64_t vacf_
     }
     // flow fields of the instance (valid once its LB phase has ended)
     double* dst[4] = {rho, jx, jy, jz};
+    std::vector<uint32_t> nodes;
+    if (rho || jx || jy || jz) {
+        nodes.resize(h.Nf);
+        LBX_TRY(download(b, b->nodes + in.node_off, h.Nf, nodes.data()));
+    }
     for (int k = 0; k < 4; ++k) {
         if (!dst[k]) continue;
         std::vector<double> tmp(h.Nf);
         const double* src = k == 0 ? b->rho + in.node_off : b->j + (uint64_t)(k - 1) * b->Np + in.node_off;
         LBX_TRY(download(b, src, h.Nf, tmp.data()));
         std::memset(dst[k], 0, (size_t)h.N * sizeof(double));
-        for (uint32_t i = 0; i < h.Nf; ++i) dst[k][h.nodes_h[i] & kIndexMask] = tmp[i];
+        for (uint32_t i = 0; i < h.Nf; ++i) dst[k][nodes[i] & kIndexMask] = tmp[i];
     }
     return LBX_OK;
 }

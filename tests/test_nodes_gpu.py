@@ -1,0 +1,55 @@
+"""The node list, map and interfacial flags built on the GPU (lbx_nodes.h) at
+the edges of its chunks (4096 box nodes) and of the launch that counts them
+(more than 8 chunks), single and as batch instances: fields and P, Pa of an
+adsorbing tracer (whose normalisation counts the interfacial nodes) bit for bit
+with the restatement's."""
+import numpy as np
+import pytest
+
+import lbref
+from laboetie_amd import lbx
+
+BOXES = [(1, 1, 1), (1, 1, 300), (5, 9, 91), (16, 16, 16), (17, 241, 1), (32, 32, 32), (33, 32, 32), (61, 89, 53)]
+
+
+def medium(dims, solid):
+    rng = np.random.default_rng(int(np.prod(dims)))
+    nat = (rng.random(int(np.prod(dims))) < solid).astype(np.int8)
+    nat[0] = 0
+    nat[nat != 0] = rng.choice([1, 2, -1], int((nat != 0).sum()))  # solid: any value but 0
+    return nat
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solid", [0.0, 0.4, 0.995])
+@pytest.mark.parametrize("dims", BOXES)
+def test_nodes(dims, solid):
+    print("nodes", dims, solid, flush=True)
+    nat = medium(dims, solid)
+    fext, steps = [2e-5, -1e-5, 3e-5], 3
+    with lbx.Lattice(dims, nat, 0.9) as L:
+        assert L.fluid_nodes == int((nat == 0).sum())
+        L.init_rest(1.0)
+        L.equilibrate(fext, 0.0, max_steps=6)
+        v0 = L.mp_init(fext, 0.01, 0.02, 0.01)
+        _, rho, j = L.get_state(populations=False)
+        m = L.mp_run(steps)
+        v = np.vstack([v0, m["vacf"]])
+        fields = L.mp_get()
+    assert np.array_equal(rho != 0.0, nat == 0)
+    flat = (nat != 0).astype(np.int8)
+    mp = lbref.MP(dims, flat, lbref.interfacial(*dims, flat), lbref.tracer_population(dims, flat, rho, j, fext), rho,
+                  0.01, 0.02, 0.01)
+    assert mp.run(steps)[0] == 0
+    assert np.array_equal(fields[0], mp.P) and np.array_equal(fields[1], mp.Pa)
+    with lbx.Batch(-(-int((nat == 0).sum()) // 256) * 256 + 512, nat.size + 7, 2) as B:
+        first = B.add((1, 1, 7), np.zeros(7, np.int8), 0.9, 1.0, fext, 0.0, 0.01, 0.0, 0.0, 1, max_lb_steps=6)
+        for _ in range(2):  # the second time in place of a removed one
+            i = B.add(dims, nat, 0.9, 1.0, fext, 0.0, 0.01, 0.02, 0.01, steps, max_lb_steps=6)
+            while B.round(4, 4):
+                pass
+            g = B.result(i, vacf_rows=steps + 1, flow=True)
+            assert np.array_equal(g["vacf"], v)
+            assert np.array_equal(g["rho"], rho) and np.array_equal(g["j"], j)
+            B.remove(i)
+        B.remove(first)
