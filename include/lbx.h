@@ -334,10 +334,11 @@ int lbx_set_floor_window(lbx_ctx* ctx, int64_t steps);
  * the reference. */
 int lbx_set_check_interval(lbx_ctx* ctx, int32_t steps);
 
-/* Element addressing of the step kernels.  The population and moment arrays
- * are addressed through 32-bit buffer offsets while 19*Np*8 < 4 GiB (Np: the
+/* Element addressing of the LB kernels.  The population and flux arrays are
+ * addressed through 32-bit buffer offsets while 19*Np*8 < 4 GiB (Np: the
  * fluid-node count rounded up to 64), and through 64-bit pointers above that;
- * the library picks the form from the size.  wide = 1 selects the 64-bit form
+ * the library picks the form from the size.  (Moment propagation addresses its
+ * arrays per tile and has one form.)  wide = 1 selects the 64-bit form
  * on a smaller lattice too, so the two forms can be checked against each other
  * (they give the same bits); wide = 0 returns to the size's choice.
  * lbx_addressing reports the form in use (1: 64-bit).  No counterpart in the
@@ -452,7 +453,7 @@ int lbxb_set_floor_window(lbxb* b, int64_t steps);
 #define LBXB_LAUNCH_PERSISTENT 2
 int lbxb_set_launch_mode(lbxb* b, int32_t mode);
 int lbxb_launch_mode(lbxb* b);
-/* Element addressing of the batch's step kernels, as lbx_set_addressing
+/* Element addressing of the batch's LB kernels, as lbx_set_addressing
  * (the capacity decides by itself; wide = 1 forces the 64-bit form). */
 int lbxb_set_addressing(lbxb* b, int32_t wide);
 int lbxb_addressing(lbxb* b);
