@@ -1,15 +1,16 @@
 """The node list, map and interfacial flags built on the GPU (lbx_nodes.h) at
 the edges of its chunks (4096 box nodes) and of the launch that counts them
-(more than 8 chunks), single and as batch instances: fields and P, Pa of an
-adsorbing tracer (whose normalisation counts the interfacial nodes) bit for bit
-with the restatement's."""
+(more than 8 chunks), and above the 1 MiB that a batch stages, single and as
+batch instances: fields and P, Pa of an adsorbing tracer (whose normalisation
+counts the interfacial nodes) bit for bit with the restatement's."""
 import numpy as np
 import pytest
 
 import lbref
 from laboetie_amd import lbx
 
-BOXES = [(1, 1, 1), (1, 1, 300), (5, 9, 91), (16, 16, 16), (17, 241, 1), (32, 32, 32), (33, 32, 32), (61, 89, 53)]
+BOXES = [(1, 1, 1), (1, 1, 300), (5, 9, 91), (16, 16, 16), (17, 241, 1), (32, 32, 32), (33, 32, 32), (61, 89, 53),
+         (103, 101, 101)]
 
 
 def medium(dims, solid):
