@@ -132,7 +132,7 @@ struct lbx_ctx {
     std::vector<double> jpart_h;
     std::vector<double> jsum_trace;   // sum of j over the fluid nodes, 3 per step
     double* jflow = nullptr;          // lbx_flow: the flux of the last step
-    double* box = nullptr;            // full-box copies: the values of a run of box nodes
+    double* box = nullptr;            // full-box copies: the values of planes or of a run of box nodes
     uint32_t box_n = 0;               // ... and how many it holds
 };
 
@@ -444,108 +444,156 @@ int build_nodes(lbx_ctx* c, const int8_t* nature, uint32_t* nfi) {
 }
 
 // ---- full-box host arrays <-> packed device planes
-// A plane of the full box passes through a device buffer, a run of box nodes
-// at a time: the kernel below spreads (gathers) the packed values, and the copy
-// goes straight to (from) the caller's array.  One host thread doing this per
-// node through a temporary took 160 ms for the density and flux of a 256^3
-// medium; now it is the copy.
+// The planes of the full box pass through a device buffer, as many whole
+// planes at a time as it holds (a run of box nodes of one plane where it is
+// smaller than a plane): one kernel spreads (gathers) the packed values, and
+// the copies go straight to (from) the caller's arrays, adjacent ones as one.
+// One host thread doing this per node through a temporary took 160 ms for the
+// density and flux of a 256^3 medium; now it is the copy.  A launch, a copy and
+// a wait of their own for each of a state's 23 planes cost a small lattice
+// 20 us a plane: lbx_get_state and lbx_set_state, us, plane by plane /
+// together: 4^3 nodes 535 / 58 and 464 / 30, 32^3 820 / 468 and 840 / 270.
 
-// The buffer's nodes (*run), kept until the context goes.  32 MB, or as much
+constexpr int kMaxPlanes = kQ + 4;  // a whole state: populations, density, flux
+
+// The planes of one transfer.
+struct Planes {
+    int n = 0;
+    double* host[kMaxPlanes];
+    struct Dev {
+        void* at[kMaxPlanes];     // packed: FP64 values, or FP32 deviations from rest
+        double rest[kMaxPlanes];
+        uint32_t f32 = 0;         // bit p: plane p is FP32
+    } dev;
+    void add(double* d, const double* h) {
+        dev.at[n] = d;
+        dev.rest[n] = 0.0;
+        host[n++] = const_cast<double*>(h);
+    }
+    void add(float* d, double rest, const double* h) {
+        dev.f32 |= 1u << n;
+        dev.at[n] = d;
+        dev.rest[n] = rest;
+        host[n++] = const_cast<double*>(h);
+    }
+};
+
+// Values the transfer buffer holds: all planes of a state of a small box,
+// 2 MB or, of a large box, one plane's up to 32 MB.
+uint32_t box_values(uint64_t N) {
+    return (uint32_t)std::min<uint64_t>(kMaxPlanes * N, std::max<uint64_t>(1u << 18, std::min<uint64_t>(N, 1u << 22)));
+}
+
+// The buffer (c->box, c->box_n values), kept until the context goes; as much
 // of it as the device still has.
-int box_buffer(lbx_ctx* c, double** box, uint32_t* run) {
-    for (uint32_t n = std::max(3u, std::min(c->N, 1u << 22)); !c->box;) {
+int box_buffer(lbx_ctx* c) {
+    for (uint32_t n = box_values(c->N); !c->box;) {
         const int st = dalloc(&c->box, n);
         c->box_n = st ? 0 : n;
         if (!st) break;
         if (st != LBX_ERR_NOMEM || n <= 4096) return st;
         n /= 4;
     }
-    *box = c->box;
-    *run = c->box_n;
     return LBX_OK;
 }
 
-// a packed plane of E as FP64 values of the box nodes [r0, r0 + n), 0 at
-// solids; FP32 deviations become rest + g
-template <typename E>
-__global__ __launch_bounds__(kBlock) void k_spread(const E* __restrict__ src, const uint32_t* __restrict__ map,
-                                                   double* __restrict__ box, uint32_t r0, uint32_t n, double rest) {
+// box nodes [r0, r0 + n) of the planes p0 + blockIdx.y: packed values as FP64,
+// 0 at solids; FP32 deviations become rest + g
+__global__ __launch_bounds__(kBlock) void k_spread(Planes::Dev d, int p0, const uint32_t* __restrict__ map,
+                                                   double* __restrict__ box, uint32_t r0, uint32_t n) {
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= n) return;
+    const int p = p0 + (int)blockIdx.y;
     const uint32_t q = map[r0 + k];
     double v = 0.0;
     if (q != kSolidSlot) {
-        if constexpr (std::is_same<E, float>::value) v = rest + (double)src[q]; else v = src[q];
+        if (d.f32 >> p & 1u) v = d.rest[p] + (double)((const float*)d.at[p])[q]; else v = ((const double*)d.at[p])[q];
     }
-    box[k] = v;
+    box[(uint64_t)blockIdx.y * n + k] = v;
 }
 
-// the inverse: the fluid nodes of the run into their packed places
-template <typename E>
-__global__ __launch_bounds__(kBlock) void k_gather(E* __restrict__ dst, const uint32_t* __restrict__ map,
+// the inverse: the fluid nodes of the run into their packed places; the pad
+// values after the last node (fewer than 64) are 0
+__global__ __launch_bounds__(kBlock) void k_gather(Planes::Dev d, int p0, const uint32_t* __restrict__ map,
                                                    const double* __restrict__ box, uint32_t r0, uint32_t n,
-                                                   double rest) {
+                                                   uint32_t Nf, uint32_t pad) {
     const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    const int p = p0 + (int)blockIdx.y;
+    const bool f32 = d.f32 >> p & 1u;
+    if (r0 == 0 && k < pad) {
+        if (f32) ((float*)d.at[p])[Nf + k] = 0.0f; else ((double*)d.at[p])[Nf + k] = 0.0;
+    }
     if (k >= n) return;
     const uint32_t q = map[r0 + k];
     if (q == kSolidSlot) return;
-    if constexpr (std::is_same<E, float>::value) dst[q] = (float)(box[k] - rest); else dst[q] = box[k];
+    const double v = box[(uint64_t)blockIdx.y * n + k];
+    if (f32) ((float*)d.at[p])[q] = (float)(v - d.rest[p]); else ((double*)d.at[p])[q] = v;
 }
 
-template <typename E>
-int download_plane(lbx_ctx* c, const E* src, double rest, double* host) {
-    double* box;
-    uint32_t run;
-    LBX_TRY(box_buffer(c, &box, &run));
-    for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
-        const uint32_t n = std::min(run, c->N - r0);
-        hipLaunchKernelGGL(k_spread<E>, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, src, c->map, box, r0, n, rest);
-        LBX_TRY(hipGetLastError());
-        LBX_TRY(hipMemcpyAsync(host + r0, box, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        LBX_TRY(hipStreamSynchronize(c->stream));
+// f(p0, planes, r0, n) for each fill of the buffer
+template <typename F>
+int box_fills(lbx_ctx* c, int planes, F&& f) {
+    if (planes == 0) return LBX_OK;
+    LBX_TRY(box_buffer(c));
+    const uint32_t run = std::min(c->N, c->box_n);
+    const int per = run < c->N ? 1 : (int)std::min<uint32_t>((uint32_t)planes, c->box_n / c->N);
+    for (int p0 = 0; p0 < planes; p0 += per)
+        for (uint32_t r0 = 0; r0 < c->N; r0 += run)
+            LBX_TRY(f(p0, std::min(per, planes - p0), r0, std::min(run, c->N - r0)));
+    return LBX_OK;
+}
+
+// the copies of one fill; planes whose host arrays follow one another are one copy
+int box_copies(lbx_ctx* c, const Planes& s, int p0, int np, uint32_t r0, uint32_t n, bool down) {
+    for (int p = 0; p < np;) {
+        int m = 1;
+        while (n == c->N && p + m < np && s.host[p0 + p + m] == s.host[p0 + p] + (size_t)m * n) ++m;
+        double *dev = c->box + (size_t)p * n, *host = s.host[p0 + p] + r0;
+        const size_t bytes = (size_t)m * n * sizeof(double);
+        LBX_TRY(down ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream)
+                     : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c->stream));
+        p += m;
     }
     return LBX_OK;
 }
 
-template <typename E>
-int upload_plane(lbx_ctx* c, const double* host, double rest, E* dst) {
-    double* box;
-    uint32_t run;
-    LBX_TRY(box_buffer(c, &box, &run));
-    // the padding after the last node is 0
-    LBX_TRY(hipMemsetAsync(dst + c->Nf, 0, (c->Np - c->Nf) * sizeof(E), c->stream));
-    for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
-        const uint32_t n = std::min(run, c->N - r0);
-        LBX_TRY(hipMemcpyAsync(box, host + r0, (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        hipLaunchKernelGGL(k_gather<E>, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, dst, c->map, box, r0, n, rest);
+int download(lbx_ctx* c, const Planes& s) {
+    return box_fills(c, s.n, [&](int p0, int np, uint32_t r0, uint32_t n) -> int {
+        hipLaunchKernelGGL(k_spread, dim3(nblocks(n), np), dim3(kBlock), 0, c->stream, s.dev, p0, c->map, c->box, r0,
+                           n);
         LBX_TRY(hipGetLastError());
-        LBX_TRY(hipStreamSynchronize(c->stream));
+        LBX_TRY(box_copies(c, s, p0, np, r0, n, true));
+        return hip_status(hipStreamSynchronize(c->stream));
+    });
+}
+
+int upload(lbx_ctx* c, const Planes& s) {
+    return box_fills(c, s.n, [&](int p0, int np, uint32_t r0, uint32_t n) -> int {
+        LBX_TRY(box_copies(c, s, p0, np, r0, n, false));
+        hipLaunchKernelGGL(k_gather, dim3(nblocks(n), np), dim3(kBlock), 0, c->stream, s.dev, p0, c->map, c->box, r0,
+                           n, c->Nf, (uint32_t)(c->Np - c->Nf));
+        LBX_TRY(hipGetLastError());
+        return hip_status(hipStreamSynchronize(c->stream));
+    });
+}
+
+// the populations of buffer b (n = a0 rho0 + g in the FP32 forms; 0 at solid
+// nodes), and the density with the flux; NULL host arrays are left out
+void add_populations(lbx_ctx* c, Planes& s, int b, const double* n) {
+    for (int l = 0; n && l < kQ; ++l) {
+        const double* h = n + (size_t)l * c->N;
+        if (f32_storage(c->prec))
+            s.add(c->g[b] + (size_t)l * c->Np, a0(l) * c->rho0, h);
+        else
+            s.add(c->f[b] + (size_t)l * c->Np, h);
     }
-    return LBX_OK;
 }
-
-int download_full(lbx_ctx* c, const double* dsrc, int planes, double* host_full) {
-    for (int p = 0; p < planes; ++p)
-        LBX_TRY(download_plane(c, dsrc + (size_t)p * c->Np, 0.0, host_full + (size_t)p * c->N));
-    return LBX_OK;
-}
-
-int upload_full(lbx_ctx* c, const double* const* host_planes, int planes, double* ddst) {
-    for (int p = 0; p < planes; ++p) LBX_TRY(upload_plane(c, host_planes[p], 0.0, ddst + (size_t)p * c->Np));
-    return LBX_OK;
-}
-
-// FP32-shift populations <-> full-box FP64 n = a0 rho0 + g (0 at solid nodes)
-int download_shift(lbx_ctx* c, const float* gsrc, double* n_full) {
-    for (int l = 0; l < kQ; ++l)
-        LBX_TRY(download_plane(c, gsrc + (size_t)l * c->Np, a0(l) * c->rho0, n_full + (size_t)l * c->N));
-    return LBX_OK;
-}
-
-int upload_shift(lbx_ctx* c, const double* n_full, float* gdst) {
-    for (int l = 0; l < kQ; ++l)
-        LBX_TRY(upload_plane(c, n_full + (size_t)l * c->N, a0(l) * c->rho0, gdst + (size_t)l * c->Np));
-    return LBX_OK;
+void add_flow(lbx_ctx* c, Planes& s, double* rho_d, double* j_d, const double* rho, const double* jx,
+              const double* jy, const double* jz) {
+    if (rho) s.add(rho_d, rho);
+    const double* jp[3] = {jx, jy, jz};
+    for (int a = 0; a < 3; ++a)
+        if (jp[a]) s.add(j_d + a * c->Np, jp[a]);
 }
 
 // The MP tiles of the context's geometry: counted, grouped, placed and
@@ -806,7 +854,7 @@ int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precisio
     const uint64_t pop = f32_storage(precision) ? 4 : 8;  // populations; also win and u* of moment propagation
     uint64_t b = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + N * 8 +
                  18 * 4 * std::min<uint64_t>(Np, (kTabNodes + 63) / 64 * 64) +
-                 std::min<uint64_t>(N, 1u << 22) * 8 + sizeof(Ctrl) + kRing * 8;
+                 box_values(N) * 8ull + sizeof(Ctrl) + kRing * 8;
     if (with_mp > 0) {  // with_mp tracers, each with adsorption (the upper bound)
         const uint64_t T = (uint64_t)std::min(with_mp, kMaxTracers);
         const Bricks br = make_bricks((uint32_t)lx, (uint32_t)ly, (uint32_t)lz);
@@ -929,19 +977,13 @@ int lbx_set_state(lbx_ctx* c, const double* n, const double* rho, const double* 
                   const double* jz) {
     if (!c || !n || !rho || !jx || !jy || !jz) return LBX_ERR_ARG;
     c->eq.active = false;  // a paused run is abandoned
-    if (f32_storage(c->prec)) {
-        // the rest density of the deviations: the density of the first fluid
-        // node (the uniform rest density when the state is a rest state)
-        c->rho0 = rho[c->first_node];
-        LBX_TRY(upload_shift(c, n, c->g[0]));
-    } else {
-        const double* planes[kQ];
-        for (int l = 0; l < kQ; ++l) planes[l] = n + (size_t)l * c->N;
-        LBX_TRY(upload_full(c, planes, kQ, c->f[0]));
-    }
-    LBX_TRY(upload_full(c, &rho, 1, c->rho));
-    const double* jp[3] = {jx, jy, jz};
-    LBX_TRY(upload_full(c, jp, 3, c->j));
+    // the rest density of the deviations: the density of the first fluid node
+    // (the uniform rest density when the state is a rest state)
+    if (f32_storage(c->prec)) c->rho0 = rho[c->first_node];
+    Planes s;
+    add_populations(c, s, 0, n);
+    add_flow(c, s, c->rho, c->j, rho, jx, jy, jz);
+    LBX_TRY(upload(c, s));
     c->pre = 0;
     return LBX_OK;
 }
@@ -961,13 +1003,10 @@ int lbx_l2err_trace(lbx_ctx* c, int64_t first_step, int64_t count, double* out, 
 int lbx_get_state(lbx_ctx* c, double* n, double* rho, double* jx, double* jy, double* jz) {
     if (!c) return LBX_ERR_ARG;
     if (c->eq.active) return LBX_ERR_STATE;  // during a paused run: lbx_flow
-    if (n && f32_storage(c->prec)) LBX_TRY(download_shift(c, c->g[c->pre], n));
-    if (n && !f32_storage(c->prec)) LBX_TRY(download_full(c, c->f[c->pre], kQ, n));
-    if (rho) LBX_TRY(download_full(c, c->rho, 1, rho));
-    double* jp[3] = {jx, jy, jz};
-    for (int a = 0; a < 3; ++a)
-        if (jp[a]) LBX_TRY(download_full(c, c->j + a * c->Np, 1, jp[a]));
-    return LBX_OK;
+    Planes s;
+    add_populations(c, s, c->pre, n);
+    add_flow(c, s, c->rho, c->j, rho, jx, jy, jz);
+    return download(c, s);
 }
 
 // The end of an equilibration run: the post-streaming state of its last step
@@ -1181,11 +1220,9 @@ int lbx_flow(lbx_ctx* c, double* rho, double* jx, double* jy, double* jz) {
         hipLaunchKernelGGL(k_flow, dim3(gt), dim3(kBlock), 0, c->stream, c->f[src], c->jflow, c->nodes,
                            c->map, c->dlx, c->dly, c->lz, c->Nf, c->Np, Ft[0] / 2.0, Ft[1] / 2.0, Ft[2] / 2.0);
     LBX_TRY(hipGetLastError());
-    if (rho) LBX_TRY(download_full(c, c->jflow, 1, rho));
-    double* jp[3] = {jx, jy, jz};
-    for (int a = 0; a < 3; ++a)
-        if (jp[a]) LBX_TRY(download_full(c, c->jflow + (a + 1) * c->Np, 1, jp[a]));
-    return LBX_OK;
+    Planes s;
+    add_flow(c, s, c->jflow, c->jflow + c->Np, rho, jx, jy, jz);
+    return download(c, s);
 }
 
 // Whether a propagation keeps the 18 incoming probabilities per node or
@@ -1274,9 +1311,9 @@ int lbx_mp_init_batch(lbx_ctx* c, const double fext[3], double Db, int32_t ntrac
 int lbx_mp_init_from_flow(lbx_ctx* c, const double* rho, const double* jx, const double* jy, const double* jz,
                           const double fext[3], double Db, double ka, double kd, double vacf0[3]) {
     if (!c || !rho || !jx || !jy || !jz || !fext) return LBX_ERR_ARG;
-    LBX_TRY(upload_full(c, &rho, 1, c->rho));
-    const double* jp[3] = {jx, jy, jz};
-    LBX_TRY(upload_full(c, jp, 3, c->j));
+    Planes s;
+    add_flow(c, s, c->rho, c->j, rho, jx, jy, jz);
+    LBX_TRY(upload(c, s));
     return mp_setup(c, fext, Db, 1, &ka, &kd, vacf0);
 }
 
@@ -1410,33 +1447,38 @@ int lbx_mp_get_tracer(lbx_ctx* c, int32_t tracer, double* P, double* Pa) {
     if (!c) return LBX_ERR_ARG;
     if (!c->mp_ready || c->mpp.active) return LBX_ERR_STATE;  // a begun chunk is waited for first
     if (tracer < 0 || tracer >= c->ntr) return LBX_ERR_ARG;
-    // the tracer's three components into (3,lx,ly,lz), 0 at solids, a run of box nodes at a time
-    double* box;
-    uint32_t run;
-    LBX_TRY(box_buffer(c, &box, &run));
-    run /= 3;
-    auto fetch = [&](const double* src, double* dst) -> int {
+    // the tracer's three components into (3,lx,ly,lz), 0 at solids: P and Pa
+    // together where the buffer holds both, else a run of box nodes of one at a time
+    const double* src[2];
+    double* dst[2];
+    int nf = 0;
+    if (P) {
+        src[nf] = mp_moments(c, false)[c->mp_now];
+        dst[nf++] = P;
+    }
+    if (Pa && c->tp.ads[tracer]) {
+        src[nf] = mp_moments(c, true)[c->mp_now];
+        dst[nf++] = Pa;
+    }
+    if (Pa && !c->tp.ads[tracer]) std::memset(Pa, 0, 3 * (size_t)c->N * sizeof(double));
+    if (nf == 0) return LBX_OK;
+    LBX_TRY(box_buffer(c));
+    const uint32_t run = std::min(c->N, c->box_n / 3);
+    const int per = run < c->N ? 1 : (int)std::min<uint32_t>((uint32_t)nf, c->box_n / 3 / c->N);
+    for (int f0 = 0; f0 < nf; f0 += per) {
+        const int m = std::min(per, nf - f0);
         for (uint32_t r0 = 0; r0 < c->N; r0 += run) {
             const uint32_t n = std::min(run, c->N - r0);
-            LBX_TRY(hipMemsetAsync(box, 0, 3 * (uint64_t)n * sizeof(double), c->stream));
-            hipLaunchKernelGGL(k_mp_box, dim3(c->mp_ntiles), dim3(kBlock), 0, c->stream, src, c->mpt, 0u, c->nodes,
-                               c->ntr, tracer, box, r0, n);
+            hipLaunchKernelGGL(k_mp_box, dim3(nblocks(n), m), dim3(kBlock), 0, c->stream, src[f0], src[f0 + m - 1],
+                               c->mpt.inv, c->map, c->ntr, tracer, c->box, r0, n);
             LBX_TRY(hipGetLastError());
-            LBX_TRY(hipMemcpyAsync(dst + 3 * (size_t)r0, box, 3 * (uint64_t)n * sizeof(double),
-                                   hipMemcpyDeviceToHost, c->stream));
+            for (int k = 0; k < m; ++k)
+                LBX_TRY(hipMemcpyAsync(dst[f0 + k] + 3 * (size_t)r0, c->box + 3 * (size_t)k * n,
+                                       3 * (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
             LBX_TRY(hipStreamSynchronize(c->stream));
         }
-        return LBX_OK;
-    };
-    int st = LBX_OK;
-    if (P) st = fetch(mp_moments(c, false)[c->mp_now], P);
-    if (!st && Pa) {
-        if (c->tp.ads[tracer])
-            st = fetch(mp_moments(c, true)[c->mp_now], Pa);
-        else
-            std::memset(Pa, 0, 3 * (size_t)c->N * sizeof(double));
     }
-    return st;
+    return LBX_OK;
 }
 
 int lbx_mp_get(lbx_ctx* c, double* P, double* Pa) { return lbx_mp_get_tracer(c, 0, P, Pa); }

@@ -951,18 +951,18 @@ __global__ __launch_bounds__(1024) void k_mp_run(MpStepArgs<W> a, int64_t S, uin
     }
 }
 
-// P or Pa of tracer t of T into the full box, (3, box nodes): the nodes with
-// box index in [r0, r0 + n)
-__global__ __launch_bounds__(kBlock) void k_mp_box(const double* __restrict__ p, MpTiles t, uint32_t tile0,
-                                                   const uint32_t* __restrict__ nodes, int32_t T, int32_t tracer,
-                                                   double* __restrict__ out, uint32_t r0, uint32_t n) {
-    const uint32_t tile = tile0 + blockIdx.x, e = tile * kMpTile + threadIdx.x;
-    if (threadIdx.x >= t.info[tile]) return;
-    const uint32_t r = (nodes[t.perm[e]] & kIndexMask) - r0;
-    if (r >= n) return;
-    double v[3];
-    Trio<double>::load(p, e, T, tracer, v);
-    for (int c = 0; c < 3; ++c) out[3 * (uint64_t)r + c] = v[c];
+// P or Pa (p0 or p1 by blockIdx.y) of tracer t of T in the full box, three
+// values per box node of [r0, r0 + n), 0 at solids
+__global__ __launch_bounds__(kBlock) void k_mp_box(const double* __restrict__ p0, const double* __restrict__ p1,
+                                                   const uint32_t* __restrict__ inv, const uint32_t* __restrict__ map,
+                                                   int32_t T, int32_t tracer, double* __restrict__ out, uint32_t r0,
+                                                   uint32_t n) {
+    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= n) return;
+    const uint32_t q = map[r0 + k];
+    double v[3] = {0.0, 0.0, 0.0};
+    if (q != kSolidSlot) Trio<double>::load(blockIdx.y ? p1 : p0, inv[q], T, tracer, v);
+    for (int c = 0; c < 3; ++c) out[3 * ((uint64_t)blockIdx.y * n + k) + c] = v[c];
 }
 
 }  // namespace
