@@ -62,6 +62,16 @@ struct EqRun {
     int32_t reason = 0;
 };
 
+// One device allocation that several arrays share.  The driver takes and
+// gives back every large allocation by itself, some 0.1-0.2 ms each, and a
+// context made right after another went waits for the other's.  ms with an
+// allocation per array / with blocks: contexts made and destroyed in turn, 32^3
+// nodes 0.6-0.9 / 0.25, 128^3 3.4 / 0.6; lbx_mp_init again, 64^3 1.4 / 0.045.
+struct Block {
+    char* at = nullptr;
+    uint64_t bytes = 0;
+};
+
 struct lbx_ctx {
     int32_t lx = 0, ly = 0, lz = 0;
     FastDiv dlx{}, dly{};
@@ -132,6 +142,9 @@ struct lbx_ctx {
     std::vector<double> jpart_h;
     std::vector<double> jsum_trace;   // sum of j over the fluid nodes, 3 per step
     double* jflow = nullptr;          // lbx_flow: the flux of the last step
+    // the allocations behind the arrays above (Block): the LB phase's, the MP
+    // tiles' (by packed node and by tile) and a propagation's
+    Block lb_block, node_block, tile_block, mp_block;
     double* box = nullptr;            // full-box copies: the values of planes or of a run of box nodes
     uint32_t box_n = 0;               // ... and how many it holds
 };
@@ -188,35 +201,57 @@ void dfree(T*& p) {
     p = nullptr;
 }
 
+// lay(take) names a block's arrays by take(pointer, count); each begins where
+// an allocation of its own would, as far as its addresses matter: at a page, or
+// a 2 MiB page once it fills one.
+uint64_t block_align(uint64_t at, uint64_t bytes) {
+    const uint64_t a = bytes >= (2u << 20) ? 2u << 20 : 4096u;
+    return (at + a - 1) / a * a;
+}
+template <typename Lay>
+uint64_t block_bytes(Lay&& lay) {
+    uint64_t n = 0;
+    lay([&](auto*& p, uint64_t count) { n = block_align(n, count * sizeof(*p)) + count * sizeof(*p); });
+    return n;
+}
+template <typename Lay>
+void block_place(const Block& b, Lay&& lay) {
+    uint64_t n = 0;
+    lay([&](auto*& p, uint64_t count) {
+        n = block_align(n, count * sizeof(*p));
+        p = (std::remove_reference_t<decltype(p)>)(b.at + n);
+        n += count * sizeof(*p);
+    });
+}
+void give_block(Block* b) {
+    dfree(b->at);
+    b->bytes = 0;
+}
+// A block that lay's arrays fit, and them in it.  The one there is kept while
+// they fill three quarters of it.
+template <typename Lay>
+int take_block(Block* b, Lay&& lay) {
+    const uint64_t n = block_bytes(lay);
+    if (n > b->bytes || n < b->bytes / 4 * 3) {
+        give_block(b);
+        LBX_TRY(dalloc(&b->at, n));
+        b->bytes = n;
+    }
+    block_place(*b, lay);
+    return LBX_OK;
+}
+
 void free_mp(lbx_ctx* c) {
     if (c->mpp.active) {  // a begun chunk is dropped once its kernels are done with the buffers
         (void)hipStreamSynchronize(c->stream);
         c->mpp.active = false;
     }
-    auto fields = [](auto& f) {
-        dfree(f.rv);
-        dfree(f.win);
-        dfree(f.rem);
-        dfree(f.ustar);
-        for (int b = 0; b < 2; ++b) {
-            dfree(f.P[b]);
-            dfree(f.Pa[b]);
-        }
-    };
-    fields(c->mpf);
-    fields(c->mpf32);
-    dfree(c->vtrace);
     c->mp_ready = false;
 }
 
 void free_tiles(lbx_ctx* c) {
-    dfree(c->mpt.info);
-    dfree(c->mpt.halo);
-    dfree(c->mpt.tab4);
-    dfree(c->mpt.tab2);
-    dfree(c->mpt.perm);
-    dfree(c->mpt.inv);
-    dfree(c->part);
+    give_block(&c->node_block);
+    give_block(&c->tile_block);
     c->mp_ntiles = 0;
 }
 
@@ -227,19 +262,8 @@ void free_all(lbx_ctx* c) {
     if (c->mpp.ctrl_h) (void)hipHostFree(c->mpp.ctrl_h);
     c->mpp.vt_h = nullptr;
     c->mpp.ctrl_h = nullptr;
-    dfree(c->f[0]);
-    dfree(c->f[1]);
-    dfree(c->g[0]);
-    dfree(c->g[1]);
-    dfree(c->j32);
-    dfree(c->j);
-    dfree(c->rho);
-    dfree(c->nodes);
-    dfree(c->map);
-    dfree(c->pulls);
-    dfree(c->slots);
-    dfree(c->ctrl);
-    dfree(c->l2ring);
+    give_block(&c->mp_block);
+    give_block(&c->lb_block);
     dfree(c->jpart);
     dfree(c->jflow);
     dfree(c->box);
@@ -596,6 +620,22 @@ void add_flow(lbx_ctx* c, Planes& s, double* rho_d, double* j_d, const double* r
         if (jp[a]) s.add(j_d + a * c->Np, jp[a]);
 }
 
+// the arrays of a geometry's MP tiles: by tile that it may use and packed node,
+// and by tile and entry
+template <typename Take>
+void node_arrays(lbx_ctx* c, uint64_t bound, Take&& take) {
+    take(c->mpt.info, bound);
+    take(c->mpt.inv, (uint64_t)c->Nf);
+}
+template <typename Take>
+void tile_arrays(lbx_ctx* c, uint64_t tiles, uint32_t pitch, Take&& take) {
+    take(c->mpt.perm, tiles * kMpTile);
+    take(c->mpt.halo, tiles * pitch);
+    take(c->mpt.tab4, tiles * kMpTile);
+    take(c->mpt.tab2, tiles * kMpTile);
+    take(c->part, 6 * (uint64_t)kMaxTracers * tiles);
+}
+
 // The MP tiles of the context's geometry: counted, grouped, placed and
 // tabled on the device (lbx_mp.h).  Tiles whose halo outgrows a brick's are
 // taken apart while the tile count stays within mp_tile_bound; beyond that
@@ -614,6 +654,7 @@ int build_tiles(lbx_ctx* c) {
     MpBuilt* db = nullptr;
     uint32_t *count = nullptr, *base = nullptr;
     uint8_t* split = nullptr;
+    Block scratch;
     MpBuilt h{};
     const uint32_t gw = (d.b.norder + kBlock / 64 - 1) / (kBlock / 64);
     MpTiles& t = c->mpt;
@@ -627,15 +668,7 @@ int build_tiles(lbx_ctx* c) {
     };
     auto table = [&](uint32_t pitch, uint8_t* sp) {
         if (st) return;
-        const uint64_t entries = (uint64_t)h.ntiles * kMpTile;
-        dfree(t.perm);
-        dfree(t.halo);
-        dfree(t.tab4);
-        dfree(t.tab2);
-        st = dalloc(&t.perm, entries);
-        if (!st) st = dalloc(&t.halo, (uint64_t)h.ntiles * pitch);
-        if (!st) st = dalloc(&t.tab4, entries);
-        if (!st) st = dalloc(&t.tab2, entries);
+        st = take_block(&c->tile_block, [&](auto&& take) { tile_arrays(c, h.ntiles, pitch, take); });
         if (st) return;
         t.pitch = pitch;
         hipLaunchKernelGGL(k_mpb_place, dim3(gw), dim3(kBlock), 0, s, dd, db, base, t.perm, t.inv);
@@ -645,13 +678,14 @@ int build_tiles(lbx_ctx* c) {
         if (!st) st = hip_status(hipMemcpyAsync(&h, db, sizeof(h), hipMemcpyDeviceToHost, s));
         if (!st) st = hip_status(hipStreamSynchronize(s));
     };
-    st = dalloc(&dd, 1);
-    if (!st) st = dalloc(&db, 1);
-    if (!st) st = dalloc(&count, d.b.norder);
-    if (!st) st = dalloc(&base, d.b.norder);
-    if (!st) st = dalloc(&split, d.bound);
-    if (!st) st = dalloc(&t.info, d.bound);
-    if (!st) st = dalloc(&t.inv, (uint64_t)c->Nf);
+    st = take_block(&scratch, [&](auto&& take) {
+        take(dd, (uint64_t)1);
+        take(db, (uint64_t)1);
+        take(count, (uint64_t)d.b.norder);
+        take(base, (uint64_t)d.b.norder);
+        take(split, (uint64_t)d.bound);
+    });
+    if (!st) st = take_block(&c->node_block, [&](auto&& take) { node_arrays(c, d.bound, take); });
     if (!st) st = hip_status(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
     if (!st) {
         hipLaunchKernelGGL(k_mpb_count, dim3(gw), dim3(kBlock), 0, s, dd, count);
@@ -669,12 +703,7 @@ int build_tiles(lbx_ctx* c) {
             }
         }
     }
-    if (!st) st = dalloc(&c->part, 6 * (uint64_t)kMaxTracers * h.ntiles);
-    dfree(dd);
-    dfree(db);
-    dfree(count);
-    dfree(base);
-    dfree(split);
+    give_block(&scratch);
     if (st) {
         free_tiles(c);
         return st;
@@ -694,20 +723,21 @@ double* const* mp_moments(lbx_ctx* c, bool adsorbed) {
     return adsorbed ? c->mpf.Pa : c->mpf.P;
 }
 
-// the arrays of a propagation of ntr tracers
-template <typename W>
-int alloc_fields(lbx_ctx* c, int ntr, bool any_ads, bool stored) {
+// the arrays of a propagation of ntr tracers on `tiles` tiles
+template <typename W, typename Take>
+void mp_arrays(lbx_ctx* c, int ntr, bool any_ads, bool stored, uint64_t tiles, Take&& take) {
     MpFields<W>& f = mp_fields<W>(c);
-    const uint64_t n = (uint64_t)c->mp_ntiles * kMpTile;
-    int st = stored ? dalloc(&f.win, 9 * n) : dalloc(&f.rv, 2 * n);
-    if (!st) st = dalloc(&f.rem, n);
-    if (!st) st = dalloc(&f.ustar, 3 * n);
+    f = MpFields<W>{};
+    const uint64_t n = tiles * kMpTile;
+    if (stored) take(f.win, 9 * n); else take(f.rv, 2 * n);
+    take(f.rem, n);
+    take(f.ustar, 3 * n);
     for (int b = 0; b < 2; ++b) {
-        if (!st) st = dalloc(&f.P[b], 3 * (uint64_t)ntr * n);
+        take(f.P[b], 3 * (uint64_t)ntr * n);
         // Pa of a tracer without adsorption is never read or written
-        if (!st && any_ads) st = dalloc(&f.Pa[b], 3 * (uint64_t)ntr * n);
+        if (any_ads) take(f.Pa[b], 3 * (uint64_t)ntr * n);
     }
-    return st;
+    take(c->vtrace, 3 * (uint64_t)ntr * kMpChunk);
 }
 
 template <int T, typename W>
@@ -847,6 +877,28 @@ int lbx_d3q19_tables(int32_t c[57], double a0o[19], double a1o[19], double a2o[1
     return LBX_OK;
 }
 
+}  // extern "C"
+
+namespace {
+// the arrays of the LB phase
+template <typename Take>
+void lb_arrays(lbx_ctx* c, Take&& take) {
+    for (int b = 0; b < 2; ++b)
+        if (f32_storage(c->prec)) take(c->g[b], kQ * c->Np); else take(c->f[b], kQ * c->Np);
+    if (c->prec == LBX_PREC_FP32_SHIFT) take(c->j32, 3 * c->Np);
+    take(c->j, 3 * c->Np);
+    take(c->rho, c->Np);
+    take(c->nodes, (uint64_t)c->Nf);
+    take(c->map, (uint64_t)c->N);
+    if (c->Nf <= kTabNodes) take(c->pulls, 18 * c->Np);
+    take(c->slots, (uint64_t)(3 * kSlots));
+    take(c->ctrl, (uint64_t)1);
+    take(c->l2ring, (uint64_t)kRing);
+}
+}  // namespace
+
+extern "C" {
+
 int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precision, int32_t with_mp) {
     if (lx <= 0 || ly <= 0 || lz <= 0) return -1;
     // upper bound: every node fluid
@@ -912,19 +964,7 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     // together exceed the 256 MiB last-level cache, no written line survives
     // there to the next step
     c->nt = 2 * kQ * c->Np * (shift ? sizeof(float) : sizeof(double)) > (uint64_t)LBX_NT_MIN_BYTES;
-    if (!st && !shift) st = dalloc(&c->f[0], kQ * c->Np);
-    if (!st && !shift) st = dalloc(&c->f[1], kQ * c->Np);
-    if (!st && shift) st = dalloc(&c->g[0], kQ * c->Np);
-    if (!st && shift) st = dalloc(&c->g[1], kQ * c->Np);
-    if (!st && precision == LBX_PREC_FP32_SHIFT) st = dalloc(&c->j32, 3 * c->Np);
-    if (!st) st = dalloc(&c->j, 3 * c->Np);
-    if (!st) st = dalloc(&c->rho, c->Np);
-    if (!st) st = dalloc(&c->nodes, (uint64_t)c->Nf);
-    if (!st) st = dalloc(&c->map, (uint64_t)c->N);
-    if (!st && c->Nf <= kTabNodes) st = dalloc(&c->pulls, 18 * c->Np);
-    if (!st) st = dalloc(&c->slots, 3 * kSlots);
-    if (!st) st = dalloc(&c->ctrl, 1);
-    if (!st) st = dalloc(&c->l2ring, kRing);
+    if (!st) st = take_block(&c->lb_block, [&](auto&& take) { lb_arrays(c, take); });
     if (!st && (hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
     uint32_t nfi = 0;
@@ -1267,11 +1307,14 @@ static int mp_setup(lbx_ctx* c, const double fext[3], double Db, int32_t ntr, co
     }
     LBX_TRY(build_tiles(c));
     const bool stored = mp_stored(c, ntr);
-    int st = f32_storage(c->prec) ? alloc_fields<float>(c, ntr, any_ads, stored)
-                                  : alloc_fields<double>(c, ntr, any_ads, stored);
-    if (!st) st = dalloc(&c->vtrace, 3 * (uint64_t)ntr * kMpChunk);
-    if (st) {
-        free_mp(c);
+    const auto lay = [&](auto&& take) {
+        if (f32_storage(c->prec))
+            mp_arrays<float>(c, ntr, any_ads, stored, c->mp_ntiles, take);
+        else
+            mp_arrays<double>(c, ntr, any_ads, stored, c->mp_ntiles, take);
+    };
+    if (const int st = take_block(&c->mp_block, lay)) {
+        give_block(&c->mp_block);
         return st;
     }
     LBX_TRY(reset_ctrl(c));
