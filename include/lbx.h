@@ -140,9 +140,10 @@ int lbx_supercell_xsf(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, 
 
 /* --------------------------------------------------------------- context */
 
-/* HBM bytes a context of this shape needs (admission control for batching
- * and serving); with_mp > 0 adds the moment-propagation arrays of that many
- * tracers (lbx_mp_init_batch). */
+/* HBM bytes that a context of this shape needs at most (admission control for
+ * batching and serving; all nodes fluid); with_mp > 0 adds the
+ * moment-propagation arrays of that many tracers (lbx_mp_init_batch), with
+ * adsorption and in the form that takes most (LBX_MP_STORED). */
 int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precision, int32_t with_mp);
 
 /* Create a context on the current HIP device holding one lattice: nature

@@ -901,18 +901,26 @@ extern "C" {
 
 int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precision, int32_t with_mp) {
     if (lx <= 0 || ly <= 0 || lz <= 0) return -1;
-    // upper bound: every node fluid
-    const uint64_t N = (uint64_t)lx * ly * lz, Np = (N + 63) / 64 * 64;
-    const uint64_t pop = f32_storage(precision) ? 4 : 8;  // populations; also win and u* of moment propagation
-    uint64_t b = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + N * 8 +
-                 18 * 4 * std::min<uint64_t>(Np, (kTabNodes + 63) / 64 * 64) +
-                 box_values(N) * 8ull + sizeof(Ctrl) + kRing * 8;
-    if (with_mp > 0) {  // with_mp tracers, each with adsorption (the upper bound)
-        const uint64_t T = (uint64_t)std::min(with_mp, kMaxTracers);
+    // upper bound: every node fluid, and the pull table of a box with fewer; with_mp tracers, each
+    // adsorbing, their probabilities stored, on the tiles of the general layout's wider halo lists
+    lbx_ctx c;
+    c.prec = precision;
+    c.N = c.Nf = (uint32_t)((uint64_t)lx * ly * lz);
+    c.Np = ((uint64_t)c.Nf + 63) / 64 * 64;
+    uint64_t b = block_bytes([&](auto&& take) { lb_arrays(&c, take); }) + box_values(c.N) * 8ull;
+    if (c.Nf > kTabNodes) b += 18 * 4 * (uint64_t)kTabNodes;
+    if (with_mp > 0) {
+        const int T = std::min(with_mp, kMaxTracers);
         const Bricks br = make_bricks((uint32_t)lx, (uint32_t)ly, (uint32_t)lz);
-        const uint64_t tiles = std::min<uint64_t>((uint64_t)br.nbx * br.nby * br.nbz, mp_tile_bound((uint32_t)N));
-        b += tiles * kMpTile * (4 * 8 + 8 + 3 * pop + 24 + 4 + 12 * T * 8) + tiles * (kHaloMax * 4 + 6 * kMaxTracers * 8) +
-             Np * 4 + kMpChunk * 3 * T * 8;
+        const uint64_t bound = mp_tile_bound(c.Nf), tiles = std::min<uint64_t>((uint64_t)br.nbx * br.nby * br.nbz, bound);
+        b += block_bytes([&](auto&& take) { node_arrays(&c, bound, take); }) +
+             block_bytes([&](auto&& take) { tile_arrays(&c, tiles, kHaloMaxGen, take); }) +
+             block_bytes([&](auto&& take) {
+                 if (f32_storage(precision))
+                     mp_arrays<float>(&c, T, true, true, tiles, take);
+                 else
+                     mp_arrays<double>(&c, T, true, true, tiles, take);
+             });
     }
     return (int64_t)b;
 }
