@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "../../include/lbx.h"
+#include "lbx_block.h"
 #include "lbx_device.h"
 #include "lbx_kernels.h"
 #include "lbx_mp.h"
@@ -420,37 +421,6 @@ __global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void kb_mp_round(BatchMpView
 
 // ------------------------------------------------------------------ host
 
-int hip_status(hipError_t e) {
-    if (e == hipSuccess) return LBX_OK;
-    (void)hipGetLastError();
-    return e == hipErrorOutOfMemory ? LBX_ERR_NOMEM : LBX_ERR_DEVICE;
-}
-int hip_status(int st) { return st; }
-
-#define LBX_TRY(expr)                            \
-    do {                                         \
-        int _st = hip_status(expr);              \
-        if (_st != LBX_OK) return _st;           \
-    } while (0)
-
-template <typename T>
-int dalloc(T** p, uint64_t count) {
-    *p = nullptr;
-    if (count == 0) return LBX_OK;
-    hipError_t e = hipMalloc((void**)p, count * sizeof(T));
-    if (e != hipSuccess) {
-        *p = nullptr;
-        (void)hipGetLastError();
-        return e == hipErrorOutOfMemory ? LBX_ERR_NOMEM : LBX_ERR_DEVICE;
-    }
-    return LBX_OK;
-}
-template <typename T>
-void dfree(T*& p) {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-}
-
 // first-fit allocator of [0, cap) in units
 struct RangeAlloc {
     std::map<uint64_t, uint64_t> free_;  // start -> length
@@ -545,8 +515,8 @@ struct lbxb {
     uint32_t* mp_tile_inst = nullptr;
     MpFields<double> mpf;        // FP64 form
     MpFields<float> mpf32;       // FP32-storage forms
-    uint32_t* walk = nullptr;    // scratch of the layout builds, grown as needed
-    uint64_t walk_cap = 0;
+    uint32_t *walk_count = nullptr, *walk_base = nullptr;  // scratch of the layout builds, grown as needed
+    Block block, walk_block;     // the allocations: all arrays above and below, the scratch
     uint32_t* ids = nullptr;     // [max instances]
     // admissions go through two pinned buffers in turn (kStage bytes each)
     char* stage[2] = {nullptr, nullptr};
@@ -591,57 +561,14 @@ void clear_graphs(lbxb* b) {
 
 void free_all(lbxb* b) {
     clear_graphs(b);
-    for (int k = 0; k < 2; ++k) {
-        dfree(b->f[k]);
-        dfree(b->g[k]);
-        dfree(b->part[k]);
-    }
-    dfree(b->j32);
-    dfree(b->j);
-    dfree(b->rho);
-    dfree(b->nodes);
-    dfree(b->maps);
-    dfree(b->tile_inst);
-    dfree(b->nature);
-    dfree(b->counts);
-    dfree(b->nfi);
-    dfree(b->act[0]);
-    dfree(b->act[1]);
-    dfree(b->insts);
-    dfree(b->slots);
-    dfree(b->l2ring);
-    dfree(b->ctrl);
-    auto fields = [](auto& f) {
-        dfree(f.rv);
-        dfree(f.win);
-        dfree(f.rem);
-        dfree(f.ustar);
-        for (int k = 0; k < 2; ++k) {
-            dfree(f.P[k]);
-            dfree(f.Pa[k]);
-        }
-    };
-    fields(b->mpf);
-    fields(b->mpf32);
-    dfree(b->mpt.info);
-    dfree(b->mpt.halo);
-    dfree(b->mpt.tab4);
-    dfree(b->mpt.tab2);
-    dfree(b->mpt.perm);
-    dfree(b->mpt.inv);
-    dfree(b->mp_tile_inst);
-    dfree(b->walk);
-    dfree(b->builds);
-    dfree(b->built);
-    dfree(b->split);
-    dfree(b->ids);
+    give_block(&b->block);
+    give_block(&b->walk_block);
     for (int k = 0; k < 2; ++k) {
         if (b->stage[k]) (void)hipHostFree(b->stage[k]);
         if (b->stage_ev[k]) (void)hipEventDestroy(b->stage_ev[k]);
         b->stage[k] = nullptr;
         b->stage_ev[k] = nullptr;
     }
-    dfree(b->vtrace);
     for (auto& e : b->ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
     if (b->stream) (void)hipStreamDestroy(b->stream), b->stream = nullptr;
@@ -931,13 +858,11 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         d.bound = mp_tile_bound(h.Nf);  // 2 in.ntiles
         walk += d.b.norder;
     }
-    if (walk > b->walk_cap) {  // counts and bases
-        dfree(b->walk);
-        b->walk_cap = 0;
-        LBX_TRY(dalloc(&b->walk, 2 * walk));
-        b->walk_cap = walk;
-    }
-    uint32_t *count = b->walk, *base = b->walk + walk;
+    LBX_TRY(take_block(&b->walk_block, [&](auto&& take) {
+        take(b->walk_count, walk);
+        take(b->walk_base, walk);
+    }, true));
+    uint32_t *count = b->walk_count, *base = b->walk_base;
     // one pass over the lattices `which`; general: keep what has an LDS slot
     auto pass = [&](const std::vector<size_t>& which, bool counted, const uint8_t* by, uint8_t* mark,
                     bool general) -> int {
@@ -1060,6 +985,67 @@ int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
     return LBX_OK;
 }
 
+void set_capacity(lbxb* b, int32_t precision, int64_t nodes, int64_t box, int32_t instances) {
+    b->prec = precision;
+    b->Np = ((uint64_t)nodes + kTile - 1) / kTile * kTile;
+    b->cap_box = (uint64_t)box;
+    b->cap_inst = (uint32_t)instances;
+    b->ntiles_cap = (uint32_t)(b->Np / kTile);
+    b->mpt.pitch = kHaloMaxGen;
+}
+
+// all device arrays of a batch
+template <typename Take>
+void batch_arrays(lbxb* b, Take&& take) {
+    const uint64_t Np = b->Np, tiles = b->ntiles_cap, ni = b->cap_inst;
+    const uint64_t M = 2 * Np;  // entries of the MP tiles
+    for (int k = 0; k < 2; ++k)
+        if (shift(b)) take(b->g[k], kQ * Np); else take(b->f[k], kQ * Np);
+    if (b->prec == LBX_PREC_FP32_SHIFT) take(b->j32, 3 * Np);
+    take(b->j, 3 * Np);
+    take(b->rho, Np);
+    take(b->nodes, Np);
+    take(b->maps, b->cap_box);
+    take(b->tile_inst, tiles);
+    take(b->nature, (b->cap_box + 15) / 16 * 16);
+    take(b->counts, (uint64_t)node_chunks(b->cap_box));
+    take(b->nfi, ni);
+    take(b->act[0], tiles);
+    take(b->act[1], 2 * tiles);
+    take(b->insts, ni);
+    take(b->slots, ni * 3 * kSlots);
+    take(b->l2ring, ni * kRing);
+    take(b->ctrl, ni);
+    const auto fields = [&](auto& f) {
+        take(f.rem, M);
+        take(f.ustar, 3 * M);
+        for (int k = 0; k < 2; ++k) {
+            take(f.P[k], 3 * M);
+            take(f.Pa[k], 3 * M);
+        }
+    };
+    if (shift(b)) {
+        fields(b->mpf32);
+        take(b->mpf32.win, 9 * M);
+    } else {
+        fields(b->mpf);
+        take(b->mpf.rv, 2 * M);
+    }
+    for (int k = 0; k < 2; ++k) take(b->part[k], 2 * tiles * 3);
+    take(b->mpt.info, M / kTile);
+    take(b->mpt.halo, M / kTile * b->mpt.pitch);
+    take(b->mpt.tab4, M);
+    take(b->mpt.tab2, M);
+    take(b->mpt.perm, M);
+    take(b->mpt.inv, Np);
+    take(b->mp_tile_inst, M / kTile);
+    take(b->split, M / kTile);
+    take(b->builds, ni);
+    take(b->built, ni);
+    take(b->ids, ni);
+    take(b->vtrace, (uint64_t)kRoundMax * ni * 3);
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------ C-ABI
@@ -1068,18 +1054,9 @@ extern "C" {
 
 int64_t lbxb_footprint_bytes(int32_t precision, int64_t capacity_nodes, int64_t capacity_box, int32_t max_instances) {
     if (capacity_nodes <= 0 || capacity_box <= 0 || max_instances <= 0) return -1;
-    const uint64_t Np = ((uint64_t)capacity_nodes + kTile - 1) / kTile * kTile;
-    const uint64_t pop = (precision == LBX_PREC_FP32_SHIFT || precision == LBX_PREC_FP32_STORE) ? 4 : 8;
-    uint64_t by = 2 * kQ * Np * pop + (precision == LBX_PREC_FP32_SHIFT ? 3 * Np * 4 : 0) + 4 * Np * 8 + Np * 4 +
-                  (uint64_t)capacity_box * 5 + node_chunks((uint64_t)capacity_box) * 4ull + Np / kTile * 4;
-    by += (uint64_t)max_instances * (4 + sizeof(BInst) + 3 * kSlots * 8 + kRing * 8 + sizeof(Ctrl));
-    // MP: twice the nodes' entries (probabilities or (rho, v), rem, u*, P and Pa twice, slot table, node),
-    // halo lists, partials, each node's entry
-    const uint64_t M = 2 * Np;
-    by += M * ((pop == 8 ? 4 * 8 : 18 * 4) + 8 + 3 * pop + 4 * 3 * 8 + 24 + 4) +
-          M / kTile * (kHaloMaxGen * 4 + 2 * 3 * 8 + 3 * 4 + 1) + Np * 4;
-    by += (uint64_t)kRoundMax * max_instances * 3 * 8;
-    return (int64_t)by;
+    lbxb b;
+    set_capacity(&b, precision, capacity_nodes, capacity_box, max_instances);
+    return (int64_t)block_bytes([&](auto&& take) { batch_arrays(&b, take); });
 }
 
 int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box, int32_t max_instances,
@@ -1093,11 +1070,7 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
     if (kQ * Np >= (1ull << 32) || (uint64_t)capacity_box >= (1ull << 32)) return LBX_ERR_ARG;
     lbxb* b = new (std::nothrow) lbxb();
     if (!b) return LBX_ERR_NOMEM;
-    b->prec = precision;
-    b->Np = Np;
-    b->cap_box = (uint64_t)capacity_box;
-    b->cap_inst = (uint32_t)max_instances;
-    b->ntiles_cap = (uint32_t)(Np / kTile);
+    set_capacity(b, precision, capacity_nodes, capacity_box, max_instances);
     // 32-bit byte offsets reach every array while the populations (the
     // largest: 19 per node, FP64 or FP32 by form) stay below 4 GiB
     b->wide = b->wide_auto =
@@ -1107,62 +1080,13 @@ int lbxb_create(int32_t precision, int64_t capacity_nodes, int64_t capacity_box,
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&b->num_cu, hipDeviceAttributeMultiprocessorCount, dev);
     }
-    const bool sh = precision == LBX_PREC_FP32_SHIFT || precision == LBX_PREC_FP32_STORE;
     int st = LBX_OK;
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) st = LBX_ERR_DEVICE;
-    for (int k = 0; k < 2; ++k) {
-        if (!st && !sh) st = dalloc(&b->f[k], kQ * Np);
-        if (!st && sh) st = dalloc(&b->g[k], kQ * Np);
-        if (!st) st = dalloc(&b->part[k], 2 * (uint64_t)b->ntiles_cap * 3);
-    }
-    if (!st && precision == LBX_PREC_FP32_SHIFT) st = dalloc(&b->j32, 3 * Np);
-    if (!st) st = dalloc(&b->j, 3 * Np);
-    if (!st) st = dalloc(&b->rho, Np);
-    if (!st) st = dalloc(&b->nodes, Np);
-    if (!st) st = dalloc(&b->maps, (uint64_t)capacity_box);
-    if (!st) st = dalloc(&b->tile_inst, (uint64_t)b->ntiles_cap);
-    if (!st) st = dalloc(&b->nature, ((uint64_t)capacity_box + 15) / 16 * 16);
-    if (!st) st = dalloc(&b->counts, (uint64_t)node_chunks((uint64_t)capacity_box));
-    if (!st) st = dalloc(&b->nfi, (uint64_t)max_instances);
-    if (!st) st = dalloc(&b->act[0], (uint64_t)b->ntiles_cap);
-    if (!st) st = dalloc(&b->act[1], 2 * (uint64_t)b->ntiles_cap);
-    if (!st) st = dalloc(&b->insts, (uint64_t)max_instances);
-    if (!st) st = dalloc(&b->slots, (uint64_t)max_instances * 3 * kSlots);
-    if (!st) st = dalloc(&b->l2ring, (uint64_t)max_instances * kRing);
-    if (!st) st = dalloc(&b->ctrl, (uint64_t)max_instances);
-    const uint64_t M = 2 * Np;  // entries of the MP tiles
-    auto fields = [&](auto& f) {
-        if (!st) st = dalloc(&f.rem, M);
-        if (!st) st = dalloc(&f.ustar, 3 * M);
-        for (int k = 0; k < 2; ++k) {
-            if (!st) st = dalloc(&f.P[k], 3 * M);
-            if (!st) st = dalloc(&f.Pa[k], 3 * M);
-        }
-    };
-    if (sh) {
-        fields(b->mpf32);
-        if (!st) st = dalloc(&b->mpf32.win, 9 * M);
-    } else {
-        fields(b->mpf);
-        if (!st) st = dalloc(&b->mpf.rv, 2 * M);
-    }
-    b->mpt.pitch = kHaloMaxGen;
-    if (!st) st = dalloc(&b->mpt.info, M / kTile);
-    if (!st) st = dalloc(&b->mpt.halo, M / kTile * b->mpt.pitch);
-    if (!st) st = dalloc(&b->mpt.tab4, M);
-    if (!st) st = dalloc(&b->mpt.tab2, M);
-    if (!st) st = dalloc(&b->mpt.perm, M);
-    if (!st) st = dalloc(&b->mpt.inv, Np);
-    if (!st) st = dalloc(&b->mp_tile_inst, M / kTile);
-    if (!st) st = dalloc(&b->split, M / kTile);
-    if (!st) st = dalloc(&b->builds, (uint64_t)max_instances);
-    if (!st) st = dalloc(&b->built, (uint64_t)max_instances);
-    if (!st) st = dalloc(&b->ids, (uint64_t)max_instances);
+    if (!st) st = take_block(&b->block, [&](auto&& take) { batch_arrays(b, take); });
     for (int k = 0; k < 2; ++k) {
         if (!st) st = hip_status(hipHostMalloc((void**)&b->stage[k], kStage));
         if (!st) st = hip_status(hipEventCreateWithFlags(&b->stage_ev[k], hipEventDisableTiming));
     }
-    if (!st) st = dalloc(&b->vtrace, (uint64_t)kRoundMax * max_instances * 3);
     if (!st && (hipEventCreate(&b->ev[0]) != hipSuccess || hipEventCreate(&b->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
     if (!st) {
