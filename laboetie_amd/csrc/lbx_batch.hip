@@ -524,7 +524,8 @@ struct lbxb {
     int stage_at = 0;
     MpBuild* builds = nullptr;   // [max instances]
     MpBuilt* built = nullptr;
-    uint8_t* split = nullptr;
+    uint8_t* split = nullptr;    // layout builds: parts of each tile (log2), the tile that each is part of
+    uint32_t* owner = nullptr;
     double* part[2] = {nullptr, nullptr};
     double* vtrace = nullptr;
     // host state
@@ -863,8 +864,9 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         take(b->walk_base, walk);
     }, true));
     uint32_t *count = b->walk_count, *base = b->walk_base;
-    // one pass over the lattices `which`; general: keep what has an LDS slot
-    auto pass = [&](const std::vector<size_t>& which, bool counted, const uint8_t* by, uint8_t* mark,
+    // one pass over the lattices `which`: tiles cut by `by`, `mark` for the next
+    // pass; general: keep what has an LDS slot
+    auto pass = [&](const std::vector<size_t>& which, const uint8_t* by, uint8_t* mark, uint32_t level,
                     bool general) -> int {
         std::vector<MpBuild> d;
         uint32_t gw = 0, gt = 0;
@@ -875,14 +877,14 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         }
         const uint32_t nd = (uint32_t)d.size();
         LBX_TRY(hipMemcpyAsync(b->builds, d.data(), nd * sizeof(MpBuild), hipMemcpyHostToDevice, b->stream));
-        if (!counted)
+        if (level == 1)
             hipLaunchKernelGGL(k_mpb_count, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, count);
         hipLaunchKernelGGL(k_mpb_group, dim3(nd), dim3(kBlock), 0, b->stream, b->builds, b->built, count, base,
-                           b->mpt.info, by);
+                           b->mpt.info, by, b->owner);
         hipLaunchKernelGGL(k_mpb_place, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, b->built, base,
                            b->mpt.perm, b->mpt.inv);
         hipLaunchKernelGGL((general ? k_mpb_table<true> : k_mpb_table<false>), dim3(gt, nd), dim3(kBlock), 0,
-                           b->stream, b->builds, b->built, b->mpt, mark);
+                           b->stream, b->builds, b->built, b->mpt, b->owner, mark, level);
         LBX_TRY(hipGetLastError());
         std::vector<MpBuilt> r(nd);
         LBX_TRY(hipMemcpyAsync(r.data(), b->built, nd * sizeof(MpBuilt), hipMemcpyDeviceToHost, b->stream));
@@ -892,15 +894,21 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
     };
     std::vector<size_t> all, again, gen;
     for (size_t k = 0; k < ids.size(); ++k) all.push_back(k);
-    LBX_TRY(pass(all, false, nullptr, b->split, false));
+    LBX_TRY(pass(all, nullptr, b->split, 1, false));
     for (size_t k : all)
         if (built[k].halo_max > kHaloMax) again.push_back(k);
-    if (!again.empty()) {
-        LBX_TRY(pass(again, true, b->split, nullptr, false));
-        for (size_t k : again)
-            if (built[k].ntiles == 0) gen.push_back(k);
-        if (!gen.empty()) LBX_TRY(pass(gen, true, nullptr, nullptr, true));
+    for (uint32_t level = 2; !again.empty(); ++level) {
+        LBX_TRY(pass(again, b->split, b->split, level, false));
+        std::vector<size_t> more;
+        for (size_t k : again) {
+            if (built[k].ntiles == 0)
+                gen.push_back(k);
+            else if (built[k].halo_max > kHaloMax)
+                more.push_back(k);
+        }
+        again.swap(more);
     }
+    if (!gen.empty()) LBX_TRY(pass(gen, nullptr, nullptr, 0, true));
     for (size_t k = 0; k < ids.size(); ++k) {
         BInst& in = b->tab[ids[k]];
         in.mp_tile0 = 2 * in.tile_first;
@@ -1040,6 +1048,7 @@ void batch_arrays(lbxb* b, Take&& take) {
     take(b->mpt.inv, Np);
     take(b->mp_tile_inst, M / kTile);
     take(b->split, M / kTile);
+    take(b->owner, M / kTile);
     take(b->builds, ni);
     take(b->built, ni);
     take(b->ids, ni);

@@ -1,7 +1,7 @@
 // Moment propagation of liblbx on tiles of spatially compact nodes, shared by
 // the single-lattice path (lbx.hip) and the batch engine (lbx_batch.hip).
 //
-// The box is cut into bricks of at most 256 box nodes (8 x 8 x 4 where the
+// The box is cut into bricks of at most 256 box nodes (8 x 4 x 8 where the
 // box allows it).  A tile is one 256-thread block's share: the fluid nodes of
 // one brick, or of consecutive bricks together while they hold at most 256.
 // A node's 18 neighbours then lie in its own tile or in the shell around its
@@ -31,7 +31,7 @@ constexpr uint32_t kMpTile = 256;                // nodes (and threads) of a til
 constexpr uint32_t kZeroSlot = 256;              // LDS slot of the solid neighbour: P = 0
 constexpr uint32_t kHalo0 = 257;                 // LDS slot of the first halo node
 constexpr uint32_t kFarSlot = 1023;              // neighbour without an LDS slot (general tiles only)
-constexpr uint32_t kHaloMax = 344;               // halo nodes of one brick at most (shell of 8 x 8 x 4)
+constexpr uint32_t kHaloMax = 344;               // halo nodes of one brick at most (shell of 8 x 4 x 8)
 constexpr uint32_t kHaloMaxGen = kFarSlot - kHalo0;  // halo nodes of a general tile at most
 constexpr uint32_t kSlots1 = 608;                // LDS slots of a tile with at most kHaloMax halo nodes
 constexpr uint32_t kSlotsGen = 1024;
@@ -39,7 +39,7 @@ constexpr uint32_t kTabInterfacial = 1u << 31;   // table bits: the node is inte
 constexpr uint32_t kTabNode = 1u << 30;          // the entry holds a node
 static_assert(kHalo0 + kHaloMax <= kSlots1, "slots of a brick tile");
 constexpr int kPace = 3;                         // neighbours whose LDS reads are in flight together
-constexpr uint32_t kColumn = 8;                  // bricks are walked in columns of 8 x 8 along z
+constexpr uint32_t kColumn = 8;                  // bricks are walked in columns of 8 by 8 bricks along z
 
 // A lattice's cut into bricks.
 struct Bricks {
@@ -159,42 +159,42 @@ __global__ __launch_bounds__(kBlock) void k_mpb_count(const MpBuild* __restrict_
 
 // Bricks into tiles, in walk order: a brick joins the current tile while the
 // tile holds at most 256 nodes.  base[o] = entry of the brick's first node.
-// split != NULL: the tiles it marks (numbered as the call without it numbers
-// them) are taken apart into their bricks.  One block per lattice; a thread
+// split != NULL: tile k of the call without it is cut into 2^split[k] parts, by
+// the place of each brick's first node in it (256 parts: every brick alone),
+// and owner[t] is the k that tile t is part of.  One block per lattice; a thread
 // groups whole runs of kRun bricks, so tiles end at the runs' ends (under 1%
 // of a tile's fill), unless that takes more tiles than the lattice may use:
 // then one thread groups all bricks (one thread's walk of a 256^3 medium's
 // 65 536 bricks took 15 ms).
 constexpr uint32_t kRun = 128;
 
-// f(o, nodes, tile of the run, nodes of the tile before it) per brick with
-// nodes; returns the run's tiles.  split: of the lattice's tiles, those of the
-// unsplit run beginning at old0.
+// f(o, nodes, tile of the run, nodes of the tile before it, unsplit tile) per
+// brick with nodes; returns the run's tiles.  The unsplit run's tiles begin at
+// old0.
 template <typename F>
 __device__ __forceinline__ uint32_t group_run(const uint32_t* __restrict__ count, uint32_t o0, uint32_t o1,
                                               const uint8_t* __restrict__ split, uint32_t old0, F&& f) {
-    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0;
-    bool any = false, was = false;
+    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0, part = 0;
+    bool any = false;
     for (uint32_t o = o0; o < o1; ++o) {
         const uint32_t c = count[o];
         if (c == 0) continue;
-        bool cut = acc + c > kMpTile;
-        if (split) {
-            if (old_acc + c > kMpTile) {
-                ++old;
-                old_acc = 0;
-                cut = true;
-            }
-            old_acc += c;
-            const bool is = split[old0 + old] != 0;
-            cut = cut || (any && (is || was));
-            was = is;
+        bool cut = old_acc + c > kMpTile;
+        if (cut) {
+            ++old;
+            old_acc = 0;
         }
+        if (split) {
+            const uint32_t p = (old_acc << split[old0 + old]) >> 8;
+            cut = cut || (any && p != part);
+            part = p;
+        }
+        old_acc += c;
         if (cut) {
             ++tile;
             acc = 0;
         }
-        f(o, c, tile, acc);
+        f(o, c, tile, acc, old0 + old);
         acc += c;
         any = true;
     }
@@ -203,7 +203,8 @@ __device__ __forceinline__ uint32_t group_run(const uint32_t* __restrict__ count
 
 __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict__ builds, MpBuilt* built,
                                                       const uint32_t* __restrict__ counts, uint32_t* base,
-                                                      uint32_t* info, const uint8_t* __restrict__ split) {
+                                                      uint32_t* info, const uint8_t* __restrict__ split,
+                                                      uint32_t* owner) {
     __shared__ uint32_t sums[kBlock + 1];
     const MpBuild& d = builds[blockIdx.x];
     const uint32_t* count = counts + d.order_off;
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
         __syncthreads();
         return sums[threadIdx.x];
     };
-    const auto none = [](uint32_t, uint32_t, uint32_t, uint32_t) {};
+    const auto none = [](uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) {};
     uint32_t old0 = 0;
     for (int pass = 0; pass < 2; ++pass) {
         const uint32_t nruns = (n + run - 1) / run;
@@ -258,11 +259,14 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
     uint32_t old = old0;
     for (uint32_t r = r0; r < r1; ++r) {
         const uint32_t o0 = r * run, o1 = min(n, (r + 1) * run), t0 = d.tile0 + tile0;
-        tile0 += group_run(count, o0, o1, split, d.tile0 + old, [&](uint32_t o, uint32_t c, uint32_t tile, uint32_t acc) {
-            base[d.order_off + o] = (t0 + tile) * kMpTile + acc;
-            info[t0 + tile] = acc + c;
-        });
-        if (split) old += group_run(count, o0, o1, nullptr, 0, none);
+        const uint32_t k = group_run(count, o0, o1, split, d.tile0 + old,
+                                     [&](uint32_t o, uint32_t c, uint32_t tile, uint32_t acc, uint32_t was) {
+                                         base[d.order_off + o] = (t0 + tile) * kMpTile + acc;
+                                         info[t0 + tile] = acc + c;
+                                         owner[t0 + tile] = was;
+                                     });
+        tile0 += k;
+        old += split ? group_run(count, o0, o1, nullptr, 0, none) : k;
     }
 }
 
@@ -287,12 +291,14 @@ __global__ __launch_bounds__(kBlock) void k_mpb_place(const MpBuild* __restrict_
 // Halo list and slot table of every tile (grid x: a lattice's tiles, y:
 // lattices).  The distinct outside neighbours are collected in an LDS hash
 // table and sorted, so that consecutive slots read consecutive entries.
-// split (may be NULL) receives 1 for a tile with more than kHaloMax.
-// A table of 1024 places is enough to tell a tile that must be taken apart;
-// the general tiles keep up to kHaloMaxGen of theirs.
+// split[owner] (split may be NULL) receives `level` for a tile with more than
+// kHaloMax halo nodes, and in the first pass (level 1, owners their own tiles)
+// 0 for every other.  A table of 1024 places is enough to tell a tile that must
+// be cut; the general tiles keep up to kHaloMaxGen of theirs.
 template <bool GEN>
 __global__ __launch_bounds__(kBlock) void k_mpb_table(const MpBuild* __restrict__ builds, MpBuilt* built, MpTiles t,
-                                                      uint8_t* split) {
+                                                      const uint32_t* __restrict__ owner, uint8_t* split,
+                                                      uint32_t level) {
     constexpr uint32_t kHashSize = GEN ? 4096 : 1024, kHashMax = GEN ? 2048 : 512;
     static_assert(kHashMax + 2 * kMpTile <= kHashSize && kHashMax > kHaloMax, "room to stop inserting");
     __shared__ uint32_t key[kHashSize];
@@ -366,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void k_mpb_table(const MpBuild* __restrict_
     t.tab4[e] = make_uint4(w[0], w[1], w[2], w[3]);
     t.tab2[e] = make_uint2(w[4], w[5]);
     if (threadIdx.x == 0) {
-        if (split) split[tile] = n > kHaloMax ? 1 : 0;
+        if (split && (n > kHaloMax || level == 1)) split[owner[tile]] = n > kHaloMax ? (uint8_t)level : 0;
         atomicMax(&built[blockIdx.y].halo_max, n);
     }
 }
