@@ -790,8 +790,8 @@ int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
     return hip_status(hipGraphLaunch(it->second.exec, b->stream));
 }
 
-// One phase of a round as a single cooperative launch (grid: as many blocks as
-// can be resident at once, at most one per tile)
+// One phase of a round as a single cooperative launch (grid: blocks that are
+// resident at once, at most one per tile)
 int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
     if (S <= 0) return LBX_OK;
     uint32_t nt = grid_of(b, b->lb_block, phase), ni = b->cap_inst;
@@ -800,6 +800,11 @@ int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
         int per_cu = 0;
         LBX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, 0));
         if (per_cu <= 0) return LBX_ERR_DEVICE;
+        // 8 waves a CU: the grid barrier's time grows with the blocks, faster than more of them
+        // save.  LB + MP us per step of 256-thread blocks, all that fit / 2 / 1 a CU: six 96^3 media
+        // FP64 538 + 298 / 421 + 267 / 454 + 358, FP32-shift 567 + 327 / 340 + 248 / 389 + 279;
+        // 64 cells 1x100x100 FP64 185 + 143 / 117 + 86 / 94 + 77
+        per_cu = std::min(per_cu, 512 / block);
         const uint32_t grid = std::min<uint32_t>(nt, (uint32_t)per_cu * (uint32_t)b->num_cu);
         return hip_status(hipLaunchCooperativeKernel((const void*)kern, dim3(grid), dim3(block), args, 0, b->stream));
     };
