@@ -75,6 +75,7 @@ struct BInst {
     int64_t mp_it0, mp_n;         // launch k runs MP step mp_it0 + k + 1 while k < mp_n
     int32_t mp_repeat;            // every launch recomputes step mp_it0 + 1 (timing)
     uint32_t mp_tile0, mp_ntiles; // its MP tiles
+    int32_t mp_general;           // its MP steps need the general kernel (lbx_mp.h)
     double lambda;
     TracerParams tp;
     // set-up of its moment propagation: the end of its LB phase (step, F/2), lb.in's f_ext
@@ -189,7 +190,7 @@ template <typename W>
 struct BatchMpView {
     const BInst* insts;
     const uint32_t* tile_inst;    // of each MP tile
-    const uint32_t* act;          // the MP tiles of the instances in the phase, ascending
+    const uint32_t* act;          // the MP tiles of the instances in the phase, the general ones last, each ascending
     MpTiles t;
     MpFields<W> f;
     const uint32_t* nodes;
@@ -416,7 +417,8 @@ __global__ __launch_bounds__(kBlock, (GEN ? 2 : 4)) void kb_mp_round(BatchMpView
         block_share(ntiles, [&](uint32_t l) { kb_mp_tile<W, GEN>(v, v.act[l], k, 1); });
         grid.sync();
     }
-    for (uint32_t id = blockIdx.x; id < ninst; id += gridDim.x) kb_mp_reduce_inst(v, id);
+    for (uint32_t id = blockIdx.x; id < ninst; id += gridDim.x)
+        if ((v.insts[id].mp_general != 0) == GEN) kb_mp_reduce_inst(v, id);  // those that this launch stepped
 }
 
 // ------------------------------------------------------------------ host
@@ -473,7 +475,6 @@ struct HostInst {
     double Db = 0, ka = 0, kd = 0, lambda = 0;
     int64_t t = 0, max_lb = 0, switch_step = INT64_MAX, check_after = 2;
     int64_t mp_it = 0, mp_target = 0;
-    bool general = false;           // its MP steps need the general kernel (lbx_mp.h)
     std::vector<double> vacf;       // (mp_it+1) x 3
     double deff[3] = {0, 0, 0};
 };
@@ -483,7 +484,6 @@ struct HostInst {
 struct lbxb {
     int32_t prec = LBX_PREC_FP64;
     bool wide = false;       // 64-bit addressing of the population buffers
-    uint32_t n_general = 0;  // live instances whose MP steps need the general kernel
     bool wide_auto = false;  // what the capacity alone selects
     uint64_t Np = 0, cap_box = 0;
     uint32_t cap_inst = 0, ntiles_cap = 0;
@@ -538,13 +538,14 @@ struct lbxb {
     uint32_t* act[2] = {nullptr, nullptr};
     std::vector<uint32_t> act_h[2];
     uint32_t n_act[2] = {0, 0};
+    uint32_t n_gen = 0;       // general MP tiles, the last of act[1]
     RangeAlloc node_alloc, map_alloc;
     // graphs of a round's launches, keyed by (phase, launches)
     struct Graph {
         hipGraphExec_t exec = nullptr;
         int32_t block = 0;
         uint32_t grid_tiles = 0;  // active tiles of the phase
-        bool general = false;     // the MP launches run the general kernel
+        uint32_t gen_tiles = 0;   // ... of the general kernel
     };
     std::map<std::pair<int, int64_t>, Graph> graph_cache;
     // statistics
@@ -604,13 +605,19 @@ uint32_t grid_of(const lbxb* b, int block, int phase /*0 LB, 1 MP*/) {
 int upload_active(lbxb* b) {
     LBX_TRY(hipStreamSynchronize(b->stream));  // the previous lists' uploads have been read
     for (int ph = 0; ph < 2; ++ph) {
-        std::vector<std::pair<uint32_t, uint32_t>> r;  // (first tile, tiles) of the phase's instances
+        // (first tile, tiles) of the phase's instances, those of the general MP kernel last
+        std::vector<std::pair<uint32_t, uint32_t>> r, gen;
         for (uint32_t id = 0; id < b->cap_inst; ++id) {
             const BInst& in = b->tab[id];
             if (ph == 0 && in.lb_on) r.emplace_back(in.tile_first, in.ntiles);
-            if (ph == 1 && in.mp_on) r.emplace_back(in.mp_tile0, in.mp_ntiles);
+            if (ph == 1 && in.mp_on) (in.mp_general ? gen : r).emplace_back(in.mp_tile0, in.mp_ntiles);
         }
         std::sort(r.begin(), r.end());
+        std::sort(gen.begin(), gen.end());
+        uint32_t n_gen = 0;
+        for (const auto& x : gen) n_gen += x.second;
+        if (ph == 1) b->n_gen = n_gen;
+        r.insert(r.end(), gen.begin(), gen.end());
         std::vector<uint32_t>& a = b->act_h[ph];
         a.clear();
         for (const auto& x : r)
@@ -710,14 +717,19 @@ void launch_lb(lbxb* b, int64_t k, int block) {
     });
 }
 
+// MP step k of a round: one launch for the instances on brick tiles, and one
+// for those that need the general kernel (236 VGPRs and 65 KB of LDS in FP64,
+// two waves per SIMD: two 128x128x96 boxes 112 us a step, 213 when a small
+// general instance beside them took them to it, 130 with a launch of its own)
 void launch_mp(lbxb* b, int64_t k, int reduce_prev) {
-    const uint32_t grid = grid_of(b, kBlock, 1);
-    if (!grid) return;
-    const bool gen = b->n_general > 0;
     auto go = [&](auto wtag) {
         using W = decltype(wtag);
-        auto kern = gen ? kb_mp_step<W, true> : kb_mp_step<W, false>;
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(kBlock), 0, b->stream, mp_view<W>(b), k, reduce_prev);
+        BatchMpView<W> v = mp_view<W>(b);
+        const uint32_t n = b->n_act[1] - b->n_gen;
+        if (n) hipLaunchKernelGGL((kb_mp_step<W, false>), dim3(n), dim3(kBlock), 0, b->stream, v, k, reduce_prev);
+        v.act += n;
+        if (b->n_gen)
+            hipLaunchKernelGGL((kb_mp_step<W, true>), dim3(b->n_gen), dim3(kBlock), 0, b->stream, v, k, reduce_prev);
     };
     if (shift(b))
         go(float{});
@@ -761,9 +773,9 @@ int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
     }
     auto key = std::make_pair(phase, S);
     auto it = b->graph_cache.find(key);
-    const bool gen = phase == 1 && b->n_general > 0;
+    const uint32_t gen = phase == 1 ? b->n_gen : 0;
     if (it != b->graph_cache.end() &&
-        (it->second.block != block || it->second.grid_tiles != b->n_act[phase] || it->second.general != gen)) {
+        (it->second.block != block || it->second.grid_tiles != b->n_act[phase] || it->second.gen_tiles != gen)) {
         (void)hipGraphExecDestroy(it->second.exec);
         b->graph_cache.erase(it);
         it = b->graph_cache.end();
@@ -784,7 +796,7 @@ int run_phase(lbxb* b, int phase /*0 LB, 1 MP*/, int64_t S) {
         if (ie != hipSuccess) return hip_status(ie);
         gr.block = block;
         gr.grid_tiles = b->n_act[phase];
-        gr.general = gen;
+        gr.gen_tiles = gen;
         it = b->graph_cache.emplace(key, gr).first;
     }
     return hip_status(hipGraphLaunch(it->second.exec, b->stream));
@@ -796,7 +808,7 @@ int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
     if (S <= 0) return LBX_OK;
     uint32_t nt = grid_of(b, b->lb_block, phase), ni = b->cap_inst;
     if (!nt) return LBX_OK;
-    auto launch = [&](auto kern, int block, void** args) -> int {
+    auto launch = [&](auto kern, uint32_t tiles, int block, void** args) -> int {
         int per_cu = 0;
         LBX_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, block, 0));
         if (per_cu <= 0) return LBX_ERR_DEVICE;
@@ -805,15 +817,20 @@ int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
         // FP64 538 + 298 / 421 + 267 / 454 + 358, FP32-shift 567 + 327 / 340 + 248 / 389 + 279;
         // 64 cells 1x100x100 FP64 185 + 143 / 117 + 86 / 94 + 77
         per_cu = std::min(per_cu, 512 / block);
-        const uint32_t grid = std::min<uint32_t>(nt, (uint32_t)per_cu * (uint32_t)b->num_cu);
+        const uint32_t grid = std::min<uint32_t>(tiles, (uint32_t)per_cu * (uint32_t)b->num_cu);
         return hip_status(hipLaunchCooperativeKernel((const void*)kern, dim3(grid), dim3(block), args, 0, b->stream));
     };
     if (phase == 1) {
         auto go = [&](auto wtag) -> int {
             using W = decltype(wtag);
             BatchMpView<W> v = mp_view<W>(b);
+            uint32_t ngen = b->n_gen;
+            nt -= ngen;
             void* args[] = {&v, &S, &nt, &ni};
-            return launch(b->n_general > 0 ? kb_mp_round<W, true> : kb_mp_round<W, false>, kBlock, args);
+            if (nt) LBX_TRY(launch(kb_mp_round<W, false>, nt, kBlock, args));
+            v.act += nt;
+            void* gargs[] = {&v, &S, &ngen, &ni};
+            return ngen ? launch(kb_mp_round<W, true>, ngen, kBlock, gargs) : LBX_OK;
         };
         return shift(b) ? go(float{}) : go(double{});
     }
@@ -823,7 +840,7 @@ int run_phase_persistent(lbxb* b, int phase, int64_t S, int32_t redo_only) {
         constexpr int BL = decltype(btag)::value;
         BatchView<E, R> v = lb_view<E, R>(b);
         void* args[] = {&v, &S, &nt, &ni, &redo_only};
-        return launch(b->wide ? kb_lb_round<BL, true, E, R> : kb_lb_round<BL, false, E, R>, BL, args);
+        return launch(b->wide ? kb_lb_round<BL, true, E, R> : kb_lb_round<BL, false, E, R>, nt, BL, args);
     };
     int st = LBX_OK;
     with_block(b->lb_block, [&](auto BT) {
@@ -923,7 +940,7 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
     }
     LBX_TRY(hipMemcpyAsync(b->mp_tile_inst, b->mp_tile_inst_h.data(), b->mp_tile_inst_h.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice, b->stream));
-    for (size_t k : gen) b->hi[ids[k]].general = true;
+    for (size_t k : gen) b->tab[ids[k]].mp_general = 1;
     return LBX_OK;
 }
 
@@ -984,11 +1001,9 @@ int mp_setup_insts(lbxb* b, const std::vector<uint32_t>& ids) {
         if (c.restpart) {
             h.phase = kFailed;
             h.status = LBX_ERR_RESTPART;
-            h.general = false;  // it takes no step
             continue;
         }
-        h.general = h.general || (!shift(b) && c.mp_divide);
-        if (h.general) ++b->n_general;
+        if (!shift(b) && c.mp_divide) b->tab[id].mp_general = 1;
         h.vacf.assign(c.vacf0, c.vacf0 + 3);
         h.mp_it = 0;
         h.phase = h.mp_target > 0 ? kMp : kDone;
@@ -1245,7 +1260,6 @@ int lbxb_remove(lbxb* b, int32_t id) {
                        in.ntiles, b->nfi + id);
     b->node_alloc.give(in.tile_first, in.ntiles);
     b->map_alloc.give(in.map_off, b->hi[id].map_n);
-    if (b->hi[id].general) --b->n_general;
     b->hi[id] = HostInst{};
     in = BInst{};
     return hip_status(hipGetLastError());

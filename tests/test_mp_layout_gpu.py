@@ -199,3 +199,24 @@ def test_batch_of_layouts_equals_single(prec, mode):
                 m = L.mp_run(steps)
                 assert np.array_equal(g["vacf"], np.vstack([v0, m["vacf"]])), n
                 assert np.array_equal(g["deff"], L.mp_deff()), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec", [lbx.PREC_FP64, lbx.PREC_FP32_SHIFT])
+def test_general_instance_does_not_slow_its_batch(prec):
+    """The MP time of two open boxes alone and beside a small lattice that needs
+    the general step (1.9 times as long when that took every instance to it)."""
+    print("mp layout batch time", prec, flush=True)
+    dims, steps = (128, 128, 96), 512
+    ms = []
+    for beside in (0, 1):
+        cases = [box(*dims)] * 2 + [CASES["corner_lines"][:2]] * beside
+        cap = sum(-(-int((n == 0).sum()) // 256) * 256 for _, n in cases)
+        with lbx.Batch(cap, sum(n.size for _, n in cases), len(cases), precision=prec) as B:
+            for d, n in cases:
+                assert B.add(d, n, 0.9, 1.0, FEXT, 0.0, 0.01, 0.02, 0.01, steps, max_lb_steps=4) is not None
+            while B.round(4, 128):
+                pass
+            ms.append(B.stats()["mp_ms"])
+    print("alone / beside a general one, us per step", *[m / steps * 1e3 for m in ms], flush=True)
+    assert ms[1] < 1.25 * ms[0]
