@@ -886,27 +886,41 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         take(b->walk_base, walk);
     }, true));
     uint32_t *count = b->walk_count, *base = b->walk_base;
+    constexpr uint32_t kGridY = 65535;  // lattices of one launch at most
+    const auto size_of = [&](size_t k) { return std::max((uint64_t)builds[k].b.norder, (uint64_t)builds[k].bound); };
     // one pass over the lattices `which`: tiles cut by `by`, `mark` for the next
     // pass; general: keep what has an LDS slot
-    auto pass = [&](const std::vector<size_t>& which, const uint8_t* by, uint8_t* mark, uint32_t level,
+    auto pass = [&](std::vector<size_t>& which, const uint8_t* by, uint8_t* mark, uint32_t level,
                     bool general) -> int {
+        // largest first, so that a launch's lattices are of like size: its grid is the largest one's for each
+        std::stable_sort(which.begin(), which.end(), [&](size_t x, size_t y) { return size_of(x) > size_of(y); });
         std::vector<MpBuild> d;
-        uint32_t gw = 0, gt = 0;
-        for (size_t k : which) {
-            d.push_back(builds[k]);
-            gw = std::max(gw, (builds[k].b.norder + kBlock / 64 - 1) / (kBlock / 64));
-            gt = std::max(gt, builds[k].bound);
-        }
+        for (size_t k : which) d.push_back(builds[k]);
         const uint32_t nd = (uint32_t)d.size();
+        // f(first, lattices, blocks for one wave a brick, blocks for one a tile) per launch
+        const auto slices = [&](auto&& f) {
+            for (uint32_t s0 = 0, s1; s0 < nd; s0 = s1) {
+                uint32_t gw = 0, gt = 0;
+                for (s1 = s0; s1 < nd && s1 - s0 < kGridY && 2 * size_of(which[s1]) >= size_of(which[s0]); ++s1) {
+                    gw = std::max(gw, (d[s1].b.norder + kBlock / 64 - 1) / (kBlock / 64));
+                    gt = std::max(gt, d[s1].bound);
+                }
+                f(s0, s1 - s0, gw, gt);
+            }
+        };
         LBX_TRY(hipMemcpyAsync(b->builds, d.data(), nd * sizeof(MpBuild), hipMemcpyHostToDevice, b->stream));
         if (level == 1)
-            hipLaunchKernelGGL(k_mpb_count, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, count);
+            slices([&](uint32_t s0, uint32_t n, uint32_t gw, uint32_t) {
+                hipLaunchKernelGGL(k_mpb_count, dim3(gw, n), dim3(kBlock), 0, b->stream, b->builds + s0, count);
+            });
         hipLaunchKernelGGL(k_mpb_group, dim3(nd), dim3(kBlock), 0, b->stream, b->builds, b->built, count, base,
                            b->mpt.info, by, b->owner);
-        hipLaunchKernelGGL(k_mpb_place, dim3(gw, nd), dim3(kBlock), 0, b->stream, b->builds, b->built, base,
-                           b->mpt.perm, b->mpt.inv);
-        hipLaunchKernelGGL((general ? k_mpb_table<true> : k_mpb_table<false>), dim3(gt, nd), dim3(kBlock), 0,
-                           b->stream, b->builds, b->built, b->mpt, b->owner, mark, level);
+        slices([&](uint32_t s0, uint32_t n, uint32_t gw, uint32_t gt) {
+            hipLaunchKernelGGL(k_mpb_place, dim3(gw, n), dim3(kBlock), 0, b->stream, b->builds + s0, b->built + s0,
+                               base, b->mpt.perm, b->mpt.inv);
+            hipLaunchKernelGGL((general ? k_mpb_table<true> : k_mpb_table<false>), dim3(gt, n), dim3(kBlock), 0,
+                               b->stream, b->builds + s0, b->built + s0, b->mpt, b->owner, mark, level);
+        });
         LBX_TRY(hipGetLastError());
         std::vector<MpBuilt> r(nd);
         LBX_TRY(hipMemcpyAsync(r.data(), b->built, nd * sizeof(MpBuilt), hipMemcpyDeviceToHost, b->stream));
