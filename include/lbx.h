@@ -459,12 +459,12 @@ int lbxb_launch_mode(lbxb* b);
 int lbxb_set_addressing(lbxb* b, int32_t wide);
 int lbxb_addressing(lbxb* b);
 /* Autotuner: on the current state, without changing it, times 64-, 128-
- * and 256-node LB blocks with one launch per step and keeps the fastest (the
- * MP launches, the same for every mp_block, are timed under each), then times
- * those launches replayed from a captured graph and as one persistent
+ * and 256-node LB blocks with one launch per step and keeps the fastest, times
+ * the MP launches (the same for every mp_block, which stays as it is), then
+ * times those launches replayed from a captured graph and as one persistent
  * cooperative launch per phase, and keeps the launch mode with the least
  * LB + MP time.  times[LBXB_AUTOTUNE_TIMES] (may be NULL) = mean ms per step of
- * LB-64, LB-128, LB-256, MP-64, MP-128, MP-256, LB-graph, MP-graph,
+ * LB-64, LB-128, LB-256, MP (three times), LB-graph, MP-graph,
  * LB-persistent, MP-persistent (0: phase not timed). */
 #define LBXB_AUTOTUNE_TIMES 10
 int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_block, double* times);

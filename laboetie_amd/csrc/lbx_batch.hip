@@ -1537,25 +1537,24 @@ int lbxb_launch_mode(lbxb* b) {
     return b->persistent ? LBXB_LAUNCH_PERSISTENT : (b->graphs ? LBXB_LAUNCH_GRAPH : LBXB_LAUNCH_STREAM);
 }
 
-// The autotuner's search space: the block size of each phase (64, 128 or
+// The autotuner's search space: the block size of the LB launches (64, 128 or
 // 256 nodes, i.e. 1, 2 or 4 waves per block and 4, 2 or 1 blocks per
-// 256-node tile) and the launch mode of the rounds (one launch per step, the
-// same launches replayed from a captured graph, or one cooperative
-// persistent launch per phase).  Every point is timed on the current state
-// without changing it: LB launches redo each LB instance's last completed step
-// (same inputs, same outputs), MP launches recompute its last MP step without
-// the VACF reduction.  The fastest block size per phase is kept, then the
-// mode with the least LB + MP time at those sizes (the persistent launch
-// runs both phases with the LB block size).  times[LBXB_AUTOTUNE_TIMES] (may be
-// NULL): mean ms per step of LB-64, LB-128, LB-256, MP-64, MP-128, MP-256
-// (per-step launches), LB-graph, MP-graph, LB-persistent, MP-persistent (0
-// when a phase had no instance to time).
+// 256-node tile; an MP launch has one block a tile) and the launch mode of the
+// rounds (one launch per step, the same launches replayed from a captured
+// graph, or one cooperative persistent launch per phase).  Every point is timed
+// on the current state without changing it: LB launches redo each LB instance's
+// last completed step (same inputs, same outputs), MP launches recompute its
+// last MP step without the VACF reduction.  The fastest LB block size is kept,
+// then the mode with the least LB + MP time at that size; mp_block stays as it
+// is.  times[LBXB_AUTOTUNE_TIMES] (may be NULL): mean ms per step of LB-64,
+// LB-128, LB-256, MP three times (per-step launches), LB-graph, MP-graph,
+// LB-persistent, MP-persistent (0 when a phase had no instance to time).
 int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_block, double* times) {
     if (!b || launches <= 0) return LBX_ERR_ARG;
     const uint32_t ni = b->cap_inst;
     constexpr int kSizes = 3;
     const int sizes[kSizes] = {64, 128, 256};
-    double tm[2][kSizes] = {{0, 0, 0}, {0, 0, 0}};
+    double tm[kSizes] = {0, 0, 0}, tmp = 0;  // LB by block size, MP
     bool any[2] = {false, false};
     for (uint32_t id = 0; id < ni; ++id) {
         BInst& in = b->tab[id];
@@ -1593,33 +1592,28 @@ int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_bloc
         *out = ms / launches;
         return LBX_OK;
     };
-    // per-step launches of every block size
-    for (int s = 0; s < kSizes; ++s)
-        for (int phase = 0; phase < 2; ++phase) {
-            if (!any[phase]) continue;
-            launch(phase, sizes[s]);  // warm
-            LBX_TRY(hipEventRecord(b->ev[0], b->stream));
-            for (int32_t k = 0; k < launches; ++k) launch(phase, sizes[s]);
-            LBX_TRY(elapsed(&tm[phase][s]));
-        }
-    int best[2] = {b->lb_block, b->mp_block};
-    for (int phase = 0; phase < 2; ++phase) {
-        if (!any[phase]) continue;
-        int k = 0;
-        for (int s = 1; s < kSizes; ++s)
-            if (tm[phase][s] < tm[phase][k]) k = s;
-        best[phase] = sizes[k];
+    // per-step launches: LB with every block size, MP
+    auto timed = [&](int phase, int block, double* out) -> int {
+        launch(phase, block);  // warm
+        LBX_TRY(hipEventRecord(b->ev[0], b->stream));
+        for (int32_t k = 0; k < launches; ++k) launch(phase, block);
+        return elapsed(out);
+    };
+    int best = 0;
+    for (int k = 0; any[0] && k < kSizes; ++k) {
+        LBX_TRY(timed(0, sizes[k], &tm[k]));
+        if (tm[k] < tm[best]) best = k;
     }
-    b->lb_block = best[0];
-    b->mp_block = best[1];
-    // the same launches at those sizes replayed from a captured graph
+    if (any[0]) b->lb_block = sizes[best];
+    if (any[1]) LBX_TRY(timed(1, kBlock, &tmp));
+    // the same launches replayed from a captured graph
     double tg[2] = {0, 0};
     for (int phase = 0; phase < 2; ++phase) {
         if (!any[phase]) continue;
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         LBX_TRY(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        for (int32_t k = 0; k < launches; ++k) launch(phase, best[phase]);
+        for (int32_t k = 0; k < launches; ++k) launch(phase, b->lb_block);
         const hipError_t ce = hipStreamEndCapture(b->stream, &graph);
         if (ce != hipSuccess) return hip_status(ce);
         const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -1633,8 +1627,7 @@ int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_bloc
         (void)hipGraphExecDestroy(exec);
         LBX_TRY(st);
     }
-    // one cooperative launch of `launches` repeated steps per phase, with the
-    // LB block size (kb_round runs both phases with one size)
+    // one cooperative launch of `launches` repeated steps per phase
     double tp[2] = {0, 0};
     for (uint32_t id = 0; id < ni; ++id) {
         BInst& in = b->tab[id];
@@ -1657,14 +1650,7 @@ int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_bloc
     LBX_TRY(hipMemcpyAsync(b->insts, b->tab.data(), ni * sizeof(BInst), hipMemcpyHostToDevice, b->stream));
     // the launch mode with the least time over the timed phases
     if (any[0] || any[1]) {
-        double t_stream = 0, t_graph = 0, t_pers = 0;
-        for (int phase = 0; phase < 2; ++phase) {
-            if (!any[phase]) continue;
-            for (int s = 0; s < kSizes; ++s)
-                if (sizes[s] == best[phase]) t_stream += tm[phase][s];
-            t_graph += tg[phase];
-            t_pers += tp[phase];
-        }
+        const double t_stream = tm[best] + tmp, t_graph = tg[0] + tg[1], t_pers = tp[0] + tp[1];
         b->persistent = t_pers < t_graph && t_pers < t_stream;
         b->graphs = !b->persistent && t_graph <= t_stream;
     }
@@ -1672,8 +1658,10 @@ int lbxb_autotune(lbxb* b, int32_t launches, int32_t* lb_block, int32_t* mp_bloc
     if (lb_block) *lb_block = b->lb_block;
     if (mp_block) *mp_block = b->mp_block;
     if (times) {
-        for (int phase = 0; phase < 2; ++phase)
-            for (int s = 0; s < kSizes; ++s) times[phase * kSizes + s] = tm[phase][s];
+        for (int k = 0; k < kSizes; ++k) {
+            times[k] = tm[k];
+            times[kSizes + k] = tmp;
+        }
         times[6] = tg[0];
         times[7] = tg[1];
         times[8] = tp[0];

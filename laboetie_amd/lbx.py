@@ -619,9 +619,9 @@ class Batch:
         _check(lib().lbxb_set_check_interval(self._h, int(steps)), "lbxb_set_check_interval")
 
     def autotune(self, launches=10):
-        """lbxb_autotune: block size per phase (64/128/256 nodes) and launch
-        mode (per-step, graph, persistent); the chosen point and every timing
-        (mean ms per step)."""
+        """lbxb_autotune: LB block size (64/128/256 nodes) and launch mode
+        (per-step, graph, persistent); the chosen point and every timing (mean
+        ms per step; an MP launch is the same for every mp_block)."""
         lb, mp = _i32(), _i32()
         t = np.zeros(AUTOTUNE_TIMES)
         _check(lib().lbxb_autotune(self._h, int(launches), ctypes.byref(lb), ctypes.byref(mp), _ptr(t)),
