@@ -137,7 +137,8 @@ struct lbx_ctx {
     // tiles' (by packed node and by tile) and a propagation's
     Block lb_block, node_block, tile_block, mp_block;
     double* box = nullptr;            // full-box copies: the values of planes or of a run of box nodes
-    uint32_t box_n = 0;               // ... and how many it holds
+    double* box_reserve = nullptr;    // a small one that is always there
+    uint32_t box_n = 0;               // values that box holds
 };
 
 // the forms that store populations as FP32 deviations (FP32-shift: FP32
@@ -175,6 +176,11 @@ void free_tiles(lbx_ctx* c) {
     c->mp_ntiles = 0;
 }
 
+void give_box(lbx_ctx* c) {
+    if (c->box != c->box_reserve) dfree(c->box);
+    c->box = nullptr;
+}
+
 void free_all(lbx_ctx* c) {
     free_mp(c);
     free_tiles(c);
@@ -186,7 +192,7 @@ void free_all(lbx_ctx* c) {
     give_block(&c->lb_block);
     dfree(c->jpart);
     dfree(c->jflow);
-    dfree(c->box);
+    give_box(c);
     for (auto& e : c->ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
     if (c->stream) (void)hipStreamDestroy(c->stream), c->stream = nullptr;
@@ -428,19 +434,21 @@ uint32_t box_values(uint64_t N) {
     return (uint32_t)std::min<uint64_t>(kMaxPlanes * N, std::max<uint64_t>(1u << 18, std::min<uint64_t>(N, 1u << 22)));
 }
 
-// The buffer (c->box, c->box_n values), kept until the context goes; as much
-// of it as the device still has.
+constexpr uint32_t kBoxReserve = 4096;
+
+// The buffer (c->box, c->box_n values), kept until the context goes: as much of
+// it as the device still has, or the few values that every context has from
+// the start, so that a state can be fetched from a full device too.
 int box_buffer(lbx_ctx* c) {
-    for (uint32_t n = box_values(c->N); !c->box;) {
-        const int st = dalloc(&c->box, n);
-        c->box_n = st ? 0 : n;
-        if (!st) break;
-        if (st != LBX_ERR_NOMEM || n <= 4096) return st;
-        n /= 4;
+    for (uint32_t n = box_values(c->N); !c->box; n /= 4) {
+        const bool last = n <= kBoxReserve;
+        const int st = last ? LBX_OK : dalloc(&c->box, n);
+        if (st && st != LBX_ERR_NOMEM) return st;
+        if (last) c->box = c->box_reserve;
+        c->box_n = last ? (uint32_t)std::min(box_values(c->N), kBoxReserve) : n;
     }
     return LBX_OK;
 }
-
 // box nodes [r0, r0 + n) of the planes p0 + blockIdx.y: packed values as FP64,
 // 0 at solids; FP32 deviations become rest + g
 __global__ __launch_bounds__(kBlock) void k_spread(Planes::Dev d, int p0, const uint32_t* __restrict__ map,
@@ -816,6 +824,7 @@ void lb_arrays(lbx_ctx* c, Take&& take) {
     take(c->slots, (uint64_t)(3 * kSlots));
     take(c->ctrl, (uint64_t)1);
     take(c->l2ring, (uint64_t)kRing);
+    take(c->box_reserve, (uint64_t)std::min(box_values(c->N), kBoxReserve));
 }
 }  // namespace
 
@@ -1243,7 +1252,12 @@ static int mp_setup(lbx_ctx* c, const double fext[3], double Db, int32_t ntr, co
         else
             mp_arrays<double>(c, ntr, any_ads, stored, c->mp_ntiles, take);
     };
-    if (const int st = take_block(&c->mp_block, lay)) {
+    int st = take_block(&c->mp_block, lay);
+    if (st == LBX_ERR_NOMEM && c->box) {  // the transfer buffer's memory first
+        give_box(c);
+        st = take_block(&c->mp_block, lay);
+    }
+    if (st) {
         give_block(&c->mp_block);
         return st;
     }
