@@ -573,7 +573,9 @@ void tile_arrays(lbx_ctx* c, uint64_t tiles, uint32_t pitch, Take&& take) {
 int build_tiles(lbx_ctx* c) {
     if (c->mp_ntiles) return LBX_OK;
     MpBuild d{};
-    d.b = make_bricks((uint32_t)c->lx, (uint32_t)c->ly, (uint32_t)c->lz);
+    const Bricks whole = make_bricks((uint32_t)c->lx, (uint32_t)c->ly, (uint32_t)c->lz),
+                 halves = make_bricks((uint32_t)c->lx, (uint32_t)c->ly, (uint32_t)c->lz, true);
+    const uint64_t norder = std::max(whole.norder, halves.norder);
     d.nodes = c->nodes;
     d.map = c->map;
     d.dlx = c->dlx;
@@ -586,10 +588,10 @@ int build_tiles(lbx_ctx* c) {
     uint8_t* split = nullptr;
     Block scratch;
     MpBuilt h{};
-    const uint32_t gw = (d.b.norder + kBlock / 64 - 1) / (kBlock / 64);
     MpTiles& t = c->mpt;
     hipStream_t s = c->stream;
     int st = LBX_OK;
+    const auto waves = [&] { return dim3((d.b.norder + kBlock / 64 - 1) / (kBlock / 64)); };
     auto group = [&](const uint8_t* sp) {
         hipLaunchKernelGGL(k_mpb_group, dim3(1), dim3(kBlock), 0, s, dd, db, count, base, t.info, sp,
                            owner);
@@ -602,7 +604,7 @@ int build_tiles(lbx_ctx* c) {
         st = take_block(&c->tile_block, [&](auto&& take) { tile_arrays(c, h.ntiles, pitch, take); });
         if (st) return;
         t.pitch = pitch;
-        hipLaunchKernelGGL(k_mpb_place, dim3(gw), dim3(kBlock), 0, s, dd, db, base, t.perm, t.inv);
+        hipLaunchKernelGGL(k_mpb_place, waves(), dim3(kBlock), 0, s, dd, db, base, t.perm, t.inv);
         hipLaunchKernelGGL((pitch > kHaloMax ? k_mpb_table<true> : k_mpb_table<false>), dim3(h.ntiles), dim3(kBlock), 0,
                            s, dd, db, t, owner, sp, level);
         st = hip_status(hipGetLastError());
@@ -612,26 +614,38 @@ int build_tiles(lbx_ctx* c) {
     st = take_block(&scratch, [&](auto&& take) {
         take(dd, (uint64_t)1);
         take(db, (uint64_t)1);
-        take(count, (uint64_t)d.b.norder);
-        take(base, (uint64_t)d.b.norder);
+        take(count, norder);
+        take(base, norder);
         take(owner, (uint64_t)d.bound);
         take(split, (uint64_t)d.bound);
     });
     if (!st) st = take_block(&c->node_block, [&](auto&& take) { node_arrays(c, d.bound, take); });
-    if (!st) st = hip_status(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
-    if (!st) {
-        hipLaunchKernelGGL(k_mpb_count, dim3(gw), dim3(kBlock), 0, s, dd, count);
+    // the layout with bricks b on at most `bound` tiles; no tiles (h.ntiles): it takes more
+    auto settle = [&](const Bricks& b, uint32_t bound) {
+        d.b = b;
+        d.bound = bound;
+        d.serial = b.inner == 1;
+        h.ntiles = 0;
+        if (!st) st = hip_status(hipMemcpyAsync(dd, &d, sizeof(d), hipMemcpyHostToDevice, s));
+        if (st) return;
+        hipLaunchKernelGGL(k_mpb_count, waves(), dim3(kBlock), 0, s, dd, count);
         group(nullptr);
-        table(kHaloMax, split, 1);
+        if (h.ntiles > 0) table(kHaloMax, split, 1);
         for (uint32_t level = 2; !st && h.ntiles > 0 && h.halo_max > kHaloMax; ++level) {
             group(split);
             if (h.ntiles > 0) table(kHaloMax, split, level);
         }
-        c->mp_general = h.ntiles == 0;
-        if (!st && c->mp_general) {
-            group(nullptr);
-            table(kHaloMaxGen, nullptr, 0);
-        }
+    };
+    const uint32_t bound = d.bound;
+    settle(whole, bound);
+    if (!st && halves.inner > 1 && h.ntiles > 0 && try_halves(h.ntiles, c->Nf)) {
+        settle(halves, halves_bound(h.ntiles));
+        if (!st && h.ntiles == 0) settle(whole, bound);
+    }
+    c->mp_general = h.ntiles == 0;
+    if (!st && c->mp_general) {
+        group(nullptr);
+        table(kHaloMaxGen, nullptr, 0);
     }
     give_block(&scratch);
     if (st) {

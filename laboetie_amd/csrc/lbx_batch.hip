@@ -865,6 +865,7 @@ int download(lbxb* b, const T* src, uint64_t count, T* dst) {
 int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
     std::vector<MpBuild> builds(ids.size());
     std::vector<MpBuilt> built(ids.size());
+    std::vector<Bricks> halves(ids.size());
     uint64_t walk = 0;
     for (size_t k = 0; k < ids.size(); ++k) {
         const HostInst& h = b->hi[ids[k]];
@@ -872,6 +873,7 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         MpBuild& d = builds[k];
         d = MpBuild{};
         d.b = make_bricks((uint32_t)h.lx, (uint32_t)h.ly, (uint32_t)h.lz);
+        halves[k] = make_bricks((uint32_t)h.lx, (uint32_t)h.ly, (uint32_t)h.lz, true);
         d.nodes = b->nodes;
         d.map = b->maps + in.map_off;
         d.dlx = in.dlx;
@@ -879,7 +881,8 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         d.order_off = (uint32_t)walk;
         d.tile0 = 2 * in.tile_first;
         d.bound = mp_tile_bound(h.Nf);  // 2 in.ntiles
-        walk += d.b.norder;
+        d.serial = 1;
+        walk += std::max(d.b.norder, halves[k].norder);
     }
     LBX_TRY(take_block(&b->walk_block, [&](auto&& take) {
         take(b->walk_count, walk);
@@ -928,22 +931,38 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         for (uint32_t k = 0; k < nd; ++k) built[which[k]] = r[k];
         return LBX_OK;
     };
-    std::vector<size_t> all, again, gen;
-    for (size_t k = 0; k < ids.size(); ++k) all.push_back(k);
-    LBX_TRY(pass(all, nullptr, b->split, 1, false));
-    for (size_t k : all)
-        if (built[k].halo_max > kHaloMax) again.push_back(k);
-    for (uint32_t level = 2; !again.empty(); ++level) {
-        LBX_TRY(pass(again, b->split, b->split, level, false));
-        std::vector<size_t> more;
-        for (size_t k : again) {
-            if (built[k].ntiles == 0)
-                gen.push_back(k);
-            else if (built[k].halo_max > kHaloMax)
-                more.push_back(k);
+    // the layouts of the lattices `which`; returns those that take more than their bound of tiles
+    std::vector<size_t> gen;
+    auto settle = [&](std::vector<size_t> which, std::vector<size_t>* beyond) -> int {
+        for (uint32_t level = 1; !which.empty(); ++level) {
+            LBX_TRY(pass(which, level == 1 ? nullptr : b->split, b->split, level, false));
+            std::vector<size_t> more;
+            for (size_t k : which) {
+                if (built[k].ntiles == 0)
+                    beyond->push_back(k);
+                else if (built[k].halo_max > kHaloMax)
+                    more.push_back(k);
+            }
+            which.swap(more);
         }
-        again.swap(more);
+        return LBX_OK;
+    };
+    std::vector<size_t> some(ids.size()), whole;
+    for (size_t k = 0; k < ids.size(); ++k) some[k] = k;
+    LBX_TRY(settle(some, &gen));
+    some.clear();
+    for (size_t k = 0; k < ids.size(); ++k)
+        if (halves[k].inner > 1 && built[k].ntiles > 0 && try_halves(built[k].ntiles, b->hi[ids[k]].Nf))
+            some.push_back(k);
+    std::vector<MpBuild> was = builds;
+    for (size_t k : some) {
+        builds[k].b = halves[k];
+        builds[k].bound = halves_bound(built[k].ntiles);
+        builds[k].serial = 0;
     }
+    LBX_TRY(settle(some, &whole));
+    for (size_t k : whole) builds[k] = was[k];
+    LBX_TRY(settle(whole, &gen));
     if (!gen.empty()) LBX_TRY(pass(gen, nullptr, nullptr, 0, true));
     for (size_t k = 0; k < ids.size(); ++k) {
         BInst& in = b->tab[ids[k]];

@@ -1,8 +1,8 @@
 """The tiles of moment propagation (lbx_mp.h) with the bricks that a box is cut
 into: whole and merged bricks, tiles cut once and several times because their
 halo outgrows a brick's, and a lattice that runs out of tiles on the way and
-takes the general step, some of whose neighbours have no LDS slot.  P, Pa bit
-for bit against the restatement; FP32 forms: each of several tracers as alone;
+takes the general step, some of whose neighbours have no LDS slot; lattices whose
+bricks fill little over half a tile, with halves of them.  P, Pa bit for bit against the restatement; FP32 forms: each of several tracers as alone;
 batch instances: VACF and D_eff are the single lattice's bits.
 
 layout() restates the cut and the grouping, so that each case is known to be
@@ -31,17 +31,17 @@ def brick(lx, ly, lz):
     return bx, best[1], best[2]
 
 
-def layout(dims, nat):
-    """(times that the worst tile is cut, or "general"; largest halo of the uncut tiles)"""
-    lx, ly, lz = dims
-    fluid, b = nat.reshape(lz, ly, lx) == 0, brick(*dims)
-    nb = [-(-n // k) for n, k in zip(dims, b)]
+def settle(fluid, b, inner, bound):
+    """(tiles, times that the worst one is cut, largest halo of the uncut ones)
+    with bricks b, `inner` of them along z walked together; no tiles: it takes
+    more than `bound`."""
+    lz, ly, lx = fluid.shape
+    nb = [-(-n // k) for n, k in zip((lx, ly, lz), b)]
     cx, cy = min(8, nb[0]), min(8, nb[1])
-    walk = [(x0 + x, y0 + y, z) for y0 in range(0, nb[1], cy) for x0 in range(0, nb[0], cx) for z in range(nb[2])
-            for y in range(cy) for x in range(cx)]
+    walk = [(x0 + x, y0 + y, z0 + z) for y0 in range(0, nb[1], cy) for x0 in range(0, nb[0], cx)
+            for z0 in range(0, nb[2], inner) for y in range(cy) for x in range(cx) for z in range(inner)]
     nodes = [np.argwhere(fluid[z * b[2]:(z + 1) * b[2], y * b[1]:(y + 1) * b[1], x * b[0]:(x + 1) * b[0]])
              + (z * b[2], y * b[1], x * b[0]) for x, y, z in walk]
-    bound = 2 * -(-int(fluid.sum()) // 256)
 
     def group(run):
         tiles = []
@@ -68,20 +68,41 @@ def layout(dims, nat):
             at += len(n)
         return list(out.values())
 
-    tiles = group(128)
-    if len(tiles) > bound:
+    tiles = group(128 * inner)
+    if len(tiles) > bound and inner == 1:
         tiles = group(len(walk))
-    largest = max(map(halo, tiles))
-    todo, level = [t for t in tiles if halo(t) > HALO], 0
-    kept = len(tiles) - len(todo)
+    halos = list(map(halo, tiles))
+    if len(tiles) > bound:
+        return 0, 0, max(halos)
+    todo, level = [t for t, h in zip(tiles, halos) if h > HALO], 0
+    kept = total = len(tiles) - len(todo)
+    total += len(todo)
     while todo:
         level += 1
         cut = [parts(t, level) for t in todo]
-        if kept + sum(map(len, cut)) > bound:
-            return "general", largest
-        kept += sum(len(p) for p in cut if max(map(halo, p)) <= HALO)
-        todo = [t for t, p in zip(todo, cut) if max(map(halo, p)) > HALO]
-    return level, largest
+        total = kept + sum(map(len, cut))
+        if total > bound:
+            return 0, level, max(halos)
+        fits = [max(map(halo, p)) <= HALO for p in cut]
+        kept += sum(len(p) for p, f in zip(cut, fits) if f)
+        todo = [t for t, f in zip(todo, fits) if not f]
+    return total, level, max(halos)
+
+
+def layout(dims, nat):
+    """(times that the worst tile is cut, or "general", or "halves" / "whole" for
+    a lattice that tries halves of its bricks and takes them or not; largest
+    halo of the uncut tiles)"""
+    lx, ly, lz = dims
+    fluid, b = nat.reshape(lz, ly, lx) == 0, brick(*dims)
+    nf = int(fluid.sum())
+    whole = settle(fluid, b, 1, 2 * -(-nf // 256))
+    if not whole[0]:
+        return "general", whole[2]
+    if whole[0] >= 256 and whole[0] * 179 > nf and b[2] > 1:
+        half = settle(fluid, (b[0], b[1], -(-b[2] // 2)), 2, whole[0] - whole[0] // 10)
+        return ("halves", half[2]) if half[0] else ("whole", whole[2])
+    return whole[1], whole[2]
 
 
 def channels(dims, w, period):
@@ -111,6 +132,9 @@ CASES = {
     "channels": ((64, 64, 16), channels((64, 64, 16), 5, 8), 1),
     "ragged_box": (*box(33, 33, 33), 3),
     "ragged_noise": (*noise((37, 21, 11), 0.3, 1), 2),
+    "fine_noise": (*noise((64, 64, 64), 0.42, 6), "halves"),
+    "fine_ragged": (*noise((61, 67, 50), 0.45, 7), "halves"),
+    "wide_channels": ((64, 64, 48), channels((64, 64, 48), 7, 9), "whole"),
     "corner_lines": (*corner_lines(), "general"),
 }
 FEXT, KA, KD = [2e-5, -1e-5, 3e-5], [0.02, 0.0, 0.05], [0.01, 0.0, 0.01]
