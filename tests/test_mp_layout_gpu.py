@@ -2,7 +2,8 @@
 into: whole and merged bricks, tiles cut once and several times because their
 halo outgrows a brick's, and a lattice that runs out of tiles on the way and
 takes the general step, some of whose neighbours have no LDS slot; lattices whose
-bricks fill little over half a tile, with halves of them.  P, Pa bit for bit against the restatement; FP32 forms: each of several tracers as alone;
+bricks fill little over half a tile, with halves of them.  P, Pa bit for bit
+against the restatement, in the FP32 forms each of several tracers also as alone;
 batch instances: VACF and D_eff are the single lattice's bits.
 
 layout() restates the cut and the grouping, so that each case is known to be
@@ -178,22 +179,25 @@ def test_layouts_match_restatement(name, form, monkeypatch):
 @pytest.mark.parametrize("prec", [lbx.PREC_FP32_SHIFT, lbx.PREC_FP32_STORE])
 @pytest.mark.parametrize("form", [lbx.MP_STORED, lbx.MP_RECOMPUTED])
 @pytest.mark.parametrize("name", CASES)
-def test_fp32_tracers_as_alone(name, form, prec):
+def test_fp32_tracers_match_restatement(name, form, prec):
     dims, nat, _ = CASES[name]
     print("mp layout fp32", name, form, prec, flush=True)
     with lbx.Lattice(dims, nat, 0.9, precision=prec) as L:
         L.set_mp_coefficients(form)
         L.init_rest(1.0)
         L.equilibrate(FEXT, 0.0, max_steps=12)
+        _, rho, j = L.get_state(populations=False)
         v0 = L.mp_init_batch(FEXT, 0.01, KA, KD)
         v = L.mp_run(9)["vacf"].reshape(9, 3, 3)
         fields = [L.mp_get(t) for t in range(3)]
         for t in range(3):
+            st, _, P, Pa = lbref.mp_shift(dims, nat, lbref.interfacial(*dims, nat), rho, j, FEXT, 0.01, KA[t], KD[t], 9)
+            assert st == 0
             w0 = L.mp_init(FEXT, 0.01, KA[t], KD[t])
             w = L.mp_run(9)["vacf"]
             assert np.array_equal(v0[t], w0) and np.array_equal(v[:, t], w)
-            for a, b in zip(fields[t], L.mp_get()):
-                assert np.array_equal(a, b)
+            for a, b, ref in zip(fields[t], L.mp_get(), (P, Pa)):
+                assert np.array_equal(a, b) and np.array_equal(a, ref)
 
 
 @pytest.mark.gpu
