@@ -566,8 +566,8 @@ void tile_arrays(lbx_ctx* c, uint64_t tiles, uint32_t pitch, Take&& take) {
 
 // The MP tiles of the context's geometry: counted, grouped, placed and
 // tabled on the device (lbx_mp.h).  Tiles whose halo outgrows a brick's are cut
-// in two, and again, while the tile count stays within mp_tile_bound; beyond
-// that the lattice runs the general step, whose tiles may have neighbours
+// into as few parts as fit, while the tile count stays within mp_tile_bound;
+// beyond that the lattice runs the general step, whose tiles may have neighbours
 // without an LDS slot.  (Taken apart into their bricks at once, channels 5 wide
 // in 8 of a 128^3 box ran out of tiles, 56.8 us a step in FP64 for 33.4 now.)
 int build_tiles(lbx_ctx* c) {
@@ -584,7 +584,6 @@ int build_tiles(lbx_ctx* c) {
     MpBuild* dd = nullptr;
     MpBuilt* db = nullptr;
     uint32_t *count = nullptr, *base = nullptr;
-    uint32_t* owner = nullptr;
     uint8_t* split = nullptr;
     Block scratch;
     MpBuilt h{};
@@ -593,20 +592,19 @@ int build_tiles(lbx_ctx* c) {
     int st = LBX_OK;
     const auto waves = [&] { return dim3((d.b.norder + kBlock / 64 - 1) / (kBlock / 64)); };
     auto group = [&](const uint8_t* sp) {
-        hipLaunchKernelGGL(k_mpb_group, dim3(1), dim3(kBlock), 0, s, dd, db, count, base, t.info, sp,
-                           owner);
+        hipLaunchKernelGGL(k_mpb_group, dim3(1), dim3(kBlock), 0, s, dd, db, count, base, t.info, sp);
         if (!st) st = hip_status(hipGetLastError());
         if (!st) st = hip_status(hipMemcpyAsync(&h, db, sizeof(h), hipMemcpyDeviceToHost, s));
         if (!st) st = hip_status(hipStreamSynchronize(s));
     };
-    auto table = [&](uint32_t pitch, uint8_t* sp, uint32_t level) {
+    auto table = [&](uint32_t pitch, uint8_t* sp) {
         if (st) return;
         st = take_block(&c->tile_block, [&](auto&& take) { tile_arrays(c, h.ntiles, pitch, take); });
         if (st) return;
         t.pitch = pitch;
         hipLaunchKernelGGL(k_mpb_place, waves(), dim3(kBlock), 0, s, dd, db, base, t.perm, t.inv);
         hipLaunchKernelGGL((pitch > kHaloMax ? k_mpb_table<true> : k_mpb_table<false>), dim3(h.ntiles), dim3(kBlock), 0,
-                           s, dd, db, t, owner, sp, level);
+                           s, dd, db, t, sp);
         st = hip_status(hipGetLastError());
         if (!st) st = hip_status(hipMemcpyAsync(&h, db, sizeof(h), hipMemcpyDeviceToHost, s));
         if (!st) st = hip_status(hipStreamSynchronize(s));
@@ -616,7 +614,6 @@ int build_tiles(lbx_ctx* c) {
         take(db, (uint64_t)1);
         take(count, norder);
         take(base, norder);
-        take(owner, (uint64_t)d.bound);
         take(split, (uint64_t)d.bound);
     });
     if (!st) st = take_block(&c->node_block, [&](auto&& take) { node_arrays(c, d.bound, take); });
@@ -630,10 +627,11 @@ int build_tiles(lbx_ctx* c) {
         if (st) return;
         hipLaunchKernelGGL(k_mpb_count, waves(), dim3(kBlock), 0, s, dd, count);
         group(nullptr);
-        if (h.ntiles > 0) table(kHaloMax, split, 1);
-        for (uint32_t level = 2; !st && h.ntiles > 0 && h.halo_max > kHaloMax; ++level) {
+        if (h.ntiles > 0) table(kHaloMax, split);
+        if (!st && h.ntiles > 0 && h.halo_max > kHaloMax) {
+            hipLaunchKernelGGL(k_mpb_parts, dim3(h.ntiles), dim3(kBlock), 0, s, dd, db, base, t, split);
             group(split);
-            if (h.ntiles > 0) table(kHaloMax, split, level);
+            if (h.ntiles > 0) table(kHaloMax, nullptr);
         }
     };
     const uint32_t bound = d.bound;
@@ -645,7 +643,7 @@ int build_tiles(lbx_ctx* c) {
     c->mp_general = h.ntiles == 0;
     if (!st && c->mp_general) {
         group(nullptr);
-        table(kHaloMaxGen, nullptr, 0);
+        table(kHaloMaxGen, nullptr);
     }
     give_block(&scratch);
     if (st) {

@@ -524,8 +524,7 @@ struct lbxb {
     int stage_at = 0;
     MpBuild* builds = nullptr;   // [max instances]
     MpBuilt* built = nullptr;
-    uint8_t* split = nullptr;    // layout builds: parts of each tile (log2), the tile that each is part of
-    uint32_t* owner = nullptr;
+    uint8_t* split = nullptr;    // layout builds: parts of each tile (log2)
     double* part[2] = {nullptr, nullptr};
     double* vtrace = nullptr;
     // host state
@@ -889,13 +888,21 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         take(b->walk_base, walk);
     }, true));
     uint32_t *count = b->walk_count, *base = b->walk_base;
-    constexpr uint32_t kGridY = 65535;  // lattices of one launch at most
+    constexpr uint32_t kGridY = 65535;        // lattices of one launch at most,
+    constexpr uint64_t kEmptyBlocks = 65536;  // and its empty blocks
+    std::vector<MpBuilt> counts_h;            // read until the stream has synchronised
+    const auto counted = [&](const std::vector<size_t>& which) -> const std::vector<MpBuilt>& {
+        counts_h.clear();
+        for (size_t k : which) counts_h.push_back(built[k]);
+        return counts_h;
+    };
     const auto size_of = [&](size_t k) { return std::max((uint64_t)builds[k].b.norder, (uint64_t)builds[k].bound); };
-    // one pass over the lattices `which`: tiles cut by `by`, `mark` for the next
-    // pass; general: keep what has an LDS slot
-    auto pass = [&](std::vector<size_t>& which, const uint8_t* by, uint8_t* mark, uint32_t level,
-                    bool general) -> int {
-        // largest first, so that a launch's lattices are of like size: its grid is the largest one's for each
+    // one pass over the lattices `which`: their tiles, cut by split where `cut`;
+    // marks (in split) those whose halo is too large where `mark`; general: keep
+    // what has an LDS slot
+    auto pass = [&](std::vector<size_t>& which, bool cut, bool mark, bool general) -> int {
+        // largest first; a launch's grid is the largest lattice's for each, so it ends
+        // before its empty blocks get to be many, and at a grid's rows
         std::stable_sort(which.begin(), which.end(), [&](size_t x, size_t y) { return size_of(x) > size_of(y); });
         std::vector<MpBuild> d;
         for (size_t k : which) d.push_back(builds[k]);
@@ -904,7 +911,10 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         const auto slices = [&](auto&& f) {
             for (uint32_t s0 = 0, s1; s0 < nd; s0 = s1) {
                 uint32_t gw = 0, gt = 0;
-                for (s1 = s0; s1 < nd && s1 - s0 < kGridY && 2 * size_of(which[s1]) >= size_of(which[s0]); ++s1) {
+                uint64_t empty = 0;
+                for (s1 = s0; s1 < nd && s1 - s0 < kGridY; ++s1) {
+                    empty += size_of(which[s0]) - size_of(which[s1]);
+                    if (empty > kEmptyBlocks) break;
                     gw = std::max(gw, (d[s1].b.norder + kBlock / 64 - 1) / (kBlock / 64));
                     gt = std::max(gt, d[s1].bound);
                 }
@@ -912,17 +922,23 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
             }
         };
         LBX_TRY(hipMemcpyAsync(b->builds, d.data(), nd * sizeof(MpBuild), hipMemcpyHostToDevice, b->stream));
-        if (level == 1)
-            slices([&](uint32_t s0, uint32_t n, uint32_t gw, uint32_t) {
+        if (cut)  // by the last pass's tiles, of lattices in another order there: their counts once more
+            LBX_TRY(hipMemcpyAsync(b->built, counted(which).data(), nd * sizeof(MpBuilt), hipMemcpyHostToDevice,
+                                   b->stream));
+        slices([&](uint32_t s0, uint32_t n, uint32_t gw, uint32_t gt) {
+            if (cut)
+                hipLaunchKernelGGL(k_mpb_parts, dim3(gt, n), dim3(kBlock), 0, b->stream, b->builds + s0,
+                                   b->built + s0, base, b->mpt, b->split);
+            else if (!general)
                 hipLaunchKernelGGL(k_mpb_count, dim3(gw, n), dim3(kBlock), 0, b->stream, b->builds + s0, count);
-            });
+        });
         hipLaunchKernelGGL(k_mpb_group, dim3(nd), dim3(kBlock), 0, b->stream, b->builds, b->built, count, base,
-                           b->mpt.info, by, b->owner);
+                           b->mpt.info, cut ? b->split : nullptr);
         slices([&](uint32_t s0, uint32_t n, uint32_t gw, uint32_t gt) {
             hipLaunchKernelGGL(k_mpb_place, dim3(gw, n), dim3(kBlock), 0, b->stream, b->builds + s0, b->built + s0,
                                base, b->mpt.perm, b->mpt.inv);
             hipLaunchKernelGGL((general ? k_mpb_table<true> : k_mpb_table<false>), dim3(gt, n), dim3(kBlock), 0,
-                               b->stream, b->builds + s0, b->built + s0, b->mpt, b->owner, mark, level);
+                               b->stream, b->builds + s0, b->built + s0, b->mpt, mark ? b->split : nullptr);
         });
         LBX_TRY(hipGetLastError());
         std::vector<MpBuilt> r(nd);
@@ -931,20 +947,21 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         for (uint32_t k = 0; k < nd; ++k) built[which[k]] = r[k];
         return LBX_OK;
     };
-    // the layouts of the lattices `which`; returns those that take more than their bound of tiles
+    // the layouts of the lattices `which`; those that take more than their bound of tiles go to `beyond`
     std::vector<size_t> gen;
     auto settle = [&](std::vector<size_t> which, std::vector<size_t>* beyond) -> int {
-        for (uint32_t level = 1; !which.empty(); ++level) {
-            LBX_TRY(pass(which, level == 1 ? nullptr : b->split, b->split, level, false));
-            std::vector<size_t> more;
-            for (size_t k : which) {
-                if (built[k].ntiles == 0)
-                    beyond->push_back(k);
-                else if (built[k].halo_max > kHaloMax)
-                    more.push_back(k);
-            }
-            which.swap(more);
-        }
+        if (which.empty()) return LBX_OK;
+        LBX_TRY(pass(which, false, true, false));
+        std::vector<size_t> cut;
+        for (size_t k : which)
+            if (built[k].ntiles == 0)
+                beyond->push_back(k);
+            else if (built[k].halo_max > kHaloMax)
+                cut.push_back(k);
+        if (cut.empty()) return LBX_OK;
+        LBX_TRY(pass(cut, true, false, false));
+        for (size_t k : cut)
+            if (built[k].ntiles == 0) beyond->push_back(k);
         return LBX_OK;
     };
     std::vector<size_t> some(ids.size()), whole;
@@ -963,7 +980,7 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
     LBX_TRY(settle(some, &whole));
     for (size_t k : whole) builds[k] = was[k];
     LBX_TRY(settle(whole, &gen));
-    if (!gen.empty()) LBX_TRY(pass(gen, nullptr, nullptr, 0, true));
+    if (!gen.empty()) LBX_TRY(pass(gen, false, false, true));
     for (size_t k = 0; k < ids.size(); ++k) {
         BInst& in = b->tab[ids[k]];
         in.mp_tile0 = 2 * in.tile_first;
@@ -1101,7 +1118,6 @@ void batch_arrays(lbxb* b, Take&& take) {
     take(b->mpt.inv, Np);
     take(b->mp_tile_inst, M / kTile);
     take(b->split, M / kTile);
-    take(b->owner, M / kTile);
     take(b->builds, ni);
     take(b->built, ni);
     take(b->ids, ni);

@@ -177,8 +177,8 @@ __global__ __launch_bounds__(kBlock) void k_mpb_count(const MpBuild* __restrict_
 // Bricks into tiles, in walk order: a brick joins the current tile while the
 // tile holds at most 256 nodes.  base[o] = entry of the brick's first node.
 // split != NULL: tile k of the call without it is cut into 2^split[k] parts, by
-// the place of each brick's first node in it (256 parts: every brick alone),
-// and owner[t] is the k that tile t is part of.  One block per lattice; a thread
+// the place of each brick's first node in it (256 parts: every brick alone).
+// One block per lattice; a thread
 // groups whole runs of kRun bricks, so tiles end at the runs' ends (under 1%
 // of a tile's fill where a run fills a hundred, up to a quarter where a sparse
 // medium's fills two), unless that takes more tiles than the lattice may use:
@@ -186,43 +186,51 @@ __global__ __launch_bounds__(kBlock) void k_mpb_count(const MpBuild* __restrict_
 // 65 536 bricks took 15 ms).
 constexpr uint32_t kRun = 128;
 
-// f(o, nodes, tile of the run, nodes of the tile before it, unsplit tile) per
-// brick with nodes; returns the run's tiles.  The unsplit run's tiles begin at
-// old0.
+// f(o, nodes, tile of the run, nodes of the tile before it) per brick with nodes; returns the run's tiles, and those of the unsplit run, which begin at
+// old0.  A thread's loads go out eight at a time: one by one, each a round trip
+// to memory, the second grouping of a 96^3 lattice took 113 us, now 69.
+struct RunTiles {
+    uint32_t tiles, unsplit;
+};
+
 template <typename F>
-__device__ __forceinline__ uint32_t group_run(const uint32_t* __restrict__ count, uint32_t o0, uint32_t o1,
+__device__ __forceinline__ RunTiles group_run(const uint32_t* __restrict__ count, uint32_t o0, uint32_t o1,
                                               const uint8_t* __restrict__ split, uint32_t old0, F&& f) {
-    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0, part = 0;
+    constexpr uint32_t kAhead = 8;
+    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0, part = 0, exponent = split ? split[old0] : 0u;
     bool any = false;
-    for (uint32_t o = o0; o < o1; ++o) {
-        const uint32_t c = count[o];
-        if (c == 0) continue;
-        bool cut = old_acc + c > kMpTile;
-        if (cut) {
-            ++old;
-            old_acc = 0;
-        }
-        if (split) {
-            const uint32_t p = (old_acc << split[old0 + old]) >> 8;
+    for (uint32_t o8 = o0; o8 < o1; o8 += kAhead) {
+        uint32_t c[kAhead];
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; ++k) c[k] = o8 + k < o1 ? count[o8 + k] : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; ++k) {
+            if (c[k] == 0) continue;
+            bool cut = old_acc + c[k] > kMpTile;
+            if (cut) {
+                ++old;
+                old_acc = 0;
+                if (split) exponent = split[old0 + old];
+            }
+            const uint32_t p = (old_acc << exponent) >> 8;
             cut = cut || (any && p != part);
             part = p;
+            old_acc += c[k];
+            if (cut) {
+                ++tile;
+                acc = 0;
+            }
+            f(o8 + k, c[k], tile, acc);
+            acc += c[k];
+            any = true;
         }
-        old_acc += c;
-        if (cut) {
-            ++tile;
-            acc = 0;
-        }
-        f(o, c, tile, acc, old0 + old);
-        acc += c;
-        any = true;
     }
-    return any ? tile + 1 : 0u;
+    return any ? RunTiles{tile + 1, old + 1} : RunTiles{0, 0};
 }
 
 __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict__ builds, MpBuilt* built,
                                                       const uint32_t* __restrict__ counts, uint32_t* base,
-                                                      uint32_t* info, const uint8_t* __restrict__ split,
-                                                      uint32_t* owner) {
+                                                      uint32_t* info, const uint8_t* __restrict__ split) {
     __shared__ uint32_t sums[kBlock + 1];
     const MpBuild& d = builds[blockIdx.x];
     const uint32_t* count = counts + d.order_off;
@@ -245,7 +253,7 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
         __syncthreads();
         return sums[threadIdx.x];
     };
-    const auto none = [](uint32_t, uint32_t, uint32_t, uint32_t, uint32_t) {};
+    const auto none = [](uint32_t, uint32_t, uint32_t, uint32_t) {};
     uint32_t old0 = 0;
     for (int pass = 0; pass < 2; ++pass) {
         const uint32_t nruns = (n + run - 1) / run;
@@ -253,7 +261,8 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
         r0 = min(nruns, threadIdx.x * per);
         r1 = min(nruns, r0 + per);
         uint32_t mine = 0;
-        for (uint32_t r = r0; r < r1; ++r) mine += group_run(count, r * run, min(n, (r + 1) * run), nullptr, 0, none);
+        for (uint32_t r = r0; r < r1; ++r)
+            mine += group_run(count, r * run, min(n, (r + 1) * run), nullptr, 0, none).tiles;
         old0 = scan(mine);
         if (sums[kBlock] <= d.bound || !d.serial) break;
         run = n;
@@ -263,8 +272,9 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
         uint32_t mine = 0, old = old0;
         for (uint32_t r = r0; r < r1; ++r) {
             const uint32_t o0 = r * run, o1 = min(n, (r + 1) * run);
-            mine += group_run(count, o0, o1, split, d.tile0 + old, none);
-            old += group_run(count, o0, o1, nullptr, 0, none);
+            const RunTiles k = group_run(count, o0, o1, split, d.tile0 + old, none);
+            mine += k.tiles;
+            old += k.unsplit;
         }
         tile0 = scan(mine);
         total = sums[kBlock];
@@ -277,14 +287,13 @@ __global__ __launch_bounds__(kBlock) void k_mpb_group(const MpBuild* __restrict_
     uint32_t old = old0;
     for (uint32_t r = r0; r < r1; ++r) {
         const uint32_t o0 = r * run, o1 = min(n, (r + 1) * run), t0 = d.tile0 + tile0;
-        const uint32_t k = group_run(count, o0, o1, split, d.tile0 + old,
-                                     [&](uint32_t o, uint32_t c, uint32_t tile, uint32_t acc, uint32_t was) {
+        const RunTiles k = group_run(count, o0, o1, split, d.tile0 + old,
+                                     [&](uint32_t o, uint32_t c, uint32_t tile, uint32_t acc) {
                                          base[d.order_off + o] = (t0 + tile) * kMpTile + acc;
                                          info[t0 + tile] = acc + c;
-                                         owner[t0 + tile] = was;
                                      });
-        tile0 += k;
-        old += split ? group_run(count, o0, o1, nullptr, 0, none) : k;
+        tile0 += k.tiles;
+        old += k.unsplit;
     }
 }
 
@@ -309,14 +318,12 @@ __global__ __launch_bounds__(kBlock) void k_mpb_place(const MpBuild* __restrict_
 // Halo list and slot table of every tile (grid x: a lattice's tiles, y:
 // lattices).  The distinct outside neighbours are collected in an LDS hash
 // table and sorted, so that consecutive slots read consecutive entries.
-// split[owner] (split may be NULL) receives `level` for a tile with more than
-// kHaloMax halo nodes, and in the first pass (level 1, owners their own tiles)
-// 0 for every other.  A table of 1024 places is enough to tell a tile that must
-// be cut; the general tiles keep up to kHaloMaxGen of theirs.
+// split (may be NULL) receives 1 for a tile with more than kHaloMax.
+// A table of 1024 places is enough to tell a tile that must be cut; the general
+// tiles keep up to kHaloMaxGen of theirs.
 template <bool GEN>
 __global__ __launch_bounds__(kBlock) void k_mpb_table(const MpBuild* __restrict__ builds, MpBuilt* built, MpTiles t,
-                                                      const uint32_t* __restrict__ owner, uint8_t* split,
-                                                      uint32_t level) {
+                                                      uint8_t* split) {
     constexpr uint32_t kHashSize = GEN ? 4096 : 1024, kHashMax = GEN ? 2048 : 512;
     static_assert(kHashMax + 2 * kMpTile <= kHashSize && kHashMax > kHaloMax, "room to stop inserting");
     __shared__ uint32_t key[kHashSize];
@@ -390,9 +397,74 @@ __global__ __launch_bounds__(kBlock) void k_mpb_table(const MpBuild* __restrict_
     t.tab4[e] = make_uint4(w[0], w[1], w[2], w[3]);
     t.tab2[e] = make_uint2(w[4], w[5]);
     if (threadIdx.x == 0) {
-        if (split && (n > kHaloMax || level == 1)) split[owner[tile]] = n > kHaloMax ? (uint8_t)level : 0;
+        if (split) split[tile] = n > kHaloMax ? 1 : 0;
         atomicMax(&built[blockIdx.y].halo_max, n);
     }
+}
+
+// place of brick (x, y, z) in the walk (walk_brick's inverse)
+__device__ __forceinline__ uint32_t brick_place(const Bricks& b, uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t plane = b.cx * b.cy, column = plane * ((b.nbz + b.inner - 1) / b.inner * b.inner);
+    const uint32_t m = x % b.cx + b.cx * (y % b.cy) + plane * (z / b.inner);
+    return (x / b.cx + b.ncx * (y / b.cy)) * column + m * b.inner + z % b.inner;
+}
+
+// For every tile that split marks (grid as k_mpb_table), the least k for which
+// none of its 2^k parts has more than kHaloMax halo nodes, into split: the parts'
+// distinct outside neighbours, those in the tile's other parts included, are
+// counted in an LDS hash table.  Every brick alone (k = 8) always fits.  (The
+// parts laid out and tabled at each k in turn: two more passes over a lattice's
+// tiles, 0.85 ms more for a batch of eight 3-D lattices.)
+__global__ __launch_bounds__(kBlock) void k_mpb_parts(const MpBuild* __restrict__ builds,
+                                                      const MpBuilt* __restrict__ built,
+                                                      const uint32_t* __restrict__ base, MpTiles t, uint8_t* split) {
+    constexpr uint32_t kPlaces = 8192;  // for at most 18 pairs a node
+    static_assert(18 * kMpTile < kPlaces, "room for every pair");
+    __shared__ unsigned long long key[kPlaces];
+    __shared__ uint32_t count[kMpTile];
+    __shared__ uint8_t start[kMpTile];  // of its brick in the tile, by node
+    const MpBuild& d = builds[blockIdx.y];
+    if (blockIdx.x >= built[blockIdx.y].ntiles) return;
+    const uint32_t tile = d.tile0 + blockIdx.x;
+    if (split[tile] == 0) return;
+    const bool valid = threadIdx.x < t.info[tile];
+    uint32_t q[kQ];
+    if (valid) {
+        const uint32_t r = d.nodes[t.perm[tile * kMpTile + threadIdx.x]] & kIndexMask;
+        const uint32_t x = r % d.b.lx, y = r / d.b.lx % d.b.ly, z = r / d.b.lx / d.b.ly;
+        start[threadIdx.x] =
+            (uint8_t)(base[d.order_off + brick_place(d.b, x / d.b.bx, y / d.b.by, z / d.b.bz)] - tile * kMpTile);
+        Neighbours nb;
+        nb.load(d.map, r, d.dlx, d.dly, d.b.lz);
+        static_for<1, kQ>([&](auto I) { q[I] = nb.q[I] != kSolidSlot ? t.inv[nb.q[I]] : kSolidSlot; });
+    }
+    uint32_t k = 0;
+    for (bool over = true; over && k < 8;) {
+        ++k;
+        __syncthreads();  // the last round's counts have been read
+        for (uint32_t i = threadIdx.x; i < kPlaces; i += kBlock) key[i] = ~0ull;
+        count[threadIdx.x] = 0;
+        __syncthreads();
+        if (valid) {
+            const uint32_t part = ((uint32_t)start[threadIdx.x] << k) >> 8;
+            static_for<1, kQ>([&](auto I) {
+                constexpr int L = I;
+                if (q[L] == kSolidSlot) return;
+                if (q[L] / kMpTile == tile && ((uint32_t)start[q[L] % kMpTile] << k) >> 8 == part) return;
+                const unsigned long long want = (unsigned long long)part << 32 | q[L];
+                uint32_t h = ((q[L] ^ part * 0x9E3779B9u) * 2654435761u) >> 19;
+                for (uint32_t n = 0; n < kPlaces; ++n) {
+                    const unsigned long long was = atomicCAS(&key[h], ~0ull, want);
+                    if (was == ~0ull) atomicAdd(&count[part], 1u);
+                    if (was == ~0ull || was == want) break;
+                    h = (h + 1) & (kPlaces - 1);
+                }
+            });
+        }
+        __syncthreads();
+        over = __syncthreads_or(count[threadIdx.x] > kHaloMax) != 0;
+    }
+    if (threadIdx.x == 0) split[tile] = (uint8_t)k;
 }
 
 // ------------------------------------------------------- per-node values
