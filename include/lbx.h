@@ -309,9 +309,11 @@ int lbx_collide_noalloc(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature
                         const double* f_ext_x, const double* f_ext_y, const double* f_ext_z);
 
 /* ------------------------------------------------------------- timing
- * Average device duration (ms) of the launches of one kernel family since
- * the last reset, measured with HIP events on the context's stream around
- * back-to-back launch runs.  which: 0 = LB step, 1 = MP step. */
+ * Device time (total_ms) of one kind of time step since the last reset,
+ * measured with HIP events on the context's stream around back-to-back launch
+ * runs, and the steps it covers (launches: one launch a step, but small
+ * lattices take many steps in one launch, each counted).  which: 0 = LB step,
+ * 1 = MP step. */
 #define LBX_KERNEL_LB 0
 #define LBX_KERNEL_MP 1
 int lbx_timing_enable(lbx_ctx* ctx, int32_t on);
