@@ -92,8 +92,8 @@ inline Bricks make_bricks(uint32_t lx, uint32_t ly, uint32_t lz, bool halves = f
 
 // Tiles a lattice of nf fluid nodes is laid out in at most: two consecutive
 // tiles hold more than 256 nodes together (so k tiles need floor(k/2) 257 <= nf,
-// less than twice nf/256 rounded up), and bricks are only taken out of a tile
-// again while the count stays within this.
+// less than twice nf/256 rounded up), and tiles are only cut while the count
+// stays within this.
 inline uint32_t mp_tile_bound(uint32_t nf) { return 2u * ((nf + kMpTile - 1) / kMpTile); }
 
 // Whether a layout of nt tiles is tried again with halves of the bricks: bricks

@@ -295,7 +295,7 @@ def main(argv=None):
     rng = np.random.default_rng(args.seed)
     reqs = [serving_request(rng) for _ in range(args.requests)]
     prec = _prec("fp32_shift" if args.precision in ("both", "all") else args.precision)
-    # HBM budget (default 48 M fluid nodes, ~20 GB in the FP32-shift form: room
+    # HBM budget (default 48 M fluid nodes, 34 GB in the FP32-shift form: room
     # for several of the largest requests at once)
     cap_nodes, cap_box = args.capacity_nodes, args.capacity_box
     # saturation throughput: a closed batch of the first requests, all admitted at t = 0
