@@ -551,9 +551,9 @@ void add_flow(lbx_ctx* c, Planes& s, double* rho_d, double* j_d, const double* r
 // the arrays of a geometry's MP tiles: by tile that it may use and packed node,
 // and by tile and entry
 template <typename Take>
-void node_arrays(lbx_ctx* c, uint64_t bound, Take&& take) {
+void node_arrays(lbx_ctx* c, uint64_t bound, uint64_t Nf, Take&& take) {
     take(c->mpt.info, bound);
-    take(c->mpt.inv, (uint64_t)c->Nf);
+    take(c->mpt.inv, Nf);
 }
 template <typename Take>
 void tile_arrays(lbx_ctx* c, uint64_t tiles, uint32_t pitch, Take&& take) {
@@ -580,7 +580,7 @@ int build_tiles(lbx_ctx* c) {
     d.map = c->map;
     d.dlx = c->dlx;
     d.dly = c->dly;
-    d.bound = mp_tile_bound(c->Nf);
+    d.bound = (uint32_t)mp_tile_bound(c->Nf);
     MpBuild* dd = nullptr;
     MpBuilt* db = nullptr;
     uint32_t *count = nullptr, *base = nullptr;
@@ -616,7 +616,7 @@ int build_tiles(lbx_ctx* c) {
         take(base, norder);
         take(split, (uint64_t)d.bound);
     });
-    if (!st) st = take_block(&c->node_block, [&](auto&& take) { node_arrays(c, d.bound, take); });
+    if (!st) st = take_block(&c->node_block, [&](auto&& take) { node_arrays(c, d.bound, c->Nf, take); });
     // the layout with bricks b on at most `bound` tiles; no tiles (h.ntiles): it takes more
     auto settle = [&](const Bricks& b, uint32_t bound) {
         d.b = b;
@@ -822,21 +822,23 @@ int lbx_d3q19_tables(int32_t c[57], double a0o[19], double a1o[19], double a2o[1
 }  // extern "C"
 
 namespace {
-// the arrays of the LB phase
+// the arrays of the LB phase of N nodes, Nf of them fluid (64-bit counts: a
+// footprint is asked for beyond what a context may be)
 template <typename Take>
-void lb_arrays(lbx_ctx* c, Take&& take) {
+void lb_arrays(lbx_ctx* c, uint64_t N, uint64_t Nf, Take&& take) {
+    const uint64_t Np = (Nf + 63) / 64 * 64;
     for (int b = 0; b < 2; ++b)
-        if (f32_storage(c->prec)) take(c->g[b], kQ * c->Np); else take(c->f[b], kQ * c->Np);
-    if (c->prec == LBX_PREC_FP32_SHIFT) take(c->j32, 3 * c->Np);
-    take(c->j, 3 * c->Np);
-    take(c->rho, c->Np);
-    take(c->nodes, (uint64_t)c->Nf);
-    take(c->map, (uint64_t)c->N);
-    if (c->Nf <= kTabNodes) take(c->pulls, 18 * c->Np);
+        if (f32_storage(c->prec)) take(c->g[b], kQ * Np); else take(c->f[b], kQ * Np);
+    if (c->prec == LBX_PREC_FP32_SHIFT) take(c->j32, 3 * Np);
+    take(c->j, 3 * Np);
+    take(c->rho, Np);
+    take(c->nodes, Nf);
+    take(c->map, N);
+    if (Nf <= kTabNodes) take(c->pulls, 18 * Np);
     take(c->slots, (uint64_t)(3 * kSlots));
     take(c->ctrl, (uint64_t)1);
     take(c->l2ring, (uint64_t)kRing);
-    take(c->box_reserve, (uint64_t)std::min(box_values(c->N), kBoxReserve));
+    take(c->box_reserve, (uint64_t)std::min(box_values(N), kBoxReserve));
 }
 }  // namespace
 
@@ -848,15 +850,14 @@ int64_t lbx_footprint_bytes(int32_t lx, int32_t ly, int32_t lz, int32_t precisio
     // adsorbing, their probabilities stored, on the tiles of the general layout's wider halo lists
     lbx_ctx c;
     c.prec = precision;
-    c.N = c.Nf = (uint32_t)((uint64_t)lx * ly * lz);
-    c.Np = ((uint64_t)c.Nf + 63) / 64 * 64;
-    uint64_t b = block_bytes([&](auto&& take) { lb_arrays(&c, take); }) + box_values(c.N) * 8ull;
-    if (c.Nf > kTabNodes) b += 18 * 4 * (uint64_t)kTabNodes;
+    const uint64_t N = (uint64_t)lx * ly * lz;
+    uint64_t b = block_bytes([&](auto&& take) { lb_arrays(&c, N, N, take); }) + box_values(N) * 8ull;
+    if (N > kTabNodes) b += 18 * 4 * (uint64_t)kTabNodes;
     if (with_mp > 0) {
         const int T = std::min(with_mp, kMaxTracers);
         const Bricks br = make_bricks((uint32_t)lx, (uint32_t)ly, (uint32_t)lz);
-        const uint64_t bound = mp_tile_bound(c.Nf), tiles = std::min<uint64_t>((uint64_t)br.nbx * br.nby * br.nbz, bound);
-        b += block_bytes([&](auto&& take) { node_arrays(&c, bound, take); }) +
+        const uint64_t bound = mp_tile_bound(N), tiles = std::min<uint64_t>((uint64_t)br.nbx * br.nby * br.nbz, bound);
+        b += block_bytes([&](auto&& take) { node_arrays(&c, bound, N, take); }) +
              block_bytes([&](auto&& take) { tile_arrays(&c, tiles, kHaloMaxGen, take); }) +
              block_bytes([&](auto&& take) {
                  if (f32_storage(precision))
@@ -915,7 +916,7 @@ int lbx_create(int32_t lx, int32_t ly, int32_t lz, const int8_t* nature, double 
     // together exceed the 256 MiB last-level cache, no written line survives
     // there to the next step
     c->nt = 2 * kQ * c->Np * (shift ? sizeof(float) : sizeof(double)) > (uint64_t)LBX_NT_MIN_BYTES;
-    if (!st) st = take_block(&c->lb_block, [&](auto&& take) { lb_arrays(c, take); });
+    if (!st) st = take_block(&c->lb_block, [&](auto&& take) { lb_arrays(c, c->N, c->Nf, take); });
     if (!st && (hipEventCreate(&c->ev[0]) != hipSuccess || hipEventCreate(&c->ev[1]) != hipSuccess))
         st = LBX_ERR_DEVICE;
     uint32_t nfi = 0;

@@ -879,7 +879,7 @@ int build_tiles(lbxb* b, const std::vector<uint32_t>& ids) {
         d.dly = in.dly;
         d.order_off = (uint32_t)walk;
         d.tile0 = 2 * in.tile_first;
-        d.bound = mp_tile_bound(h.Nf);  // 2 in.ntiles
+        d.bound = (uint32_t)mp_tile_bound(h.Nf);  // 2 in.ntiles
         d.serial = 1;
         walk += std::max(d.b.norder, halves[k].norder);
     }
@@ -1075,7 +1075,7 @@ void set_capacity(lbxb* b, int32_t precision, int64_t nodes, int64_t box, int32_
 // all device arrays of a batch
 template <typename Take>
 void batch_arrays(lbxb* b, Take&& take) {
-    const uint64_t Np = b->Np, tiles = b->ntiles_cap, ni = b->cap_inst;
+    const uint64_t Np = b->Np, tiles = Np / kTile, ni = b->cap_inst;
     const uint64_t M = 2 * Np;  // entries of the MP tiles
     for (int k = 0; k < 2; ++k)
         if (shift(b)) take(b->g[k], kQ * Np); else take(b->f[k], kQ * Np);
@@ -1086,7 +1086,7 @@ void batch_arrays(lbxb* b, Take&& take) {
     take(b->maps, b->cap_box);
     take(b->tile_inst, tiles);
     take(b->nature, (b->cap_box + 15) / 16 * 16);
-    take(b->counts, (uint64_t)node_chunks(b->cap_box));
+    take(b->counts, (b->cap_box + kNodeChunk - 1) / kNodeChunk);
     take(b->nfi, ni);
     take(b->act[0], tiles);
     take(b->act[1], 2 * tiles);

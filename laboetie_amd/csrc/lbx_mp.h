@@ -94,7 +94,7 @@ inline Bricks make_bricks(uint32_t lx, uint32_t ly, uint32_t lz, bool halves = f
 // tiles hold more than 256 nodes together (so k tiles need floor(k/2) 257 <= nf,
 // less than twice nf/256 rounded up), and tiles are only cut while the count
 // stays within this.
-inline uint32_t mp_tile_bound(uint32_t nf) { return 2u * ((nf + kMpTile - 1) / kMpTile); }
+inline uint64_t mp_tile_bound(uint64_t nf) { return 2 * ((nf + kMpTile - 1) / kMpTile); }
 
 // Whether a layout of nt tiles is tried again with halves of the bricks: bricks
 // that hold a little over half a tile each (fine-grained media of porosity 0.5

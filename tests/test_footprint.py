@@ -58,3 +58,13 @@ def test_footprint_bounds_the_memory_in_use(what, prec):
             bound = lbx.footprint_bytes(*dims, prec, ntr)
             print(used, bound, flush=True)
             assert used <= bound + (16 << 20)  # allocations are rounded to the driver's pages
+
+
+def test_footprint_beyond_32_bit_counts():
+    """The sizes are 64-bit numbers, also of boxes and batches that are refused."""
+    for prec in PRECS:
+        for ntr in (0, 1, 3):
+            small, large = (lbx.footprint_bytes(n, n, n, prec, ntr) for n in (800, 3200))
+            assert 60 < large / small < 68, (prec, ntr, small, large)
+        small, large = (lbx.Batch.footprint_bytes(n, n, 1, prec) for n in (1 << 27, 1 << 41))
+        assert 1.6e4 < large / small < 1.7e4, (prec, small, large)
