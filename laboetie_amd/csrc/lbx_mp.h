@@ -197,7 +197,7 @@ template <typename F>
 __device__ __forceinline__ RunTiles group_run(const uint32_t* __restrict__ count, uint32_t o0, uint32_t o1,
                                               const uint8_t* __restrict__ split, uint32_t old0, F&& f) {
     constexpr uint32_t kAhead = 8;
-    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0, part = 0, exponent = split ? split[old0] : 0u;
+    uint32_t tile = 0, acc = 0, old = 0, old_acc = 0, part = 0, exponent = 0;
     bool any = false;
     for (uint32_t o8 = o0; o8 < o1; o8 += kAhead) {
         uint32_t c[kAhead];
@@ -210,8 +210,9 @@ __device__ __forceinline__ RunTiles group_run(const uint32_t* __restrict__ count
             if (cut) {
                 ++old;
                 old_acc = 0;
-                if (split) exponent = split[old0 + old];
             }
+            // read with a brick of the tile only: past the last tile there is no entry
+            if (split && (cut || !any)) exponent = split[old0 + old];
             const uint32_t p = (old_acc << exponent) >> 8;
             cut = cut || (any && p != part);
             part = p;
